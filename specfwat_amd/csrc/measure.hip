@@ -1387,81 +1387,176 @@ __global__ void __launch_bounds__(256) k_ws_prep(int nstep, double dt, double t0
   }
 }
 
-// sliding_cc (win_sel.f90:76-100), correlation part: one wavefront per window
-// start i; the Hann tapered windows of d and s in LDS, the full correlation
-// with every lag's sum in the reference's order, and its first maximum; the
-// lag goes to ish, the coefficient is k_ws_coef's.  Lags come in blocks of
-// four consecutive lags (a sliding register window over s, as k_cc_corr,
-// unrolled by four so the window needs no register moves).  Block b costs
-// about min(4 b, 2 nlen - 4 b) multiply-adds and a wavefront runs as long as
-// its slowest lane, so the blocks are dealt to the lanes in descending cost
-// (the block holding lag nlen - 1 first, then alternately its neighbours):
-// the 64 dearest blocks run together, then the next 64
-__device__ __forceinline__ int ws_block_of_rank(int r, int c, int nb) {
-  const int L = c, R = nb - 1 - c, m = L < R ? L : R;
-  if (r == 0) return c;
-  if (r <= 2 * m) { const int k = (r + 1) / 2; return (r & 1) ? c - k : c + k; }
-  const int k = r - m;
-  return L > R ? c - k : c + k;
+// Window starts whose time shift or coefficient k_ws_select reads: those whose centre lies in
+// the trace's time range [tstart, tend], and the neighbours its time-shift jump rule looks at
+// (nint(jump / dt) on either side and the one before), with two samples to spare.  The rest of
+// the trace, before the first arrival and after the slowest one, is never asked for: 31 % of
+// 9,800 window starts remain at 10,000 samples of 4 ms and a 12 s range.
+__device__ __forceinline__ int2 ws_needed(int t, int nlen, int nw, double dt, double t0, double min_period,
+                                          double min_velocity, double jump_fac, const double* __restrict__ tp,
+                                          const double* __restrict__ dist) {
+  const double tstart = tp[t] - min_period * 1.5 + t0;
+  const double tend = dist[t] / min_velocity + min_period * 1.5 + t0;
+  const double nj = round(jump_fac * min_period / dt) + 3.0, half = (double)nlen / 2.0;
+  const double lo = floor(tstart / dt - half) - nj, hi = ceil(tend / dt - half) + nj;
+  // clamped as doubles; a NaN bound keeps its end of the trace
+  return make_int2((int)fmin(fmax(lo, 0.0), (double)nw), (int)fmax(fmin(hi, (double)(nw - 1)), -1.0));
 }
 
-__global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
-                                                             const double* __restrict__ wt,
-                                                             const double* __restrict__ Dn,
-                                                             const double* __restrict__ Sn, int* __restrict__ ish_out) {
+// sliding_cc (win_sel.f90:76-100), correlation part: one wavefront per window start i, the lag
+// of the first maximum of the full correlation of the Hann tapered windows of d and s (every
+// lag's sum in double precision in the reference's order); the coefficient is k_ws_coef's.
+//
+// The correlations are bound by arithmetic (nlen^2 products per window start), so single
+// precision sorts out the lags first: both windows are scaled by powers of two into [-1, 1],
+// every lag's sum is taken in fp32, and only lags within the rounding of those sums of the
+// largest one - the error of a sum of n products is at most about n 2^-24 |d| |s|, twice that
+// for the positive lags, which are differences - can be the maximum.  When one lag is left it is the
+// answer; else the remaining ones are summed in double precision as the reference sums them and
+// compared, so the lag is the double-precision one in every case (ties go to the smaller lag).
+// With s laid out twice in a row, lag m and lag m - nlen together read nlen products, so every
+// lane does the same work: a running sum over j whose value at j = m is the negative lag's, and
+// the rest the positive one's.  Four lags per lane, one 16-byte LDS read of d and one of s per
+// sixteen products.  400 x 3 traces of 10,000 samples, nlen 201: 92.5 ms when every lag of every
+// window start was summed in double precision.
+__device__ __forceinline__ double ws_lag_sum(int mm, int nlen, const double* dw, const double* sw) {
+  // the lags come in fours and run over the union of their ranges, s zero outside its window
+  const int mb = mm & ~3;
+  const int lo = mb - (nlen - 1) > 0 ? mb - (nlen - 1) : 0, hi = mb + 3 < nlen - 1 ? mb + 3 : nlen - 1;
+  const int off = nlen - 1 - mm;
+  double c = 0.0;
+  for (int j = lo; j <= hi; ++j) {
+    const int k = j + off;
+    c = c + dw[j] * (k >= 0 && k < nlen ? sw[k] : 0.0);
+  }
+  return c;
+}
+
+// LDS of one wavefront of k_ws_sliding (bytes, a multiple of 16): dw, sw, the lags' fp32 sums,
+// fp32 d (padded to a multiple of four) and fp32 s twice, with room for the lags of the last four
+__host__ __device__ inline int ws_quad(int nlen) { return (nlen + 3) & ~3; }
+__host__ __device__ inline size_t ws_lds(int nlen) {
+  const size_t q = (size_t)ws_quad(nlen);
+  return 2 * q * sizeof(double) + (2 * q + q + 2 * q + 8) * sizeof(float);
+}
+
+__global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw, double dt, double t0,
+                                                    double min_period, double min_velocity, double jump_fac,
+                                                    const double* __restrict__ tp, const double* __restrict__ dist,
+                                                    const double* __restrict__ wt, const double* __restrict__ Dn,
+                                                    const double* __restrict__ Sn, int* __restrict__ ish_out) {
   extern __shared__ double wsh[];
-  const int nwv = blockDim.x / 64;  // one window start per wavefront, 2 nlen + 7 doubles of LDS each
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, t = blockIdx.y;
-  const int i = blockIdx.x * nwv + wave;
-  double* dw = wsh + (size_t)wave * (2 * nlen + 7);
-  double* sw = dw + nlen + 3;  // s with three zeros before and four after (indices -3 .. nlen + 3)
-  if (i < nw) {
+  const int nwv = blockDim.x / 64, wave = threadIdx.x / 64, lane = threadIdx.x % 64, t = blockIdx.y;
+  const int2 need = ws_needed(t, nlen, nw, dt, t0, min_period, min_velocity, jump_fac, tp, dist);
+  const int i = need.x + blockIdx.x * nwv + wave;
+  if (i > need.y) return;  // the wavefronts of a workgroup share nothing
+  const int nq = ws_quad(nlen);
+  double* dw = wsh + wave * (ws_lds(nlen) / sizeof(double));
+  double* sw = dw + nq;
+  float* cs = reinterpret_cast<float*>(sw + nq);  // fp32 sums of lag index 0 .. 2 nlen - 2
+  float* df = cs + 2 * nq;
+  float* sf = df + nq;  // s[x mod nlen] at sf[x + nq + 4], x = -nq - 4 .. nq + 3
+  float dm = 0.0f, sm = 0.0f;
+  bool odd = false;  // a value that is not finite
+  {
     const double* d = Dn + (size_t)t * nstep + i;
     const double* s = Sn + (size_t)t * nstep + i;
-    for (int j = lane; j < nlen; j += 64) { dw[j] = d[j] * wt[j]; sw[j] = s[j] * wt[j]; }
-    if (lane < 3) sw[-1 - lane] = 0.0;
-    if (lane < 4) sw[nlen + lane] = 0.0;
-  }
-  __syncthreads();
-  if (i >= nw) return;
-  double best = -INFINITY;
-  int bm = 0x7fffffff;
-  const int nlag = 2 * nlen - 1, nb = (nlag + 3) / 4, cb = (nlen - 1) / 4;
-  for (int r = lane; r < nb; r += 64) {
-    const int mb = 4 * ws_block_of_rank(r, cb, nb);
-    const int lo = mb - (nlen - 1) > 0 ? mb - (nlen - 1) : 0, hi = mb + 3 < nlen - 1 ? mb + 3 : nlen - 1;
-    const int off = nlen - 1 - mb;  // s index of lag mb + q at i1: i1 + off - q, in [-3, nlen + 3]
-    double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
-    double r0 = sw[lo + off], r1 = sw[lo + off - 1], r2 = sw[lo + off - 2], r3 = sw[lo + off - 3];
-    int i1 = lo;
-    for (; i1 + 3 <= hi; i1 += 4) {
-      const double d0 = dw[i1], d1 = dw[i1 + 1], d2 = dw[i1 + 2], d3 = dw[i1 + 3];
-      const double s0 = sw[i1 + 1 + off], s1 = sw[i1 + 2 + off], s2 = sw[i1 + 3 + off], s3 = sw[i1 + 4 + off];
-      c0 = c0 + d0 * r0; c1 = c1 + d0 * r1; c2 = c2 + d0 * r2; c3 = c3 + d0 * r3;
-      c0 = c0 + d1 * s0; c1 = c1 + d1 * r0; c2 = c2 + d1 * r1; c3 = c3 + d1 * r2;
-      c0 = c0 + d2 * s1; c1 = c1 + d2 * s0; c2 = c2 + d2 * r0; c3 = c3 + d2 * r1;
-      c0 = c0 + d3 * s2; c1 = c1 + d3 * s1; c2 = c2 + d3 * s0; c3 = c3 + d3 * r0;
-      r0 = s3; r1 = s2; r2 = s1; r3 = s0;
+    double dmx = 0.0, smx = 0.0;
+    for (int j = lane; j < nlen; j += 64) {
+      const double a = d[j] * wt[j], b = s[j] * wt[j];
+      dw[j] = a;
+      sw[j] = b;
+      dmx = fmax(dmx, fabs(a));
+      smx = fmax(smx, fabs(b));
+      odd = odd || !(fabs(a) < INFINITY) || !(fabs(b) < INFINITY);
     }
-    for (; i1 <= hi; ++i1) {
-      const double dv = dw[i1];
-      c0 = c0 + dv * r0;
-      c1 = c1 + dv * r1;
-      c2 = c2 + dv * r2;
-      c3 = c3 + dv * r3;
-      r3 = r2;
-      r2 = r1;
-      r1 = r0;
-      r0 = sw[i1 + 1 + off];
+    for (int o = 32; o > 0; o >>= 1) {
+      dmx = fmax(dmx, __shfl_xor(dmx, o));
+      smx = fmax(smx, __shfl_xor(smx, o));
     }
-    const double cv[4] = {c0, c1, c2, c3};
-    for (int q = 0; q < 4; ++q)  // blocks arrive out of lag order: ties go to the smaller lag
-      if (mb + q < nlag && (cv[q] > best || (cv[q] == best && mb + q < bm))) { best = cv[q]; bm = mb + q; }
+    odd = __any(odd);
+    // powers of two: the scaled windows' largest magnitudes lie in [1/2, 1)
+    const int de = dmx > 0.0 && !odd ? ilogb(dmx) + 1 : 0, se = smx > 0.0 && !odd ? ilogb(smx) + 1 : 0;
+    __threadfence_block();
+    for (int j = lane; j < nq; j += 64) {
+      const float v = j < nlen ? (float)ldexp(dw[j], -de) : 0.0f;
+      df[j] = v;
+      dm = fmaf(v, v, dm);
+    }
+    for (int k = lane; k < 2 * nq + 8; k += 64) {
+      const int x = k - nq - 4, y = x < 0 ? x + nlen : x;
+      const float v = y >= 0 && y < nlen ? (float)ldexp(sw[y], -se) : 0.0f;
+      sf[k] = v;
+      if (x >= 0) sm = fmaf(v, v, sm);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      dm += __shfl_xor(dm, o);
+      sm += __shfl_xor(sm, o);
+    }
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    const double v2 = __shfl_xor(best, o);
-    const int m2 = __shfl_xor(bm, o);
-    if (v2 > best || (v2 == best && m2 < bm)) { best = v2; bm = m2; }
+  __threadfence_block();  // LDS of this wavefront, written and read by its own lanes
+  const int nlag = 2 * nlen - 1;
+  float best = -INFINITY;
+  for (int r = lane; 4 * r < nlen; r += 64) {
+    const int mb = 4 * r;
+    float a0 = 0, a1 = 0, a2 = 0, a3 = 0, n0 = 0, n1 = 0, n2 = 0, n3 = 0;
+    const float* sp = sf + nq + 4 - mb;
+    float4 lo = *reinterpret_cast<const float4*>(sp - 4);
+    for (int j = 0; j < nq; j += 4) {
+      const float4 d = *reinterpret_cast<const float4*>(df + j), hi = *reinterpret_cast<const float4*>(sp + j);
+      const bool at = j == mb;  // lag mb + q passes from m - nlen to m at j = mb + q
+      n0 = at ? a0 : n0;
+      a0 = fmaf(d.x, hi.x, a0); a1 = fmaf(d.x, lo.w, a1); a2 = fmaf(d.x, lo.z, a2); a3 = fmaf(d.x, lo.y, a3);
+      n1 = at ? a1 : n1;
+      a0 = fmaf(d.y, hi.y, a0); a1 = fmaf(d.y, hi.x, a1); a2 = fmaf(d.y, lo.w, a2); a3 = fmaf(d.y, lo.z, a3);
+      n2 = at ? a2 : n2;
+      a0 = fmaf(d.z, hi.z, a0); a1 = fmaf(d.z, hi.y, a1); a2 = fmaf(d.z, hi.x, a2); a3 = fmaf(d.z, lo.w, a3);
+      n3 = at ? a3 : n3;
+      a0 = fmaf(d.w, hi.w, a0); a1 = fmaf(d.w, hi.z, a1); a2 = fmaf(d.w, hi.y, a2); a3 = fmaf(d.w, hi.x, a3);
+      lo = hi;
+    }
+    const float c1[4] = {a0 - n0, a1 - n1, a2 - n2, a3 - n3}, c2[4] = {n0, n1, n2, n3};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int m = mb + q;
+      if (m < nlen) {
+        cs[nlen - 1 + m] = c1[q];
+        best = fmaxf(best, c1[q]);
+        if (m > 0) {
+          cs[m - 1] = c2[q];
+          best = fmaxf(best, c2[q]);
+        }
+      }
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) best = fmaxf(best, __shfl_xor(best, o));
+  __threadfence_block();
+  // error of a sum: (nlen + 3) roundings of at most |d| |s| (two of the scaled inputs, nq of the
+  // running sum), twice for the differences, twice for two sums compared, 1/16 to spare
+  const float bound = 4.25f * (float)(nq + 8) * 5.9604645e-8f * sqrtf(dm * sm);
+  const float thr = odd || !(bound < INFINITY) ? -INFINITY : best - bound;
+  int count = 0, only = 0;
+  for (int m0 = 0; m0 < nlag; m0 += 64) {
+    const unsigned long long w = __ballot(m0 + lane < nlag && !(cs[min(m0 + lane, nlag - 1)] < thr));
+    if (w) only = m0 + __builtin_ctzll(w);
+    count += __builtin_popcountll(w);
+  }
+  int bm = only;
+  if (!odd && (dm == 0.0f || sm == 0.0f)) {
+    bm = 0;  // every sum is zero: the first lag
+  } else if (count != 1) {
+    double bv = -INFINITY;
+    bm = 0x7fffffff;
+    for (int m = lane; m < nlag; m += 64)
+      if (!(cs[m] < thr)) {
+        const double c = ws_lag_sum(m, nlen, dw, sw);
+        if (c > bv || (c == bv && m < bm)) { bv = c; bm = m; }
+      }
+    for (int o = 32; o > 0; o >>= 1) {
+      const double v2 = __shfl_xor(bv, o);
+      const int m2 = __shfl_xor(bm, o);
+      if (v2 > bv || (v2 == bv && m2 < bm)) { bv = v2; bm = m2; }
+    }
   }
   if (lane == 0) ish_out[(size_t)t * nw + i] = bm + 1 - nlen;
 }
@@ -1470,12 +1565,16 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
 // one window start per lane: a = sum(d s_shifted), b = sum(d^2), c =
 // sum(s_shifted^2) over the tapered window with d's emptied edge zeroed, each
 // sum in the reference's order; neighbouring lanes read neighbouring samples
-__global__ void __launch_bounds__(256) k_ws_coef(int nstep, int nlen, int nw, double dt,
+__global__ void __launch_bounds__(256) k_ws_coef(int nstep, int nlen, int nw, double dt, double t0, double min_period,
+                                                 double min_velocity, double jump_fac,
+                                                 const double* __restrict__ tp, const double* __restrict__ dist,
                                                  const double* __restrict__ wt, const double* __restrict__ Dn,
                                                  const double* __restrict__ Sn, const int* __restrict__ ish_in,
                                                  double* __restrict__ ts, double* __restrict__ cc) {
-  const int t = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nw) return;
+  const int t = blockIdx.y;
+  const int2 need = ws_needed(t, nlen, nw, dt, t0, min_period, min_velocity, jump_fac, tp, dist);
+  const int i = need.x + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > need.y) return;
   const int ish = ish_in[(size_t)t * nw + i];
   const double* d = Dn + (size_t)t * nstep + i;
   const double* s = Sn + (size_t)t * nstep + i;
@@ -1568,7 +1667,8 @@ __global__ void __launch_bounds__(256) k_ws_select(int nstep, int nlen, int nw, 
   auto is_jump = [&](int i) { return i > 0 && i < nw && fabs(tsr[i] - tsr[i - 1]) > jump; };
   for (int i = threadIdx.x; i < nw; i += 256) {
     const double tc = tcc(i);
-    bool good = ccr[i] > cfg.thr_corr && fabs(tsr[i]) < cfg.thr_shift_fac * min_period && tc >= tstart && tc <= tend;
+    // the time range first: outside it the shift and the coefficient are not computed (ws_needed)
+    bool good = tc >= tstart && tc <= tend && ccr[i] > cfg.thr_corr && fabs(tsr[i]) < cfg.thr_shift_fac * min_period;
     for (int k = max(1, i - nj); good && k <= min(nw - 1, i + nj); ++k)
       if (is_jump(k)) good = false;
     g[i] = good ? 1 : 0;
@@ -2525,11 +2625,16 @@ void fwat_win_sel_batch_(int* nstep, int* ntrace, double* dt, realw* obs, realw*
   hipLaunchKernelGGL(k_rows_f32, ttiles, dim3(256), 0, s, N, T, d_syn, d_synT);
   hipLaunchKernelGGL(k_ws_prep, dim3((unsigned)T), dim3(256), 0, s, N, *dt, *t0, *min_period, d_tp, d_obsT, d_synT,
                      d_Dn, d_Sn, d_noise);
-  const int nwv = nlen <= 1020 ? 4 : (nlen <= 2044 ? 2 : 1);  // at most 64 KB of LDS per workgroup
+  int nwv = 4;  // wavefronts per workgroup: at most 64 KB of LDS, more only for one wavefront of a long window
+  while (nwv > 1 && nwv * ws_lds(nlen) > 65536) nwv /= 2;
+  if (ws_lds(nlen) > 65536)
+    HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_ws_sliding),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)ws_lds(nlen)));
   hipLaunchKernelGGL(k_ws_sliding, dim3((unsigned)((nw + nwv - 1) / nwv), (unsigned)T), dim3(64 * nwv),
-                     (size_t)nwv * (2 * nlen + 7) * sizeof(double), s, N, nlen, nw, d_wt, d_Dn, d_Sn, d_ish);
+                     nwv * ws_lds(nlen), s, N, nlen, nw, *dt, *t0, *min_period, C.min_velocity, C.jump_fac, d_tp, d_dist,
+                     d_wt, d_Dn, d_Sn, d_ish);
   hipLaunchKernelGGL(k_ws_coef, dim3((unsigned)((nw + 255) / 256), (unsigned)T), dim3(256), 0, s, N, nlen, nw, *dt,
-                     d_wt, d_Dn, d_Sn, d_ish, d_ts, d_cc);
+                     *t0, *min_period, C.min_velocity, C.jump_fac, d_tp, d_dist, d_wt, d_Dn, d_Sn, d_ish, d_ts, d_cc);
   if (split)
     hipLaunchKernelGGL(k_ws_env, dim3((unsigned)T), dim3(MT_THREADS), 0, s, N, nfe, logMe, d_twe, d_Sn, d_g01,
                        d_g01 + (size_t)T * (Me + 1), d_env);
