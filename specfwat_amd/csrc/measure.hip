@@ -206,6 +206,20 @@ __global__ void __launch_bounds__(256) k_cc_rows(int ntrace, int nb, int nl, con
   }
 }
 
+// sum of lag index mm (lag mm + 1 - nlen) of two windows in the reference's order: the lags come
+// in fours and run over the union of their ranges, s zero outside its window
+__device__ __forceinline__ double lag_sum(int mm, int nlen, const double* dw, const double* sw) {
+  const int mb = mm & ~3;
+  const int lo = mb - (nlen - 1) > 0 ? mb - (nlen - 1) : 0, hi = mb + 3 < nlen - 1 ? mb + 3 : nlen - 1;
+  const int off = nlen - 1 - mm;
+  double c = 0.0;
+  for (int j = lo; j <= hi; ++j) {
+    const int k = j + off;
+    c = c + dw[j] * (k >= 0 && k < nlen ? sw[k] : 0.0);
+  }
+  return c;
+}
+
 // xcorr_shift, first stage: workgroup (trace, block of 1024 lags, 4 consecutive
 // lags per lane) of the full correlation; d and the matching stretch of s come
 // through LDS in chunks of 1024 samples taken in increasing i1, so each lag's
@@ -591,6 +605,126 @@ __device__ double mt_bmax(double v, double* red) {
   const double r = red[0];
   __syncthreads();
   return r;
+}
+
+// exp(-2 pi i j / nf), j < nf / 2
+__global__ void k_twiddles(int nf, double2* __restrict__ tw) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= nf / 2) return;
+  double sn, cn;
+  sincospi(-2.0 * (double)j / (double)nf, &sn, &cn);
+  tw[j] = make_double2(cn, sn);
+}
+
+// xcorr_shift by transforms: one workgroup per trace, the full correlation of its two windows as
+// the inverse transform of D conj(S) on nf >= 2 nl - 1 points in LDS (nf / 2 complex values), and
+// the lag of its first maximum.  A transform's rounding is at most about 5 log2(nf) u of its
+// 2-norm (u = 2^-53; windows scaled by powers of two into [-1, 1]): two times |d| |s| for the
+// spectra, sqrt(nl) |d| |s| for the inverse.  Lags within twice their sum of the largest value are
+// summed again as the reference sums them and compared, so the lag is the one of the direct sums
+// (k_cc_corr) in every case.  Real windows have one lag left and
+// sum nothing.  nl^2 products become nf log2(nf): two windows of 5,000 and 6,000 samples of
+// 1,200 traces 9.7 ms by direct sums.  G: nf / 2 + 1 spectrum values per trace.
+template <int NT>
+__global__ void __launch_bounds__(NT) k_cc_corr_fft(int nl, int nf, int logM, const double2* __restrict__ tw,
+                                                    const double* __restrict__ D, const double* __restrict__ S,
+                                                    double2* __restrict__ G, int* __restrict__ ishift) {
+  extern __shared__ double2 cbuf[];
+  __shared__ double red[NT];
+  __shared__ int ri[NT];
+  const int t = blockIdx.x, M = nf / 2, lane = threadIdx.x;
+  const unsigned shb = 32 - logM;
+  const double* d = D + (size_t)t * nl;
+  const double* s = S + (size_t)t * nl;
+  double2* g = G + (size_t)t * (M + 1);
+  double dm = 0.0, sm = 0.0, bad = 0.0;
+  for (int j = lane; j < nl; j += NT) {
+    dm = fmax(dm, fabs(d[j]));
+    sm = fmax(sm, fabs(s[j]));
+    if (!(fabs(d[j]) < INFINITY) || !(fabs(s[j]) < INFINITY)) bad = 1.0;
+  }
+  dm = mt_bmax<NT>(dm, red);
+  sm = mt_bmax<NT>(sm, red);
+  const bool odd = mt_bmax<NT>(bad, red) != 0.0;
+  const int de = dm > 0.0 && !odd ? ilogb(dm) + 1 : 0, se = sm > 0.0 && !odd ? ilogb(sm) + 1 : 0;
+  double nd = 0.0, ns = 0.0;
+  for (int j = lane; j < nl; j += NT) {
+    const double a = ldexp(d[j], -de), b = ldexp(s[j], -se);
+    nd += a * a;
+    ns += b * b;
+  }
+  nd = mt_bsum<NT>(nd, red);
+  ns = mt_bsum<NT>(ns, red);
+  const auto spectrum = [&](int k) {
+    if (k == 0 || k == M) {
+      const double2 z = cbuf[0];
+      return make_double2(k == 0 ? z.x + z.y : z.x - z.y, 0.0);
+    }
+    return mt_half(cbuf[k], cbuf[M - k], tw[k]);
+  };
+  mt_load_real<NT>(cbuf, M, logM, nl, [&](int n) { return ldexp(d[n], -de); });
+  mt_fft<NT>(cbuf, M, logM, nf, tw, false);
+  for (int k = lane; k <= M; k += NT) g[k] = spectrum(k);
+  __syncthreads();
+  mt_load_real<NT>(cbuf, M, logM, nl, [&](int n) { return ldexp(s[n], -se); });
+  mt_fft<NT>(cbuf, M, logM, nf, tw, false);
+  for (int k = lane; k <= M; k += NT) {
+    const double2 X = spectrum(k);
+    g[k] = cmul(g[k], make_double2(X.x, -X.y));
+  }
+  __syncthreads();
+  for (int k = lane; k < M; k += NT) cbuf[__brev((unsigned)k) >> shb] = mt_repack(g[k], g[M - k], tw[k]);
+  __syncthreads();
+  mt_fft<NT>(cbuf, M, logM, nf, tw, true);
+  // lag index m: lag l = m + 1 - nl at sample l (l >= 0) or nf + l
+  const int nlag = 2 * nl - 1;
+  const auto value = [&](int m) {
+    const int l = m + 1 - nl, n = l >= 0 ? l : nf + l;
+    const double2 z = cbuf[n >> 1];
+    return ((n & 1) ? z.y : z.x) / M;
+  };
+  double best = -INFINITY;
+  for (int m = lane; m < nlag; m += NT) best = fmax(best, value(m));
+  best = mt_bmax<NT>(best, red);
+  const double bound =
+      2.0 * (5.0 * (logM + 1) * (2.0 + sqrt((double)nl)) + 16.0) * 1.1102230246251565e-16 * sqrt(nd * ns);
+  const double thr = odd || !(bound < INFINITY) ? -INFINITY : best - bound;
+  double count = 0.0;
+  int only = 0x7fffffff;
+  for (int m = lane; m < nlag; m += NT)
+    if (!(value(m) < thr)) {
+      count += 1.0;
+      only = min(only, m);
+    }
+  count = mt_bsum<NT>(count, red);
+  double bv = -INFINITY;
+  int bm = 0x7fffffff;
+  if (!odd && (nd == 0.0 || ns == 0.0)) {
+    bm = 0;  // every sum is zero: the first lag
+  } else if (count == 1.0) {
+    bm = only;
+  } else {
+    for (int m = lane; m < nlag; m += NT)
+      if (!(value(m) < thr)) {
+        const double c = lag_sum(m, nl, d, s);
+        if (c > bv || (c == bv && m < bm)) { bv = c; bm = m; }
+      }
+  }
+  red[lane] = bv;
+  ri[lane] = bm;
+  __syncthreads();
+  for (int o = NT / 2; o > 0; o >>= 1) {
+    if (lane < o) {
+      const double v2 = red[lane + o];
+      const int m2 = ri[lane + o];
+      if (v2 > red[lane] || (v2 == red[lane] && m2 < ri[lane])) {
+        red[lane] = v2;
+        ri[lane] = m2;
+      }
+    }
+    __syncthreads();
+  }
+  if (lane == 0) ishift[t] = ri[0] + 1 - nl;
 }
 
 // sample-major traces [nstep][ntrace] to trace-major rows [ntrace][nstep]
@@ -1419,19 +1553,6 @@ __device__ __forceinline__ int2 ws_needed(int t, int nlen, int nw, double dt, do
 // the rest the positive one's.  Four lags per lane, one 16-byte LDS read of d and one of s per
 // sixteen products.  400 x 3 traces of 10,000 samples, nlen 201: 92.5 ms when every lag of every
 // window start was summed in double precision.
-__device__ __forceinline__ double ws_lag_sum(int mm, int nlen, const double* dw, const double* sw) {
-  // the lags come in fours and run over the union of their ranges, s zero outside its window
-  const int mb = mm & ~3;
-  const int lo = mb - (nlen - 1) > 0 ? mb - (nlen - 1) : 0, hi = mb + 3 < nlen - 1 ? mb + 3 : nlen - 1;
-  const int off = nlen - 1 - mm;
-  double c = 0.0;
-  for (int j = lo; j <= hi; ++j) {
-    const int k = j + off;
-    c = c + dw[j] * (k >= 0 && k < nlen ? sw[k] : 0.0);
-  }
-  return c;
-}
-
 // LDS of one wavefront of k_ws_sliding (bytes, a multiple of 16): dw, sw, the lags' fp32 sums,
 // fp32 d (padded to a multiple of four) and fp32 s twice, with room for the lags of the last four
 __host__ __device__ inline int ws_quad(int nlen) { return (nlen + 3) & ~3; }
@@ -1549,7 +1670,7 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
     bm = 0x7fffffff;
     for (int m = lane; m < nlag; m += 64)
       if (!(cs[m] < thr)) {
-        const double c = ws_lag_sum(m, nlen, dw, sw);
+        const double c = lag_sum(m, nlen, dw, sw);
         if (c > bv || (c == bv && m < bm)) { bv = c; bm = m; }
       }
     for (int o = 32; o > 0; o >>= 1) {
@@ -1890,6 +2011,68 @@ void window_range(double w0, double w1, double dt, int nstep, int& nb, int& nl) 
 }
 
 
+// xcorr_shift of a measurement's windows: by transforms while the whole correlation fits the LDS
+// transform (nl <= 8192) and is long enough to gain (nl > 128: below that one workgroup's direct
+// sums take no longer than the transform's passes), else by direct sums
+struct CcShift {
+  static bool fft(int nl) { return nl > 128 && nl <= MT_MAXM; }
+  static int points(int nl) {
+    int nf = 64;
+    while (nf < 2 * nl - 1) nf *= 2;
+    return nf;
+  }
+  int T;
+  hipStream_t s;
+  double* bv = nullptr;
+  int* bi = nullptr;
+  double2* G = nullptr;
+  std::vector<std::pair<int, double2*>> tw;  // one table per transform length
+  CcShift(int ntrace, const std::vector<int>& nls, hipStream_t stream) : T(ntrace), s(stream) {
+    size_t blocks = 0, spec = 0;
+    for (int nl : nls) {
+      if (fft(nl)) spec = std::max(spec, (size_t)points(nl) / 2 + 1);
+      else blocks = std::max(blocks, (size_t)(2 * nl - 1 + CC_LAGS - 1) / CC_LAGS);
+    }
+    bv = dev_alloc<double>(T * blocks);
+    bi = dev_alloc<int>(T * blocks);
+    G = dev_alloc<double2>(T * spec);
+  }
+  const double2* table(int nf) {
+    for (auto& p : tw)
+      if (p.first == nf) return p.second;
+    double2* d = dev_alloc<double2>((size_t)nf / 2);
+    hipLaunchKernelGGL(k_twiddles, dim3((unsigned)((nf / 2 + 255) / 256)), dim3(256), 0, s, nf, d);
+    tw.emplace_back(nf, d);
+    return d;
+  }
+  void run(int nl, const double* D, const double* S, int* ish) {
+    if (fft(nl)) {
+      const int nf = points(nl), M = nf / 2;
+      int logM = 0;
+      while ((1 << logM) < M) ++logM;
+      const double2* w = table(nf);
+      const size_t lds = (size_t)M * sizeof(double2);
+      const void* f = M >= 4096 ? reinterpret_cast<const void*>(k_cc_corr_fft<1024>)
+                                : reinterpret_cast<const void*>(k_cc_corr_fft<256>);
+      if (lds > 49152) HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      if (M >= 4096)
+        hipLaunchKernelGGL(k_cc_corr_fft<1024>, dim3((unsigned)T), dim3(1024), lds, s, nl, nf, logM, w, D, S, G, ish);
+      else
+        hipLaunchKernelGGL(k_cc_corr_fft<256>, dim3((unsigned)T), dim3(256), lds, s, nl, nf, logM, w, D, S, G, ish);
+      return;
+    }
+    const int nblk = (2 * nl - 1 + CC_LAGS - 1) / CC_LAGS;
+    hipLaunchKernelGGL(k_cc_corr, dim3((unsigned)nblk, (unsigned)T), dim3(256), 0, s, nl, D, S, bv, bi);
+    hipLaunchKernelGGL(k_cc_pick, dim3((unsigned)((T + MTPB - 1) / MTPB)), dim3(MTPB), 0, s, T, nblk, nl, bv, bi, ish);
+  }
+  void free_all() {
+    dev_free(bv);
+    dev_free(bi);
+    dev_free(G);
+    for (auto& p : tw) dev_free(p.second);
+  }
+};
+
 // dpss_windows (utils/dpss.f90:137-262) for the multitaper measurement: the
 // kmax largest eigenvalues of the DPSS tridiagonal matrix by bisection on
 // Sturm counts (the reference calls LAPACK dsterf), eigenvectors by the
@@ -2219,12 +2402,9 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   double* d_S = dev_alloc<double>((size_t)T * maxnl);
   double* d_tw = dev_alloc<double>(maxnl);
   double* d_A = dev_alloc<double>((size_t)T * maxnl);
-  const int maxblk = (2 * maxnl - 1 + CC_LAGS - 1) / CC_LAGS;
-  double* d_bv = dev_alloc<double>((size_t)T * maxblk);
-  int* d_bi = dev_alloc<int>((size_t)T * maxblk);
+  CcShift shift(T, nls, s);
   HIP_CHECK(hipEventRecord(e0, s));
   hipLaunchKernelGGL(k_fill_f32m, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, d_adj);
-  const unsigned nbk = (unsigned)((T + MTPB - 1) / MTPB);
   for (int w = 0; w < nw; ++w) {
     HIP_CHECK(hipMemcpyAsync(d_tw, tws[w].data(), nls[w] * sizeof(double), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_cc_rows, dim3((unsigned)((T + 63) / 64), (unsigned)((nls[w] + 63) / 64)), dim3(256), 0, s, T,
@@ -2233,10 +2413,7 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
       hipLaunchKernelGGL(k_ccc_finish, dim3((unsigned)T), dim3(256), 0, s, nls[w], *dt, C.cc_min, d_tw, d_D, d_S, d_A,
                          d_out + 8 * (size_t)w * T);
     } else {
-      const int nblk = (2 * nls[w] - 1 + CC_LAGS - 1) / CC_LAGS;
-      hipLaunchKernelGGL(k_cc_corr, dim3((unsigned)nblk, (unsigned)T), dim3(256), 0, s, nls[w], d_D, d_S, d_bv,
-                         d_bi);
-      hipLaunchKernelGGL(k_cc_pick, dim3(nbk), dim3(MTPB), 0, s, T, nblk, nls[w], d_bv, d_bi, d_ish);
+      shift.run(nls[w], d_D, d_S, d_ish);
       hipLaunchKernelGGL(k_cc_finish, dim3((unsigned)T), dim3(256), 0, s, nls[w], *dt, *imeas, C, d_tw, d_D, d_S,
                          d_ish, d_A, d_out + 8 * (size_t)w * T, 8);
     }
@@ -2275,7 +2452,8 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     misfits[t] = m;
   }
   dev_free(d_obs); dev_free(d_syn); dev_free(d_adj); dev_free(d_ish); dev_free(d_out); dev_free(d_D); dev_free(d_S);
-  dev_free(d_tw); dev_free(d_fw); dev_free(d_sos); dev_free(d_bv); dev_free(d_bi); dev_free(d_A);
+  dev_free(d_tw); dev_free(d_fw); dev_free(d_sos); dev_free(d_A);
+  shift.free_all();
   HIP_CHECK(hipEventDestroy(e0));
   HIP_CHECK(hipEventDestroy(e1));
   HIP_CHECK(hipStreamDestroy(s));
@@ -2364,9 +2542,7 @@ void fwat_mt_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   }
   double* d_tw = dev_alloc<double>(maxnl);
   double* d_tap = dev_alloc<double>((size_t)ntaper * maxnl);
-  const int maxblk = (2 * maxnl - 1 + CC_LAGS - 1) / CC_LAGS;
-  double* d_bv = dev_alloc<double>((size_t)T * maxblk);
-  int* d_bi = dev_alloc<int>((size_t)T * maxblk);
+  CcShift shift(T, nls, s);
   const int imcc = *imeas == 13 ? 11 : 12;
   float* d_obsT = dev_alloc<float>(n);
   float* d_synT = dev_alloc<float>(n);
@@ -2377,7 +2553,6 @@ void fwat_mt_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   hipLaunchKernelGGL(k_rows_f32, ttiles, dim3(256), 0, s, N, T, d_syn, d_synT);
   hipLaunchKernelGGL(k_mt_flim, dim3((unsigned)T), dim3(MT_THREADS), 0, s, N, T, *dt, nf, logM, d_twd, d_synT,
                      cfg[8], cfg[16], cfg[17], cfg[9], cfg[14], d_flim);
-  const unsigned nbk = (unsigned)((T + MTPB - 1) / MTPB);
   for (int w = 0; w < nw; ++w) {
     const int nl = nls[w];
     double* ow = d_out + 10 * (size_t)w * T;
@@ -2385,9 +2560,7 @@ void fwat_mt_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     HIP_CHECK(hipMemcpyAsync(d_tap, taps[w].data(), (size_t)ntaper * nl * sizeof(double), hipMemcpyHostToDevice, s));
     const dim3 tiles((unsigned)((T + 63) / 64), (unsigned)((nl + 63) / 64));
     hipLaunchKernelGGL(k_cc_rows, tiles, dim3(256), 0, s, T, nbs[w], nl, d_tw, d_obs, d_syn, d_D, d_S);
-    const int nblk = (2 * nl - 1 + CC_LAGS - 1) / CC_LAGS;
-    hipLaunchKernelGGL(k_cc_corr, dim3((unsigned)nblk, (unsigned)T), dim3(256), 0, s, nl, d_D, d_S, d_bv, d_bi);
-    hipLaunchKernelGGL(k_cc_pick, dim3(nbk), dim3(MTPB), 0, s, T, nblk, nl, d_bv, d_bi, d_ish);
+    shift.run(nl, d_D, d_S, d_ish);
     hipLaunchKernelGGL(k_cc_finish, dim3((unsigned)T), dim3(256), 0, s, nl, *dt, imcc, C, d_tw, d_D, d_S, d_ish, d_A,
                        ow, 10);
     hipLaunchKernelGGL(k_mt_window, dim3((unsigned)T), dim3(MT_THREADS), 0, s, N, T, *dt, nf, logM, d_twd, nbs[w], nl,
@@ -2427,8 +2600,9 @@ void fwat_mt_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     misfits[t] = m;
   }
   dev_free(d_obs); dev_free(d_syn); dev_free(d_adj); dev_free(d_twd); dev_free(d_ish); dev_free(d_flim);
-  dev_free(d_out); dev_free(d_D); dev_free(d_S); dev_free(d_A); dev_free(d_tw); dev_free(d_tap); dev_free(d_bv);
-  dev_free(d_bi); dev_free(d_fw); dev_free(d_sos); dev_free(d_g01); dev_free(d_g2); dev_free(d_obsT); dev_free(d_synT);
+  dev_free(d_out); dev_free(d_D); dev_free(d_S); dev_free(d_A); dev_free(d_tw); dev_free(d_tap);
+  shift.free_all();
+  dev_free(d_fw); dev_free(d_sos); dev_free(d_g01); dev_free(d_g2); dev_free(d_obsT); dev_free(d_synT);
   dev_free(jack.pd); dev_free(jack.pb); dev_free(jack.xj); dev_free(jack.er);
   HIP_CHECK(hipEventDestroy(ev0));
   HIP_CHECK(hipEventDestroy(ev1));
@@ -2510,7 +2684,6 @@ void fwat_ep_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
                        d_twd + toff[w], d_tw + woff[w], d_D, d_S, d_g01, d_g01 + (size_t)T * (M + 1), d_R, d_A, ow);
     hipLaunchKernelGGL(k_mt_put, tiles, dim3(256), 0, s, T, nbs[w], nl, d_A, ow, 8, d_adj);
   }
-  const unsigned nbk = (unsigned)((T + MTPB - 1) / MTPB);
   std::vector<double> fw;
   double* d_fw = nullptr;
   float* d_sos = nullptr;
