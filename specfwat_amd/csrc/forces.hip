@@ -53,6 +53,8 @@ struct ForceArgs {
   int grouped;  // element-local force rows grouped by reader (sem_floc_slot), else in local-point order
   int elem_begin, elem_count;
   int nblocks_padded;
+  int nblk;      // workgroups of the element pass; the launch's others take seismograms
+  SemSeismo se;
   realw xix_regular, jacobian_regular;
   float scale_k, scale_m, scale_jinv, scale_jac;
   const realw* u0;
@@ -101,6 +103,10 @@ __global__ __launch_bounds__(128) void k_forces(ForceArgs A) {
   __shared__ realw s_t[9][128];
 
   const int t = threadIdx.x;
+  if (NF == 1 && ASM == 1 && (int)blockIdx.x >= A.nblk) {  // block-uniform
+    sem_seismo_block(A.se, blockIdx.x - A.nblk, &s_u[0][0]);
+    return;
+  }
   if (t < 125) s_tab[t] = A.tables[t];
   const int lb = xcd_remap(blockIdx.x, A.nblocks_padded);
   if (lb >= A.elem_count) return;  // block-uniform
@@ -324,6 +330,10 @@ __device__ __forceinline__ void forces_reg_body(const ForceArgs& A) {
   __shared__ realw s_u[3][128];
   __shared__ realw s_s[6][128];
   const int t = threadIdx.x;
+  if (NF == 1 && (int)blockIdx.x >= A.nblk) {  // block-uniform
+    sem_seismo_block(A.se, blockIdx.x - A.nblk, &s_u[0][0]);
+    return;
+  }
   if (t < 125) s_tab[t] = A.tables[t];
   const bool act = t < 125;
   const int tt = act ? t : 124;
@@ -349,7 +359,7 @@ __device__ __forceinline__ void forces_reg_body(const ForceArgs& A) {
   const int La0 = 5 * J + 25 * K, Lb0 = I + 25 * K, Lc0 = I + 5 * J;
   // XCD-aware persistent schedule: XCD x = blockIdx % 8 owns elements
   // [x*chunk, (x+1)*chunk); its workgroups stride through that run together.
-  const int nblk = gridDim.x;
+  const int nblk = A.nblk;
   const int x = blockIdx.x & 7, per_xcd = nblk >> 3, slot = blockIdx.x >> 3;
   const int chunk = (A.elem_count + 7) >> 3;
   const int e_end = min(A.elem_count, (x + 1) * chunk);
@@ -490,6 +500,10 @@ __device__ __forceinline__ void forces_reg_pipe_body(const ForceArgs& A) {
   __shared__ realw s_u[3][128];
   __shared__ realw s_s[6][128];
   const int t = threadIdx.x;
+  if (NF == 1 && (int)blockIdx.x >= A.nblk) {  // block-uniform
+    sem_seismo_block(A.se, blockIdx.x - A.nblk, &s_u[0][0]);
+    return;
+  }
   if (t < 125) s_tab[t] = A.tables[t];
   const bool act = t < 125;
   const int tt = act ? t : 124;
@@ -513,7 +527,7 @@ __device__ __forceinline__ void forces_reg_pipe_body(const ForceArgs& A) {
     }
   }
   const int La0 = 5 * J + 25 * K, Lb0 = I + 25 * K, Lc0 = I + 5 * J;
-  const int nblk = gridDim.x;
+  const int nblk = A.nblk;
   const int x = blockIdx.x & 7, per_xcd = nblk >> 3, slot = blockIdx.x >> 3;
   const int chunk = (A.elem_count + 7) >> 3;
   const int e_end = min(A.elem_count, (x + 1) * chunk);
@@ -662,6 +676,10 @@ __device__ __forceinline__ void forces_reg_pp_body(const ForceArgs& A) {
   __shared__ realw s_u[2][NF][3][128];
   __shared__ realw s_s[2][NF][6][128];
   const int t = threadIdx.x;
+  if (NF == 1 && (int)blockIdx.x >= A.nblk) {  // block-uniform
+    sem_seismo_block(A.se, blockIdx.x - A.nblk, &s_u[0][0][0][0]);
+    return;
+  }
   if (t < 125) s_tab[t] = A.tables[t];
   const bool act = t < 125;
   const int tt = act ? t : 124;
@@ -685,7 +703,7 @@ __device__ __forceinline__ void forces_reg_pp_body(const ForceArgs& A) {
     }
   }
   const int La0 = 5 * J + 25 * K, Lb0 = I + 25 * K, Lc0 = I + 5 * J;
-  const int nblk = gridDim.x;
+  const int nblk = A.nblk;
   const int x = blockIdx.x & 7, per_xcd = nblk >> 3, slot = blockIdx.x >> 3;
   const int chunk = (A.elem_count + 7) >> 3;
   const int e_end = min(A.elem_count, (x + 1) * chunk);
@@ -926,8 +944,9 @@ int reg_grid(int elem_count, int blocks_per_cu) {
 }
 
 template <int NF, bool ANISO, int KMODE, int SP>
-void launch_reg(const ForceArgs& a, hipStream_t s, int blocks_per_cu, int variant = 1) {
-  const int nb = reg_grid(a.elem_count, blocks_per_cu);
+void launch_reg(ForceArgs a, hipStream_t s, int blocks_per_cu, int variant = 1) {
+  a.nblk = reg_grid(a.elem_count, blocks_per_cu);
+  const int nb = a.nblk + a.se.nrec;
   if constexpr (ANISO) SEM_LAUNCH((k_forces_reg_aniso<NF, ANISO, KMODE, SP>), dim3(nb), dim3(128), 0, s, a);
   else if (variant == 2) SEM_LAUNCH((k_forces_reg_pipe<NF, KMODE, SP>), dim3(nb), dim3(128), 0, s, a);
   else if (variant == 3 && a.rm) SEM_LAUNCH((k_forces_reg_pp<NF, KMODE, SP, false, true>), dim3(nb), dim3(128), 0, s, a);
@@ -937,8 +956,9 @@ void launch_reg(const ForceArgs& a, hipStream_t s, int blocks_per_cu, int varian
 }
 
 template <int NF, bool ANISO, int KMODE, int SP>
-void launch_t(const ForceArgs& a, hipStream_t s) {
-  const int nb = a.nblocks_padded;
+void launch_t(ForceArgs a, hipStream_t s) {
+  a.nblk = a.nblocks_padded;
+  const int nb = a.nblk + a.se.nrec;
   if (a.floc0)
     SEM_LAUNCH((k_forces<NF, ANISO, KMODE, SP, 1>), dim3(nb), dim3(128), 0, s, a);
   else
@@ -1009,9 +1029,14 @@ bool sem_interior_active(const SemMesh* m, int nfields) {
 }
 
 void sem_launch_forces(SemMesh* m, int nfields, int kernel_mode, int elem_begin, int elem_count,
-                       realw deltat, const int* elem_list, bool gather, const SemInterior* in) {
+                       realw deltat, const int* elem_list, bool gather, const SemInterior* in,
+                       const SemSeismo* se) {
   if (elem_count <= 0) return;
   ForceArgs a{};
+  if (se) {
+    if (nfields != 1 || !gather) SEM_FAIL("seismograms ride with one-field gather passes only");
+    a.se = *se;
+  }
   a.ibool = m->d_ibool;
   a.irregular = m->d_irregular;
   a.jinv10 = m->d_jinv10;

@@ -450,11 +450,42 @@ struct SemInterior {
   double dtk;
 };
 
+// Seismograms of one step: the displacement u interpolated at nrec receivers into row [nrec][3].
+struct SemSeismo {
+  int nrec = 0;
+  const int* riglob = nullptr;
+  const realw* rh = nullptr;
+  const realw* u = nullptr;
+  realw* row = nullptr;
+};
+
+// One receiver's samples by a 128-lane workgroup, s: 3 * 128 reals of its LDS.
+__device__ __forceinline__ void sem_seismo_block(const SemSeismo& S, int r, realw* s) {
+  const int t = threadIdx.x;
+  realw x = 0, y = 0, z = 0;
+  if (t < 125) {
+    const realw h = S.rh[(size_t)r * 125 + t];
+    const size_t g = (size_t)S.riglob[(size_t)r * 125 + t];
+    x = h * S.u[3 * g]; y = h * S.u[3 * g + 1]; z = h * S.u[3 * g + 2];
+  }
+  s[t] = x; s[128 + t] = y; s[256 + t] = z;
+  __syncthreads();
+  for (int w = 64; w > 0; w >>= 1) {
+    if (t < w) { s[t] += s[t + w]; s[128 + t] += s[128 + t + w]; s[256 + t] += s[256 + t + w]; }
+    __syncthreads();
+  }
+  if (t == 0) { S.row[3 * r] = s[0]; S.row[3 * r + 1] = s[128]; S.row[3 * r + 2] = s[256]; }
+}
+
 // internal launchers shared between the C-ABI files
 // (in: the element pass also finishes the element-interior points when
-// sem_interior_active(m, nfields); the assembly then covers [0, n_shared) only)
+// sem_interior_active(m, nfields); the assembly then covers [0, n_shared) only.
+// se: the launch of a one-field gather pass also takes these seismograms, in workgroups of their
+// own after the elements'; it must not change the receivers' points, which it never does: they
+// are shared points)
 void sem_launch_forces(SemMesh* m, int nfields, int kernel_mode, int elem_begin, int elem_count,
-                       realw deltat, const int* elem_list, bool gather, const SemInterior* in = nullptr);
+                       realw deltat, const int* elem_list, bool gather, const SemInterior* in = nullptr,
+                       const SemSeismo* se = nullptr);
 // true when a whole-mesh fused element pass of nfields fields finishes the element-interior points
 bool sem_interior_active(const SemMesh* m, int nfields);
 // host <-> device copies of three point fields (u, v, a) of size 3 * nglob in the

@@ -74,6 +74,112 @@ __global__ void k_corrector(int nglob, realw* __restrict__ v, realw* __restrict_
   }
 }
 
+// Incident wavefield of one step for FK injection: rows k and k + 1 of the
+// stored velocity and traction and the weight w of row k + 1 (no injection
+// when v0 is null)
+struct FkStep {
+  const realw *v0 = nullptr, *v1 = nullptr, *t0 = nullptr, *t1 = nullptr;
+  realw w = 0;
+};
+
+// Stacey term of face point q, SPECFEM's compute_stacey_viscoelastic with
+// injection: the absorbing traction of the velocity relative to the
+// incident one, minus the incident traction, times jacobian2Dw
+__device__ __forceinline__ void stacey_point(size_t q, const realw* __restrict__ C, realw vx, realw vy, realw vz,
+                                             const FkStep& fk, realw& tx, realw& ty, realw& tz) {
+  const realw nx = C[0], ny = C[1], nz = C[2], jw = C[3], rvp = C[4], rvs = C[5];
+  realw ix = 0, iy = 0, iz = 0;
+  if (fk.v0) {
+    const realw w0 = (realw)1 - fk.w, w1 = fk.w;
+    vx -= w0 * fk.v0[3 * q] + w1 * fk.v1[3 * q];
+    vy -= w0 * fk.v0[3 * q + 1] + w1 * fk.v1[3 * q + 1];
+    vz -= w0 * fk.v0[3 * q + 2] + w1 * fk.v1[3 * q + 2];
+    ix = w0 * fk.t0[3 * q] + w1 * fk.t1[3 * q];
+    iy = w0 * fk.t0[3 * q + 1] + w1 * fk.t1[3 * q + 1];
+    iz = w0 * fk.t0[3 * q + 2] + w1 * fk.t1[3 * q + 2];
+  }
+  const realw vn = vx * nx + vy * ny + vz * nz;
+  tx = (rvp * vn * nx + rvs * (vx - vn * nx) - ix) * jw;
+  ty = (rvp * vn * ny + rvs * (vy - vn * ny) - iy) * jw;
+  tz = (rvp * vn * nz + rvs * (vz - vn * nz) - iz) * jw;
+}
+
+// Stacey term of the first field taken inside the assembly: the velocity it needs is the point's
+// own predicted one, which the assembly holds, so a launch per step that read it again and wrote
+// the traction out is saved.  coef null: the traction comes from AsmField::face.  rec: where a
+// SAVE_FORWARD run stores it, or null.
+struct AsmStacey {
+  const realw* coef = nullptr;
+  realw* rec = nullptr;
+  FkStep fk;
+};
+
+// Boundary, source, receiver and left-over single element terms of point g's row from q on, added
+// in row order (element terms lead the row, receiver terms end it); v0: the point's predicted
+// velocity.  The receivers' terms are read four at a time - a point of an element with many
+// receivers has one term for each, and one dependent load after the other made such points the
+// whole launch's time (12.5 us on a mesh whose element pass takes 6) - and not at all
+// when no field takes adjoint sources.
+template <bool TWO>
+__device__ __forceinline__ void assemble_tail(int q, int q1, const int* __restrict__ idx, int nloc, int nfp, int nsp,
+                                              const realw* __restrict__ sarr, const realw* __restrict__ rech,
+                                              const AsmField& F0, const AsmField& F1, const AsmStacey& S0,
+                                              const realw* v0, realw* f) {
+  const int first_rec = nloc + nfp + nsp;
+  for (; q < q1; ++q) {
+    const int c = idx[q];
+    if (c >= first_rec) break;
+    if (c < nloc) {
+      const realw* P = F0.floc + 3 * (size_t)c;
+      f[0] += P[0]; f[1] += P[1]; f[2] += P[2];
+      if (TWO) {
+        const realw* B = F1.floc + 3 * (size_t)c;
+        f[3] += B[0]; f[4] += B[1]; f[5] += B[2];
+      }
+    } else if (c < nloc + nfp) {
+      const size_t p = (size_t)(c - nloc);
+      if (S0.coef) {
+        realw tx, ty, tz;
+        stacey_point(p, S0.coef + 8 * p, v0[0], v0[1], v0[2], S0.fk, tx, ty, tz);
+        if (S0.rec) store3(S0.rec + 3 * p, tx, ty, tz);
+        f[0] -= tx; f[1] -= ty; f[2] -= tz;
+      } else if (F0.face) {
+        f[0] -= F0.face[3 * p]; f[1] -= F0.face[3 * p + 1]; f[2] -= F0.face[3 * p + 2];
+      }
+      if (TWO && F1.face) { f[3] -= F1.face[3 * p]; f[4] -= F1.face[3 * p + 1]; f[5] -= F1.face[3 * p + 2]; }
+    } else {
+      const int p = c - nloc - nfp;
+      const realw* S = sarr + 3 * (size_t)p;
+      if (F0.stf) { const realw w = (realw)F0.stf[p / 125]; f[0] = fmaf(S[0], w, f[0]); f[1] = fmaf(S[1], w, f[1]); f[2] = fmaf(S[2], w, f[2]); }
+      if (TWO && F1.stf) { const realw w = (realw)F1.stf[p / 125]; f[3] = fmaf(S[0], w, f[3]); f[4] = fmaf(S[1], w, f[4]); f[5] = fmaf(S[2], w, f[5]); }
+    }
+  }
+  if (!F0.adj && !(TWO && F1.adj)) return;
+  for (; q < q1; q += 4) {
+    realw h[4], x[4][3], y[4][3];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const int p = idx[min(q + n, q1 - 1)] - first_rec;  // the last receiver again past the row's end
+      const size_t r = 3 * (size_t)(p / 125);
+      h[n] = rech[p];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        x[n][c] = F0.adj ? F0.adj[r + c] : 0.0f;
+        if (TWO) y[n][c] = F1.adj ? F1.adj[r + c] : 0.0f;
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      if (q + n < q1) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          if (F0.adj) f[c] = fmaf(h[n], x[n][c], f[c]);
+          if (TWO && F1.adj) f[3 + c] = fmaf(h[n], y[n][c], f[3 + c]);
+        }
+      }
+  }
+}
+
 // Gather assembly fused with the Newmark update.  For every global point:
 //   f = sum of its contributions (CSR, fixed order): element-local forces,
 //       minus the Stacey face traction, plus sourcearray * stf, plus
@@ -88,7 +194,7 @@ template <bool LAST, bool TWO>
 __global__ void k_assemble(int npts, const int* __restrict__ glist, const int* __restrict__ off,
                            const int* __restrict__ idx, int nloc, int nfp, int nsp, const realw* __restrict__ sarr,
                            const realw* __restrict__ rech, const realw* __restrict__ rm,
-                           AsmField F0, AsmField F1, double* __restrict__ rho_kl,
+                           AsmField F0, AsmField F1, AsmStacey S0, double* __restrict__ rho_kl,
                            float* __restrict__ rho_part, int flush, double* __restrict__ hess_kl, double dtk) {
   const int h = blockIdx.x * blockDim.x + threadIdx.x;
   if (h >= npts) return;
@@ -115,68 +221,10 @@ __global__ void k_assemble(int npts, const int* __restrict__ glist, const int* _
     f0x += a0; f0y += a1; f0z += a2;
     f0x += b0; f0y += b1; f0z += b2;
   }
-  for (; q < q1; ++q) {
-    const int c = idx[q];
-    if (c < nloc) {
-      const realw* P = F0.floc + 3 * (size_t)c;
-      f0x += P[0]; f0y += P[1]; f0z += P[2];
-      if (TWO) {
-        const realw* B = F1.floc + 3 * (size_t)c;
-        f1x += B[0]; f1y += B[1]; f1z += B[2];
-      }
-    } else if (c < nloc + nfp) {
-      const size_t p = 3 * (size_t)(c - nloc);
-      if (F0.face) { f0x -= F0.face[p]; f0y -= F0.face[p + 1]; f0z -= F0.face[p + 2]; }
-      if (TWO && F1.face) { f1x -= F1.face[p]; f1y -= F1.face[p + 1]; f1z -= F1.face[p + 2]; }
-    } else if (c < nloc + nfp + nsp) {
-      const int p = c - nloc - nfp;
-      const realw* S = sarr + 3 * (size_t)p;
-      if (F0.stf) { const realw w = (realw)F0.stf[p / 125]; f0x = fmaf(S[0], w, f0x); f0y = fmaf(S[1], w, f0y); f0z = fmaf(S[2], w, f0z); }
-      if (TWO && F1.stf) { const realw w = (realw)F1.stf[p / 125]; f1x = fmaf(S[0], w, f1x); f1y = fmaf(S[1], w, f1y); f1z = fmaf(S[2], w, f1z); }
-    } else {
-      const int p = c - nloc - nfp - nsp;
-      const realw h = rech[p];
-      const size_t r = 3 * (size_t)(p / 125);
-      if (F0.adj) { f0x = fmaf(h, F0.adj[r], f0x); f0y = fmaf(h, F0.adj[r + 1], f0y); f0z = fmaf(h, F0.adj[r + 2], f0z); }
-      if (TWO && F1.adj) { f1x = fmaf(h, F1.adj[r], f1x); f1y = fmaf(h, F1.adj[r + 1], f1y); f1z = fmaf(h, F1.adj[r + 2], f1z); }
-    }
-  }
-  newmark_point<TWO>((size_t)g, P, f0x, f0y, f0z, f1x, f1y, f1z, F0, F1, LAST, rho_kl, rho_part, flush != 0,
+  realw f[6] = {f0x, f0y, f0z, f1x, f1y, f1z};
+  assemble_tail<TWO>(q, q1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, S0, P.v0, f);
+  newmark_point<TWO>((size_t)g, P, f[0], f[1], f[2], f[3], f[4], f[5], F0, F1, LAST, rho_kl, rho_part, flush != 0,
                      hess_kl, dtk);
-}
-
-// Boundary and single element terms of point g's row from q on (the tail of
-// k_assemble's loop), added in row order.
-template <bool TWO>
-__device__ __forceinline__ void assemble_tail(int q, int q1, const int* __restrict__ idx, int nloc, int nfp, int nsp,
-                                              const realw* __restrict__ sarr, const realw* __restrict__ rech,
-                                              const AsmField& F0, const AsmField& F1, realw* f) {
-  for (; q < q1; ++q) {
-    const int c = idx[q];
-    if (c < nloc) {
-      const realw* P = F0.floc + 3 * (size_t)c;
-      f[0] += P[0]; f[1] += P[1]; f[2] += P[2];
-      if (TWO) {
-        const realw* B = F1.floc + 3 * (size_t)c;
-        f[3] += B[0]; f[4] += B[1]; f[5] += B[2];
-      }
-    } else if (c < nloc + nfp) {
-      const size_t p = 3 * (size_t)(c - nloc);
-      if (F0.face) { f[0] -= F0.face[p]; f[1] -= F0.face[p + 1]; f[2] -= F0.face[p + 2]; }
-      if (TWO && F1.face) { f[3] -= F1.face[p]; f[4] -= F1.face[p + 1]; f[5] -= F1.face[p + 2]; }
-    } else if (c < nloc + nfp + nsp) {
-      const int p = c - nloc - nfp;
-      const realw* S = sarr + 3 * (size_t)p;
-      if (F0.stf) { const realw w = (realw)F0.stf[p / 125]; f[0] = fmaf(S[0], w, f[0]); f[1] = fmaf(S[1], w, f[1]); f[2] = fmaf(S[2], w, f[2]); }
-      if (TWO && F1.stf) { const realw w = (realw)F1.stf[p / 125]; f[3] = fmaf(S[0], w, f[3]); f[4] = fmaf(S[1], w, f[4]); f[5] = fmaf(S[2], w, f[5]); }
-    } else {
-      const int p = c - nloc - nfp - nsp;
-      const realw h = rech[p];
-      const size_t r = 3 * (size_t)(p / 125);
-      if (F0.adj) { f[0] = fmaf(h, F0.adj[r], f[0]); f[1] = fmaf(h, F0.adj[r + 1], f[1]); f[2] = fmaf(h, F0.adj[r + 2], f[2]); }
-      if (TWO && F1.adj) { f[3] = fmaf(h, F1.adj[r], f[3]); f[4] = fmaf(h, F1.adj[r + 1], f[4]); f[5] = fmaf(h, F1.adj[r + 2], f[5]); }
-    }
-  }
 }
 
 // k_assemble with two points per lane (points h and h + blockDim.x of the
@@ -188,7 +236,7 @@ template <bool LAST, bool TWO>
 __global__ void k_assemble2(int npts, const int* __restrict__ glist, const int* __restrict__ off,
                             const int* __restrict__ idx, int nloc, int nfp, int nsp, const realw* __restrict__ sarr,
                             const realw* __restrict__ rech, const realw* __restrict__ rm,
-                            AsmField F0, AsmField F1, double* __restrict__ rho_kl,
+                            AsmField F0, AsmField F1, AsmStacey S0, double* __restrict__ rho_kl,
                             float* __restrict__ rho_part, int flush, double* __restrict__ hess_kl, double dtk) {
   const int ha = blockIdx.x * 2 * blockDim.x + threadIdx.x, hb = ha + blockDim.x;
   if (ha >= npts) return;
@@ -261,43 +309,13 @@ __global__ void k_assemble2(int npts, const int* __restrict__ glist, const int* 
       qb += 2;
     }
   }
-  assemble_tail<TWO>(qa, qa1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, fa);
-  if (vb) assemble_tail<TWO>(qb, qb1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, fb);
+  assemble_tail<TWO>(qa, qa1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, S0, Pa.v0, fa);
+  if (vb) assemble_tail<TWO>(qb, qb1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, S0, Pb.v0, fb);
   newmark_point<TWO>((size_t)ga, Pa, fa[0], fa[1], fa[2], fa[3], fa[4], fa[5], F0, F1, LAST, rho_kl, rho_part,
                      flush != 0, hess_kl, dtk);
   if (vb)
     newmark_point<TWO>((size_t)gb, Pb, fb[0], fb[1], fb[2], fb[3], fb[4], fb[5], F0, F1, LAST, rho_kl, rho_part,
                        flush != 0, hess_kl, dtk);
-}
-
-// Incident wavefield of one step for FK injection: rows k and k + 1 of the
-// stored velocity and traction and the weight w of row k + 1 (no injection
-// when v0 is null)
-struct FkStep {
-  const realw *v0 = nullptr, *v1 = nullptr, *t0 = nullptr, *t1 = nullptr;
-  realw w = 0;
-};
-
-// Stacey term of face point q, SPECFEM's compute_stacey_viscoelastic with
-// injection: the absorbing traction of the velocity relative to the
-// incident one, minus the incident traction, times jacobian2Dw
-__device__ __forceinline__ void stacey_point(size_t q, const realw* __restrict__ C, realw vx, realw vy, realw vz,
-                                             const FkStep& fk, realw& tx, realw& ty, realw& tz) {
-  const realw nx = C[0], ny = C[1], nz = C[2], jw = C[3], rvp = C[4], rvs = C[5];
-  realw ix = 0, iy = 0, iz = 0;
-  if (fk.v0) {
-    const realw w0 = (realw)1 - fk.w, w1 = fk.w;
-    vx -= w0 * fk.v0[3 * q] + w1 * fk.v1[3 * q];
-    vy -= w0 * fk.v0[3 * q + 1] + w1 * fk.v1[3 * q + 1];
-    vz -= w0 * fk.v0[3 * q + 2] + w1 * fk.v1[3 * q + 2];
-    ix = w0 * fk.t0[3 * q] + w1 * fk.t1[3 * q];
-    iy = w0 * fk.t0[3 * q + 1] + w1 * fk.t1[3 * q + 1];
-    iz = w0 * fk.t0[3 * q + 2] + w1 * fk.t1[3 * q + 2];
-  }
-  const realw vn = vx * nx + vy * ny + vz * nz;
-  tx = (rvp * vn * nx + rvs * (vx - vn * nx) - ix) * jw;
-  ty = (rvp * vn * ny + rvs * (vy - vn * ny) - iy) * jw;
-  tz = (rvp * vn * nz + rvs * (vz - vn * nz) - iz) * jw;
 }
 
 // Stacey traction of one field written per face point (no scatter):
@@ -423,24 +441,9 @@ __global__ void k_add_adjoint(int nrec, const int* __restrict__ riglob, const re
 }
 
 // seismograms: one 128-lane block per receiver, Lagrange interpolation of u
-__global__ __launch_bounds__(128) void k_seismo(int nrec, const int* __restrict__ riglob,
-                                                const realw* __restrict__ rh, const realw* __restrict__ u,
-                                                realw* __restrict__ row) {
-  __shared__ realw s[3][128];
-  const int r = blockIdx.x, t = threadIdx.x;
-  realw x = 0, y = 0, z = 0;
-  if (t < 125) {
-    const realw h = rh[(size_t)r * 125 + t];
-    const size_t g = (size_t)riglob[(size_t)r * 125 + t];
-    x = h * u[3 * g]; y = h * u[3 * g + 1]; z = h * u[3 * g + 2];
-  }
-  s[0][t] = x; s[1][t] = y; s[2][t] = z;
-  __syncthreads();
-  for (int w = 64; w > 0; w >>= 1) {
-    if (t < w) { s[0][t] += s[0][t + w]; s[1][t] += s[1][t + w]; s[2][t] += s[2][t + w]; }
-    __syncthreads();
-  }
-  if (t == 0) { row[3 * r] = s[0][0]; row[3 * r + 1] = s[1][0]; row[3 * r + 2] = s[2][0]; }
+__global__ __launch_bounds__(128) void k_seismo(SemSeismo S) {
+  __shared__ realw s[3 * 128];
+  sem_seismo_block(S, blockIdx.x, s);
 }
 
 __global__ void k_copy4(const float4* __restrict__ a, float4* __restrict__ b, size_t n4) {
@@ -559,10 +562,21 @@ void stage_stacey_face(SemMesh* m, const realw* v, realw* out, int it = 0) {
                      m->d_face_coef, v, out, fk_step(m, it));
 }
 
+// Stacey term of the forward or adjoint field, taken inside the assembly; rec: record to store or
+// null; it: the forward step (1-based) whose incident field is injected, 0 for none
+AsmStacey asm_stacey(const SemMesh* m, realw* rec, int it) {
+  AsmStacey S;
+  if (!m->absorbing || m->nfaces == 0) return S;
+  S.coef = m->d_face_coef;
+  S.rec = rec;
+  S.fk = fk_step(m, it);
+  return S;
+}
+
 // Assembly + Newmark of points 0..nglob-1 (0..n_shared-1 when the element pass
 // finished the others: interior), or of slab `slab`'s point list.
-void stage_assemble(SemMesh* m, bool last, bool two, const AsmField& F0, const AsmField& F1, double dtk,
-                    int slab = -1, bool interior = false) {
+void stage_assemble(SemMesh* m, bool last, bool two, const AsmField& F0, const AsmField& F1, const AsmStacey& S0,
+                    double dtk, int slab = -1, bool interior = false) {
   const int nfp = m->absorbing ? m->nfaces * 25 : 0;
   float* rho_part = m->kernel_block > 1 ? m->d_rho_part : nullptr;
   const int nloc = m->nspec * 125, nsp = m->nsources * 125;
@@ -578,7 +592,7 @@ void stage_assemble(SemMesh* m, bool last, bool two, const AsmField& F0, const A
     const dim3 g2((unsigned)((npts + 2 * tpb - 1) / (2 * tpb)));
 #define ASM2(L, T, RK, RP, FL, HK)                                                                              \
   SEM_LAUNCH((k_assemble2<L, T>), g2, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp, nsp, \
-             m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, RK, RP, FL, HK, dtk)
+             m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, RK, RP, FL, HK, dtk)
     if (two) {
       if (last) ASM2(true, true, m->d_rho_kl_glob, rho_part, m->kernel_flush, m->d_hess_kl_glob);
       else ASM2(false, true, m->d_rho_kl_glob, rho_part, m->kernel_flush, m->d_hess_kl_glob);
@@ -593,29 +607,32 @@ void stage_assemble(SemMesh* m, bool last, bool two, const AsmField& F0, const A
   if (two) {
     if (last)
       SEM_LAUNCH((k_assemble<true, true>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, m->d_rho_kl_glob, rho_part, m->kernel_flush,
+                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, m->d_rho_kl_glob, rho_part, m->kernel_flush,
                          m->d_hess_kl_glob, dtk);
     else
       SEM_LAUNCH((k_assemble<false, true>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, m->d_rho_kl_glob, rho_part, m->kernel_flush,
+                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, m->d_rho_kl_glob, rho_part, m->kernel_flush,
                          m->d_hess_kl_glob, dtk);
   } else {
     if (last)
       SEM_LAUNCH((k_assemble<true, false>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, (double*)nullptr, (float*)nullptr, 1,
+                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, (double*)nullptr, (float*)nullptr, 1,
                          (double*)nullptr, dtk);
     else
       SEM_LAUNCH((k_assemble<false, false>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, (double*)nullptr, (float*)nullptr, 1,
+                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, (double*)nullptr, (float*)nullptr, 1,
                          (double*)nullptr, dtk);
   }
 }
 
+SemSeismo seismo_row(const SemMesh* m, int it0) {
+  if (it0 < 0 || it0 >= m->nstep) SEM_FAIL("seismogram index %d outside NSTEP=%d", it0 + 1, m->nstep);
+  return SemSeismo{m->nrec, m->d_rec_iglob, m->d_rec_h, m->d_displ, m->d_seismograms + (size_t)it0 * m->nrec * 3};
+}
+
 void stage_seismo(SemMesh* m, int it0) {
   if (m->nrec == 0) return;
-  if (it0 < 0 || it0 >= m->nstep) SEM_FAIL("seismogram index %d outside NSTEP=%d", it0 + 1, m->nstep);
-  hipLaunchKernelGGL(k_seismo, dim3(m->nrec), dim3(128), 0, m->stream, m->nrec, m->d_rec_iglob,
-                     m->d_rec_h, m->d_displ, m->d_seismograms + (size_t)it0 * m->nrec * 3);
+  hipLaunchKernelGGL(k_seismo, dim3(m->nrec), dim3(128), 0, m->stream, seismo_row(m, it0));
 }
 
 // Timing samples every timer_stride(N)-th step (at most about 256 steps of a
@@ -701,9 +718,9 @@ struct LoopGraph {
 };
 
 void stage_forces_timed(SemMesh* m, int nfields, int kmode, realw dt, ForceTimer* tm, bool gather,
-                        const SemInterior* in = nullptr) {
+                        const SemInterior* in = nullptr, const SemSeismo* se = nullptr) {
   if (tm) tm->open(m->stream);
-  sem_launch_forces(m, nfields, kmode, 0, m->nspec, dt, nullptr, gather, in);
+  sem_launch_forces(m, nfields, kmode, 0, m->nspec, dt, nullptr, gather, in, se);
   if (tm) tm->close(m->stream);
 }
 
@@ -1035,13 +1052,9 @@ void fwat_iterate_time_(long* Mesh_pointer, int* SIMULATION_TYPE, realw* DT, int
       stage_predictor(m, false, dt);  // u_1, v_1/2 from the initial state
       for (int it = 1; it <= N; ++it) {
         step_begin(it);
-        realw* face = nullptr;
-        if (m->absorbing && m->nfaces) {
-          face = smode ? m->d_stacey_store + (size_t)(it - 1) * nfp * 3 : m->d_face_scratch;
-          stage_stacey_face(m, m->d_veloc, face, it);
-        }
+        const AsmStacey S0 = asm_stacey(m, smode ? m->d_stacey_store + (size_t)(it - 1) * nfp * 3 : nullptr, it);
         stage_seismo(m, it - 1);
-        AsmField F0{m->d_floc, face, m->nsources ? m->d_stf + (size_t)(it - 1) * m->nsources : nullptr,
+        AsmField F0{m->d_floc, nullptr, m->nsources ? m->d_stf + (size_t)(it - 1) * m->nsources : nullptr,
                     nullptr, m->d_displ, m->d_veloc, m->d_accel, dt};
         for (int sl = 0; sl < m->nslabs; ++sl) {
           const int e0 = sl * m->slab_elems, ne = std::min(m->slab_elems, m->nspec - e0);
@@ -1049,7 +1062,7 @@ void fwat_iterate_time_(long* Mesh_pointer, int* SIMULATION_TYPE, realw* DT, int
           sem_launch_forces(m, 1, 0, e0, ne, dt, nullptr, true);
           if (tm) tm->close(s);
           if (ta) ta->open(s);
-          stage_assemble(m, it == N, false, F0, F0, 0.0, sl);
+          stage_assemble(m, it == N, false, F0, F0, S0, 0.0, sl);
           if (ta) ta->close(s);
         }
       }
@@ -1064,17 +1077,13 @@ void fwat_iterate_time_(long* Mesh_pointer, int* SIMULATION_TYPE, realw* DT, int
         step_begin(it);
         const SemInterior in{AsmField{nullptr, nullptr, nullptr, nullptr, m->d_displ, m->d_veloc, m->d_accel, dt},
                              AsmField{}, it == N, 0.0};
-        stage_forces_timed(m, 1, 0, dt, tm, true, inner ? &in : nullptr);
-        realw* face = nullptr;
-        if (m->absorbing && m->nfaces) {
-          face = smode ? m->d_stacey_store + (size_t)(it - 1) * nfp * 3 : m->d_face_scratch;
-          stage_stacey_face(m, m->d_veloc, face, it);
-        }
-        stage_seismo(m, it - 1);
-        AsmField F0{m->d_floc, face, m->nsources ? m->d_stf + (size_t)(it - 1) * m->nsources : nullptr,
+        const SemSeismo se = seismo_row(m, it - 1);
+        stage_forces_timed(m, 1, 0, dt, tm, true, inner ? &in : nullptr, &se);
+        const AsmStacey S0 = asm_stacey(m, smode ? m->d_stacey_store + (size_t)(it - 1) * nfp * 3 : nullptr, it);
+        AsmField F0{m->d_floc, nullptr, m->nsources ? m->d_stf + (size_t)(it - 1) * m->nsources : nullptr,
                     nullptr, m->d_displ, m->d_veloc, m->d_accel, dt};
         if (ta) ta->open(s);
-        stage_assemble(m, it == N, false, F0, F0, 0.0, -1, inner);
+        stage_assemble(m, it == N, false, F0, F0, S0, 0.0, -1, inner);
         if (ta) ta->close(s);
       }
       lg.launch();
@@ -1146,13 +1155,9 @@ void fwat_iterate_time_(long* Mesh_pointer, int* SIMULATION_TYPE, realw* DT, int
         step_begin(it);
         const int rec0 = N - it;  // 0-based record / source row of forward step N + 1 - it
         m->kernel_flush = closes_block(it);
-        realw* face_a = nullptr;
-        if (m->absorbing && m->nfaces) {
-          face_a = m->d_face_scratch;
-          stage_stacey_face(m, m->d_veloc, face_a);
-        }
+        const AsmStacey S0 = asm_stacey(m, nullptr, 0);
         const realw* face_b = (m->absorbing && m->nfaces) ? m->d_stacey_store + (size_t)rec0 * nfp * 3 : nullptr;
-        AsmField F0{m->d_floc, face_a, nullptr, m->nrec ? m->d_adj + (size_t)rec0 * m->nrec * 3 : nullptr,
+        AsmField F0{m->d_floc, nullptr, nullptr, m->nrec ? m->d_adj + (size_t)rec0 * m->nrec * 3 : nullptr,
                     m->d_displ, m->d_veloc, m->d_accel, dt};
         AsmField F1{m->d_floc_b, face_b, m->nsources ? m->d_stf + (size_t)rec0 * m->nsources : nullptr,
                     nullptr, m->d_b_displ, m->d_b_veloc, m->d_b_accel, -dt};
@@ -1162,7 +1167,7 @@ void fwat_iterate_time_(long* Mesh_pointer, int* SIMULATION_TYPE, realw* DT, int
           sem_launch_forces(m, 2, 2, e0, ne, dt, nullptr, true);
           if (tm) tm->close(s);
           if (ta) ta->open(s);
-          stage_assemble(m, it == N, true, F0, F1, dtk, sl);
+          stage_assemble(m, it == N, true, F0, F1, S0, dtk, sl);
           if (ta) ta->close(s);
         }
       }
@@ -1179,18 +1184,14 @@ void fwat_iterate_time_(long* Mesh_pointer, int* SIMULATION_TYPE, realw* DT, int
                              AsmField{nullptr, nullptr, nullptr, nullptr, m->d_b_displ, m->d_b_veloc, m->d_b_accel, -dt},
                              it == N, dtk};
         stage_forces_timed(m, 2, 2, dt, tm, true, inner ? &in : nullptr);
-        realw* face_a = nullptr;
-        if (m->absorbing && m->nfaces) {
-          face_a = m->d_face_scratch;
-          stage_stacey_face(m, m->d_veloc, face_a);
-        }
+        const AsmStacey S0 = asm_stacey(m, nullptr, 0);
         const realw* face_b = (m->absorbing && m->nfaces) ? m->d_stacey_store + (size_t)rec0 * nfp * 3 : nullptr;
-        AsmField F0{m->d_floc, face_a, nullptr, m->nrec ? m->d_adj + (size_t)rec0 * m->nrec * 3 : nullptr,
+        AsmField F0{m->d_floc, nullptr, nullptr, m->nrec ? m->d_adj + (size_t)rec0 * m->nrec * 3 : nullptr,
                     m->d_displ, m->d_veloc, m->d_accel, dt};
         AsmField F1{m->d_floc_b, face_b, m->nsources ? m->d_stf + (size_t)rec0 * m->nsources : nullptr,
                     nullptr, m->d_b_displ, m->d_b_veloc, m->d_b_accel, -dt};
         if (ta) ta->open(s);
-        stage_assemble(m, it == N, true, F0, F1, dtk, -1, inner);
+        stage_assemble(m, it == N, true, F0, F1, S0, dtk, -1, inner);
         if (ta) ta->close(s);
       }
       lg.launch();
