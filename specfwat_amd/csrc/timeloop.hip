@@ -475,6 +475,22 @@ __global__ void k_expand_glob(int nspec, const int* __restrict__ ibool, const do
   out[idx] = rho ? scale_sign * (double)rho[idx] * v : v;
 }
 
+// save_adjoint_kernels' scaling of an accumulated kernel: out = K * (factor * modulus)
+__global__ void k_scale_kernel(size_t n, const double* __restrict__ K, const realw* __restrict__ modulus, double factor,
+                               double* __restrict__ out) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = K[i] * (factor * (double)modulus[i]);
+}
+
+// c_ij kernels of one element from rows [21][125] to the caller's [125][21], negated, through LDS
+__global__ __launch_bounds__(256) void k_cij_point_major(const double* __restrict__ K, double* __restrict__ out) {
+  __shared__ double s[2625];
+  const size_t b = (size_t)blockIdx.x * 2625;
+  for (int i = threadIdx.x; i < 2625; i += 256) s[i] = K[b + i];
+  __syncthreads();
+  for (int i = threadIdx.x; i < 2625; i += 256) out[b + i] = -s[(i % 21) * 125 + i / 21];
+}
+
 }  // namespace
 
 // ------------------------------------------------------------ internal stages
@@ -854,19 +870,15 @@ void transfer_kernels_el_to_host_dp_(long* Mesh_pointer, double* h_rho_kl, doubl
                      m->d_rho_kl_glob, -1.0, m->d_rho, tmp);
   HIP_CHECK(hipMemcpyAsync(h_rho_kl, tmp, nloc * 8, hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
-  dev_free(tmp);
   if (!m->anisotropic_kl) {
-    std::vector<float> kap(nloc), mu(nloc);
-    HIP_CHECK(hipMemcpyAsync(h_mu_kl, m->d_mu_kl, nloc * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(h_kappa_kl, m->d_kappa_kl, nloc * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(kap.data(), m->d_kappa, nloc * 4, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(mu.data(), m->d_mu, nloc * 4, hipMemcpyDeviceToHost, s));
+    // scaled on the device: the host loop over both arrays took as long as 40 adjoint steps (64x64x32)
+    hipLaunchKernelGGL(k_scale_kernel, dim3(nblk(nloc)), dim3(TPB), 0, s, nloc, m->d_mu_kl, m->d_mu, -2.0, tmp);
+    HIP_CHECK(hipMemcpyAsync(h_mu_kl, tmp, nloc * 8, hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(k_scale_kernel, dim3(nblk(nloc)), dim3(TPB), 0, s, nloc, m->d_kappa_kl, m->d_kappa, -1.0, tmp);
+    HIP_CHECK(hipMemcpyAsync(h_kappa_kl, tmp, nloc * 8, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    for (size_t L = 0; L < nloc; ++L) {
-      h_mu_kl[L] *= -2.0 * (double)mu[L];
-      h_kappa_kl[L] *= -(double)kap[L];
-    }
   }
+  dev_free(tmp);
 }
 
 // fp32 variant with SPECFEM's realw output type
@@ -888,12 +900,11 @@ void transfer_kernels_ani_to_host_dp_(long* Mesh_pointer, double* h_cijkl_kl, in
   if (*NSPEC_AB != m->nspec) SEM_FAIL("NSPEC_AB mismatch");
   if (!m->d_cijkl_kl) SEM_FAIL("anisotropic kernels not prepared");
   const size_t nloc = (size_t)m->nspec * 125;
-  std::vector<double> tmp(nloc * 21);
-  HIP_CHECK(hipMemcpyAsync(tmp.data(), m->d_cijkl_kl, tmp.size() * 8, hipMemcpyDeviceToHost, m->stream));
+  double* tmp = dev_alloc<double>(nloc * 21);
+  hipLaunchKernelGGL(k_cij_point_major, dim3(m->nspec), dim3(256), 0, m->stream, m->d_cijkl_kl, tmp);
+  HIP_CHECK(hipMemcpyAsync(h_cijkl_kl, tmp, nloc * 21 * 8, hipMemcpyDeviceToHost, m->stream));
   HIP_CHECK(hipStreamSynchronize(m->stream));
-  for (size_t e = 0; e < (size_t)m->nspec; ++e)
-    for (int q = 0; q < 21; ++q)
-      for (int L = 0; L < 125; ++L) h_cijkl_kl[((e * 125) + L) * 21 + q] = -tmp[(e * 21 + q) * 125 + L];
+  dev_free(tmp);
 }
 
 // approximate Hessian (sum of dt * a_adj . a_rec), (NGLLX,NGLLY,NGLLZ,NSPEC_AB)
