@@ -173,9 +173,10 @@ void prepare_constants_device_(long* Mesh_pointer, int* h_NGLLX, int* NSPEC_AB, 
     ib[L] = g;
   }
   {
-    // library numbering: a point is "interior" when exactly one element-local slot
-    // refers to it and no Stacey face, source or receiver term does
+    // library numbering: a point is "special" when a Stacey face, source or receiver term refers
+    // to it, "interior" when none does and exactly one element-local slot
     std::vector<uint8_t> touch(m->nglob, 0);  // element-local slots, saturating at 2
+    std::vector<uint8_t> special(m->nglob, 0);
     for (size_t L = 0; L < nloc; ++L) touch[ib[L]] = (uint8_t)std::min(2, touch[ib[L]] + 1);
     const int nf = *ABSORBING_CONDITIONS ? *h_num_abs_boundary_faces : 0;
     for (int f = 0; f < nf; ++f) {
@@ -186,25 +187,29 @@ void prepare_constants_device_(long* Mesh_pointer, int* h_NGLLX, int* NSPEC_AB, 
         const int i = h_abs_boundary_ijk[fq * 3] - 1, j = h_abs_boundary_ijk[fq * 3 + 1] - 1,
                   k = h_abs_boundary_ijk[fq * 3 + 2] - 1;
         if (i < 0 || i > 4 || j < 0 || j > 4 || k < 0 || k > 4) SEM_FAIL("abs_boundary_ijk out of range");
-        touch[ib[(size_t)e * 125 + i + 5 * j + 25 * k]] = 2;
+        special[ib[(size_t)e * 125 + i + 5 * j + 25 * k]] = 1;
       }
     }
     const auto whole_element = [&](int e) {
       if (e < 0 || e >= m->nspec) return;  // checked with a message below
-      for (int L = 0; L < 125; ++L) touch[ib[(size_t)e * 125 + L]] = 2;
+      for (int L = 0; L < 125; ++L) special[ib[(size_t)e * 125 + L]] = 1;
     };
     for (int q = 0; q < *NSOURCES; ++q) whole_element(h_ispec_selected_source[q] - 1);
     for (int q = 0; q < *nrec; ++q) whole_element(h_ispec_selected_rec[q] - 1);
-    int n_sh = 0;
+    int k = 0;
     std::vector<int> perm(m->nglob, -1);
     for (int g = 0; g < m->nglob; ++g)
-      if (touch[g] != 1) perm[g] = n_sh++;
-    int k = n_sh;
+      if (special[g]) perm[g] = k++;
+    m->n_special = k;
+    for (int g = 0; g < m->nglob; ++g)
+      if (!special[g] && touch[g] != 1) perm[g] = k++;
+    m->n_shared = k;
     for (size_t L = 0; L < nloc; ++L)
-      if (touch[ib[L]] == 1) perm[ib[L]] = k++;
+      if (!special[ib[L]] && touch[ib[L]] == 1) perm[ib[L]] = k++;
     if (k != m->nglob) SEM_FAIL("point numbering: %d of %d points placed", k, m->nglob);
-    m->n_shared = n_sh;
-    if (n_sh < m->nglob) {
+    bool identity = true;
+    for (int g = 0; g < m->nglob && identity; ++g) identity = perm[g] == g;
+    if (!identity) {
       uint64_t h = 1469598103934665603ull;  // FNV-1a over the numbering
       for (int g = 0; g < m->nglob; ++g) { h ^= (uint32_t)perm[g]; h *= 1099511628211ull; }
       m->perm_hash = h;

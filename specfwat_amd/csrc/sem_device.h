@@ -117,11 +117,13 @@ struct SemMesh {
   hipStream_t stream = nullptr;
 
   // geometry / indexing
-  // Library point numbering (prepare_constants_device_): points touched by more than one
-  // element-local slot or by a Stacey face, source or receiver term come first, in the
-  // caller's order, [0, n_shared); points touched by one element-local slot only follow,
-  // element by element.  h_perm[caller point] = library point (empty: the caller's
-  // numbering, every point shared); perm_hash identifies the numbering.
+  // Library point numbering (prepare_constants_device_): points touched by a Stacey face,
+  // source or receiver term come first, in the caller's order, [0, n_special); other points of
+  // more than one element-local slot next, in the caller's order, up to n_shared; points
+  // touched by one element-local slot only follow, element by element.
+  // h_perm[caller point] = library point (empty: the caller's numbering); perm_hash
+  // identifies the numbering.
+  int n_special = 0;
   int n_shared = 0;
   std::vector<int> h_perm;
   uint64_t perm_hash = 0;
@@ -205,7 +207,7 @@ struct SemMesh {
   realw* d_floc = nullptr;      // [nspec][125][3]
   realw* d_floc_b = nullptr;    // second field of the adjoint pass
   realw* d_face_scratch = nullptr;  // [nfaces*25][3] absorbing term of a non-stored field
-  int asm_points_per_lane = 0;  // gather assembly: 1 or 2 points per lane, 0 = by pass (see stage_assemble)
+  int asm_points_per_lane = 0;  // gather assembly: 1 or 2 points per lane, 0 = the default (see stage_assemble)
   int asm_block = 256;          // gather assembly: lanes per workgroup (64..1024)
   int floc_grouped = 1;         // floc rows grouped by reader (sem_floc_slot), 0: local-point order
   int* d_asm_off = nullptr;     // [nglob+1]

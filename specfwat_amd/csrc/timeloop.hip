@@ -30,6 +30,7 @@
 #include "sem_device.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 
@@ -114,70 +115,107 @@ struct AsmStacey {
   FkStep fk;
 };
 
-// Boundary, source, receiver and left-over single element terms of point g's row from q on, added
-// in row order (element terms lead the row, receiver terms end it); v0: the point's predicted
-// velocity.  The receivers' terms are read four at a time - a point of an element with many
-// receivers has one term for each, and one dependent load after the other made such points the
-// whole launch's time (12.5 us on a mesh whose element pass takes 6) - and not at all
-// when no field takes adjoint sources.
+// Force of one term c of a point's row, as a product: f0 += a0 * b0 and, for two fields,
+// f1 += a1 * b1 (element terms and tractions with a factor 1, which a fused multiply-add adds
+// exactly as an addition does); v0: the point's predicted velocity.
 template <bool TWO>
-__device__ __forceinline__ void assemble_tail(int q, int q1, const int* __restrict__ idx, int nloc, int nfp, int nsp,
-                                              const realw* __restrict__ sarr, const realw* __restrict__ rech,
-                                              const AsmField& F0, const AsmField& F1, const AsmStacey& S0,
-                                              const realw* v0, realw* f) {
-  const int first_rec = nloc + nfp + nsp;
-  for (; q < q1; ++q) {
-    const int c = idx[q];
-    if (c >= first_rec) break;
-    if (c < nloc) {
-      const realw* P = F0.floc + 3 * (size_t)c;
-      f[0] += P[0]; f[1] += P[1]; f[2] += P[2];
-      if (TWO) {
-        const realw* B = F1.floc + 3 * (size_t)c;
-        f[3] += B[0]; f[4] += B[1]; f[5] += B[2];
-      }
-    } else if (c < nloc + nfp) {
-      const size_t p = (size_t)(c - nloc);
-      if (S0.coef) {
-        realw tx, ty, tz;
-        stacey_point(p, S0.coef + 8 * p, v0[0], v0[1], v0[2], S0.fk, tx, ty, tz);
-        if (S0.rec) store3(S0.rec + 3 * p, tx, ty, tz);
-        f[0] -= tx; f[1] -= ty; f[2] -= tz;
-      } else if (F0.face) {
-        f[0] -= F0.face[3 * p]; f[1] -= F0.face[3 * p + 1]; f[2] -= F0.face[3 * p + 2];
-      }
-      if (TWO && F1.face) { f[3] -= F1.face[3 * p]; f[4] -= F1.face[3 * p + 1]; f[5] -= F1.face[3 * p + 2]; }
-    } else {
-      const int p = c - nloc - nfp;
-      const realw* S = sarr + 3 * (size_t)p;
-      if (F0.stf) { const realw w = (realw)F0.stf[p / 125]; f[0] = fmaf(S[0], w, f[0]); f[1] = fmaf(S[1], w, f[1]); f[2] = fmaf(S[2], w, f[2]); }
-      if (TWO && F1.stf) { const realw w = (realw)F1.stf[p / 125]; f[3] = fmaf(S[0], w, f[3]); f[4] = fmaf(S[1], w, f[4]); f[5] = fmaf(S[2], w, f[5]); }
+__device__ __forceinline__ void row_term(int c, int nloc, int nfp, int nsp, const realw* __restrict__ sarr,
+                                         const realw* __restrict__ rech, const AsmField& F0, const AsmField& F1,
+                                         const AsmStacey& S0, const realw* v0, realw* a0, realw& b0, realw* a1,
+                                         realw& b1) {
+  b0 = b1 = 0.0f;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) a0[d] = a1[d] = 0.0f;
+  if (c < nloc) {
+    const size_t p = 3 * (size_t)c;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      a0[d] = F0.floc[p + d];
+      if (TWO) a1[d] = F1.floc[p + d];
     }
+    b0 = b1 = 1.0f;
+  } else if (c < nloc + nfp) {
+    const size_t p = (size_t)(c - nloc);
+    realw x[3] = {0.0f, 0.0f, 0.0f};
+    if (S0.coef) {
+      stacey_point(p, S0.coef + 8 * p, v0[0], v0[1], v0[2], S0.fk, x[0], x[1], x[2]);
+      if (S0.rec) store3(S0.rec + 3 * p, x[0], x[1], x[2]);
+    } else if (F0.face) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) x[d] = F0.face[3 * p + d];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      a0[d] = -x[d];
+      if (TWO && F1.face) a1[d] = -F1.face[3 * p + d];
+    }
+    b0 = b1 = 1.0f;
+  } else if (c < nloc + nfp + nsp) {
+    const int p = c - nloc - nfp;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) a0[d] = a1[d] = sarr[3 * (size_t)p + d];
+    if (F0.stf) b0 = (realw)F0.stf[p / 125];
+    if (TWO && F1.stf) b1 = (realw)F1.stf[p / 125];
+  } else if (TWO && F0.adj) {  // adjoint sources act on the first of two fields only
+    const int p = c - nloc - nfp - nsp;
+    const size_t r = 3 * (size_t)(p / 125);
+    b0 = rech[p];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) a0[d] = F0.adj[r + d];
   }
-  if (!F0.adj && !(TWO && F1.adj)) return;
-  for (; q < q1; q += 4) {
-    realw h[4], x[4][3], y[4][3];
+}
+
+// Points [0, n_special), whose rows hold boundary, source or receiver terms besides the elements':
+// R = 8 lanes per point load eight terms at once, then add them in row order.  One lane (R = 1)
+// walking such a row pays one dependent load after another (edges of absorbing sides have up to
+// eight face terms, a point of an element with many receivers one for each): 10 us per assembly of
+// 16x16x8 elements, 4.5 us with eight lanes.
+template <bool LAST, bool TWO, int R>
+__device__ __forceinline__ void assemble_special(int lane, int n_special, const int* __restrict__ off,
+                                                 const int* __restrict__ idx, int nloc, int nfp, int nsp,
+                                                 const realw* __restrict__ sarr, const realw* __restrict__ rech,
+                                                 const realw* __restrict__ rm, const AsmField& F0, const AsmField& F1,
+                                                 const AsmStacey& S0, double* __restrict__ rho_kl,
+                                                 float* __restrict__ rho_part, int flush,
+                                                 double* __restrict__ hess_kl, double dtk) {
+  const int g = lane / R, j = lane % R;
+  if (g >= n_special) return;  // the same for all lanes of a point
+  const int q0 = off[g], q1 = off[g + 1];
+  const PointState P = load_point<TWO>((size_t)g, rm, F0, F1, rho_part);
+  realw f[6] = {0, 0, 0, 0, 0, 0};
+  if constexpr (R == 1) {
+    int next = q0 < q1 ? idx[q0] : 0;
+    for (int q = q0; q < q1; ++q) {
+      const int c = next;
+      if (q + 1 < q1) next = idx[q + 1];  // the next term's index, one term ahead
+      realw a0[3], a1[3], b0, b1;
+      row_term<TWO>(c, nloc, nfp, nsp, sarr, rech, F0, F1, S0, P.v0, a0, b0, a1, b1);
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      const int p = idx[min(q + n, q1 - 1)] - first_rec;  // the last receiver again past the row's end
-      const size_t r = 3 * (size_t)(p / 125);
-      h[n] = rech[p];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        x[n][c] = F0.adj ? F0.adj[r + c] : 0.0f;
-        if (TWO) y[n][c] = F1.adj ? F1.adj[r + c] : 0.0f;
+      for (int d = 0; d < 3; ++d) {
+        f[d] = fmaf(a0[d], b0, f[d]);
+        if (TWO) f[3 + d] = fmaf(a1[d], b1, f[3 + d]);
       }
     }
+  } else {
+    for (int q = q0; q < q1; q += R) {
+      realw a0[3] = {0, 0, 0}, a1[3] = {0, 0, 0}, b0 = 0, b1 = 0;
+      if (q + j < q1) row_term<TWO>(idx[q + j], nloc, nfp, nsp, sarr, rech, F0, F1, S0, P.v0, a0, b0, a1, b1);
+      const int n = min(R, q1 - q);
+      for (int k = 0; k < n; ++k) {
+        const realw w0 = __shfl(b0, k, R);
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
-      if (q + n < q1) {
+        for (int d = 0; d < 3; ++d) f[d] = fmaf(__shfl(a0[d], k, R), w0, f[d]);
+        if (TWO) {
+          const realw w1 = __shfl(b1, k, R);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          if (F0.adj) f[c] = fmaf(h[n], x[n][c], f[c]);
-          if (TWO && F1.adj) f[3 + c] = fmaf(h[n], y[n][c], f[3 + c]);
+          for (int d = 0; d < 3; ++d) f[3 + d] = fmaf(__shfl(a1[d], k, R), w1, f[3 + d]);
         }
       }
+    }
   }
+  if (j == 0)
+    newmark_point<TWO>((size_t)g, P, f[0], f[1], f[2], f[3], f[4], f[5], F0, F1, LAST, rho_kl, rho_part, flush != 0,
+                       hess_kl, dtk);
 }
 
 // Gather assembly fused with the Newmark update.  For every global point:
@@ -189,40 +227,73 @@ __device__ __forceinline__ void assemble_tail(int q, int q1, const int* __restri
 // TWO: the adjoint field (dt > 0) and the reconstructed field (dt < 0) are
 // updated together and the density kernel a_adj . u_rec is accumulated in fp64.
 
-// glist: the points of this launch (one slab's), or null for points 0..npts-1.
-template <bool LAST, bool TWO>
-__global__ void k_assemble(int npts, const int* __restrict__ glist, const int* __restrict__ off,
+// glist: the points of this launch (one slab's, any terms), or null for points 0..npts-1, of which
+// the first workgroups take the special ones (assemble_special) and the others have element terms only.
+template <bool LAST, bool TWO, int R>
+__global__ void k_assemble(int npts, int n_special, const int* __restrict__ glist, const int* __restrict__ off,
                            const int* __restrict__ idx, int nloc, int nfp, int nsp, const realw* __restrict__ sarr,
                            const realw* __restrict__ rech, const realw* __restrict__ rm,
                            AsmField F0, AsmField F1, AsmStacey S0, double* __restrict__ rho_kl,
                            float* __restrict__ rho_part, int flush, double* __restrict__ hess_kl, double dtk) {
-  const int h = blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= npts) return;
-  const int g = glist ? glist[h] : h;
-  realw f0x = 0, f0y = 0, f0z = 0, f1x = 0, f1y = 0, f1z = 0;
+  int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if constexpr (R == 0) {
+    if (g >= npts) return;
+    g = glist[g];
+  } else {
+    const int nsb = (R * n_special + blockDim.x - 1) / blockDim.x;
+    if ((int)blockIdx.x < nsb) {
+      assemble_special<LAST, TWO, R>(g, n_special, off, idx, nloc, nfp, nsp, sarr, rech, rm, F0, F1, S0, rho_kl, rho_part,
+                                  flush, hess_kl, dtk);
+      return;
+    }
+    g += n_special - nsb * (int)blockDim.x;
+    if (g >= npts) return;
+  }
   const PointState P = load_point<TWO>((size_t)g, rm, F0, F1, rho_part);
   const int q1 = off[g + 1];
   int q = off[g];
-  // pairs of element-local contributions (most of them): both rows are loaded
-  // before either is added, two loads in flight per lane; same summation order
-  for (; q + 1 < q1; q += 2) {
-    const int c0 = idx[q], c1 = idx[q + 1];
-    if (c1 >= nloc) break;  // element terms lead each row: c0 is one too
-    const realw* P0 = F0.floc + 3 * (size_t)c0;
-    const realw* P1 = F0.floc + 3 * (size_t)c1;
-    const realw a0 = P0[0], a1 = P0[1], a2 = P0[2], b0 = P1[0], b1 = P1[1], b2 = P1[2];
-    if (TWO) {
-      const realw* B0 = F1.floc + 3 * (size_t)c0;
-      const realw* B1 = F1.floc + 3 * (size_t)c1;
-      const realw d0 = B0[0], d1 = B0[1], d2 = B0[2], e0 = B1[0], e1 = B1[1], e2 = B1[2];
-      f1x += d0; f1y += d1; f1z += d2;
-      f1x += e0; f1y += e1; f1z += e2;
-    }
-    f0x += a0; f0y += a1; f0z += a2;
-    f0x += b0; f0y += b1; f0z += b2;
+  // element-local contributions four at a time: their indices, then their rows, are all requested
+  // before any is added (faces have two terms, edges four, corners eight); same summation order
+  realw f[6] = {0, 0, 0, 0, 0, 0};
+  for (bool more = true; more && q < q1;) {
+    int c[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) c[n] = q + n < q1 ? idx[q + n] : INT_MAX;
+    realw x[4][3], y[4][3];
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      if (c[n] < nloc) {
+        const realw* A = F0.floc + 3 * (size_t)c[n];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) x[n][d] = A[d];
+        if (TWO) {
+          const realw* B = F1.floc + 3 * (size_t)c[n];
+#pragma unroll
+          for (int d = 0; d < 3; ++d) y[n][d] = B[d];
+        }
+      }
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      if (c[n] < nloc) {  // element terms lead each row
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          f[d] += x[n][d];
+          if (TWO) f[3 + d] += y[n][d];
+        }
+        ++q;
+      }
+    more = c[3] < nloc;
   }
-  realw f[6] = {f0x, f0y, f0z, f1x, f1y, f1z};
-  assemble_tail<TWO>(q, q1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, S0, P.v0, f);
+  if constexpr (R == 0)
+    for (; q < q1; ++q) {
+      realw a0[3], a1[3], b0, b1;
+      row_term<TWO>(idx[q], nloc, nfp, nsp, sarr, rech, F0, F1, S0, P.v0, a0, b0, a1, b1);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        f[d] = fmaf(a0[d], b0, f[d]);
+        if (TWO) f[3 + d] = fmaf(a1[d], b1, f[3 + d]);
+      }
+    }
   newmark_point<TWO>((size_t)g, P, f[0], f[1], f[2], f[3], f[4], f[5], F0, F1, LAST, rho_kl, rho_part, flush != 0,
                      hess_kl, dtk);
 }
@@ -231,18 +302,23 @@ __global__ void k_assemble(int npts, const int* __restrict__ glist, const int* _
 // block's 2 * blockDim.x): both points' state, offsets, indices and
 // element-local rows are requested before either is summed, so a lane keeps
 // twice the loads in flight.  Each point's row is summed in the same order as
-// k_assemble (pairs of element terms, then the tail), so results are identical.
-template <bool LAST, bool TWO>
-__global__ void k_assemble2(int npts, const int* __restrict__ glist, const int* __restrict__ off,
+// k_assemble, so results are identical.
+template <bool LAST, bool TWO, int R>
+__global__ void k_assemble2(int npts, int n_special, const int* __restrict__ off,
                             const int* __restrict__ idx, int nloc, int nfp, int nsp, const realw* __restrict__ sarr,
                             const realw* __restrict__ rech, const realw* __restrict__ rm,
                             AsmField F0, AsmField F1, AsmStacey S0, double* __restrict__ rho_kl,
                             float* __restrict__ rho_part, int flush, double* __restrict__ hess_kl, double dtk) {
-  const int ha = blockIdx.x * 2 * blockDim.x + threadIdx.x, hb = ha + blockDim.x;
-  if (ha >= npts) return;
-  const bool vb = hb < npts;
-  const int ga = glist ? glist[ha] : ha;
-  const int gb = vb ? (glist ? glist[hb] : hb) : ga;
+  const int nsb = (R * n_special + blockDim.x - 1) / blockDim.x;
+  if ((int)blockIdx.x < nsb) {
+    assemble_special<LAST, TWO, R>(blockIdx.x * blockDim.x + threadIdx.x, n_special, off, idx, nloc, nfp, nsp, sarr, rech, rm,
+                                F0, F1, S0, rho_kl, rho_part, flush, hess_kl, dtk);
+    return;
+  }
+  const int ga = n_special + (blockIdx.x - nsb) * 2 * blockDim.x + threadIdx.x;
+  if (ga >= npts) return;
+  const bool vb = ga + (int)blockDim.x < npts;
+  const int gb = vb ? ga + (int)blockDim.x : ga;
   const PointState Pa = load_point<TWO>((size_t)ga, rm, F0, F1, rho_part);
   const PointState Pb = load_point<TWO>((size_t)gb, rm, F0, F1, rho_part);
   int qa = off[ga], qb = off[gb];
@@ -255,8 +331,6 @@ __global__ void k_assemble2(int npts, const int* __restrict__ glist, const int* 
     int a0 = 0, a1 = 0, b0 = 0, b1 = 0;
     if (ra) { a0 = idx[qa]; a1 = idx[qa + 1]; }
     if (rb) { b0 = idx[qb]; b1 = idx[qb + 1]; }
-    ra = ra && a1 < nloc;  // element terms lead each row: a0 is one too
-    rb = rb && b1 < nloc;
     realw x[12], y[12];
     if (ra) {
       const realw* P0 = F0.floc + 3 * (size_t)a0;
@@ -309,8 +383,23 @@ __global__ void k_assemble2(int npts, const int* __restrict__ glist, const int* 
       qb += 2;
     }
   }
-  assemble_tail<TWO>(qa, qa1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, S0, Pa.v0, fa);
-  if (vb) assemble_tail<TWO>(qb, qb1, idx, nloc, nfp, nsp, sarr, rech, F0, F1, S0, Pb.v0, fb);
+  // the odd element term of a row
+  if (qa < qa1) {
+    const size_t p = 3 * (size_t)idx[qa];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      fa[c] += F0.floc[p + c];
+      if (TWO) fa[3 + c] += F1.floc[p + c];
+    }
+  }
+  if (qb < qb1) {
+    const size_t p = 3 * (size_t)idx[qb];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      fb[c] += F0.floc[p + c];
+      if (TWO) fb[3 + c] += F1.floc[p + c];
+    }
+  }
   newmark_point<TWO>((size_t)ga, Pa, fa[0], fa[1], fa[2], fa[3], fa[4], fa[5], F0, F1, LAST, rho_kl, rho_part,
                      flush != 0, hess_kl, dtk);
   if (vb)
@@ -601,44 +690,57 @@ void stage_assemble(SemMesh* m, bool last, bool two, const AsmField& F0, const A
   if (npts == 0) return;
   const int tpb = m->asm_block;
   const dim3 bl(tpb);
-  // 0 (default): two points per lane for the one-field pass, one for the two-field pass
-  // (measured on the C2 mesh: 0.656 vs 0.668 ms one-field, 1.32 vs 1.21 ms two-field)
-  const int ppl = m->asm_points_per_lane ? m->asm_points_per_lane : (two ? 1 : 2);
-  if (ppl == 2) {
-    const dim3 g2((unsigned)((npts + 2 * tpb - 1) / (2 * tpb)));
-#define ASM2(L, T, RK, RP, FL, HK)                                                                              \
-  SEM_LAUNCH((k_assemble2<L, T>), g2, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp, nsp, \
-             m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, RK, RP, FL, HK, dtk)
-    if (two) {
-      if (last) ASM2(true, true, m->d_rho_kl_glob, rho_part, m->kernel_flush, m->d_hess_kl_glob);
-      else ASM2(false, true, m->d_rho_kl_glob, rho_part, m->kernel_flush, m->d_hess_kl_glob);
-    } else {
-      if (last) ASM2(true, false, (double*)nullptr, (float*)nullptr, 1, (double*)nullptr);
-      else ASM2(false, false, (double*)nullptr, (float*)nullptr, 1, (double*)nullptr);
-    }
-#undef ASM2
+  double* rk = two ? m->d_rho_kl_glob : nullptr;
+  double* hk = two ? m->d_hess_kl_glob : nullptr;
+  if (!two) rho_part = nullptr;
+  const int fl = two ? m->kernel_flush : 1;
+#define ASM_ARGS m->d_asm_off, m->d_asm_idx, nloc, nfp, nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, rk, rho_part, fl, hk, dtk
+#define ASM_CASES(LAUNCH)                       \
+  do {                                          \
+    if (two) {                                  \
+      if (last) LAUNCH(true, true);             \
+      else LAUNCH(false, true);                 \
+    } else {                                    \
+      if (last) LAUNCH(true, false);            \
+      else LAUNCH(false, false);                \
+    }                                           \
+  } while (0)
+  if (glist) {
+    const dim3 gr(nblk(npts, tpb));
+#define ASM_LIST(L, T) SEM_LAUNCH((k_assemble<L, T, 0>), gr, bl, 0, m->stream, npts, 0, glist, ASM_ARGS)
+    ASM_CASES(ASM_LIST);
+#undef ASM_LIST
     return;
   }
-  const dim3 gr(nblk(npts, tpb));
-  if (two) {
-    if (last)
-      SEM_LAUNCH((k_assemble<true, true>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, m->d_rho_kl_glob, rho_part, m->kernel_flush,
-                         m->d_hess_kl_glob, dtk);
-    else
-      SEM_LAUNCH((k_assemble<false, true>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, m->d_rho_kl_glob, rho_part, m->kernel_flush,
-                         m->d_hess_kl_glob, dtk);
-  } else {
-    if (last)
-      SEM_LAUNCH((k_assemble<true, false>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, (double*)nullptr, (float*)nullptr, 1,
-                         (double*)nullptr, dtk);
-    else
-      SEM_LAUNCH((k_assemble<false, false>), gr, bl, 0, m->stream, npts, glist, m->d_asm_off, m->d_asm_idx, nloc, nfp,
-                         nsp, m->d_sourcearrays, m->d_rec_h, m->d_rmass_inv, F0, F1, S0, (double*)nullptr, (float*)nullptr, 1,
-                         (double*)nullptr, dtk);
+  // 0 (default): one point per lane, whose four terms in flight are as many as two points' pairs
+  // (64x64x32: 105 against 117 us with one field, 234 against 300 with two)
+  const int ppl = m->asm_points_per_lane ? m->asm_points_per_lane : 1;
+  // eight lanes per special point while they do not crowd the launch: the step of 16x16x8 elements
+  // (13 thousand special points) 10.7 against 14.4 us with one lane, 32x32x16 (51 thousand) 37.2
+  // against 38.8; 41x37x18 (75 thousand) 81.9 against 82.1 and 64x64x32 (0.2 million) 284 against 278
+  const int R = m->n_special <= 57344 ? 8 : 1;
+  const int sb = nblk((size_t)R * m->n_special, tpb), rest = npts - m->n_special;
+  if (ppl == 2) {
+    const dim3 gr(sb + nblk(rest, 2 * tpb));
+#define ASM_TWO(L, T)                                                                                         \
+  do {                                                                                                        \
+    if (R == 8) SEM_LAUNCH((k_assemble2<L, T, 8>), gr, bl, 0, m->stream, npts, m->n_special, ASM_ARGS);       \
+    else SEM_LAUNCH((k_assemble2<L, T, 1>), gr, bl, 0, m->stream, npts, m->n_special, ASM_ARGS);              \
+  } while (0)
+    ASM_CASES(ASM_TWO);
+#undef ASM_TWO
+    return;
   }
+  const dim3 gr(sb + nblk(rest, tpb));
+#define ASM_ONE(L, T)                                                                                                   \
+  do {                                                                                                                  \
+    if (R == 8) SEM_LAUNCH((k_assemble<L, T, 8>), gr, bl, 0, m->stream, npts, m->n_special, (const int*)nullptr, ASM_ARGS); \
+    else SEM_LAUNCH((k_assemble<L, T, 1>), gr, bl, 0, m->stream, npts, m->n_special, (const int*)nullptr, ASM_ARGS);        \
+  } while (0)
+  ASM_CASES(ASM_ONE);
+#undef ASM_ONE
+#undef ASM_CASES
+#undef ASM_ARGS
 }
 
 SemSeismo seismo_row(const SemMesh* m, int it0) {

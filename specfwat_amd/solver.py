@@ -133,7 +133,7 @@ class ElasticRun:
 
     def set_assembly_lanes(self, points_per_lane):
         """Points per lane of the gather assembly (1 or 2; the same sums), 0 for
-        the default (2 for the one-field pass, 1 for the two-field pass)."""
+        the default (1)."""
         _lib.call("fwat_set_assembly_lanes_", self.h, int(points_per_lane))
 
     def set_assembly_block(self, lanes):
