@@ -1022,10 +1022,25 @@ void fwat_column_block_order_(int* nex, int* ney, int* nez, int* per_xcd, int* o
 }
 }  // extern "C"
 
+// Element pass of a handle whose launch shape was never set (fwat_set_tuning_).  Isotropic cubes
+// take the pipelined pass, which finishes the interior points: a step (element pass and assembly)
+// of 64x64x32 elements 290 against 313 us with the folded-table pass, both fields 592 against 651;
+// 32x32x16 41.9 against 45.3 and 71.9 against 77.9; 16x16x8 16.0 against 16.7 and 18.6 against
+// 19.9; the same within 2 % at 8x8x4.  Anisotropic cubes take the folded-table pass and
+// other meshes the general one, the only ones there are for them.
+static int element_path(const SemMesh* m) { return m->regular_fast_path >= 0 ? m->regular_fast_path : m->anisotropy ? 1 : 3; }
+
+// Persistent workgroups per CU of the pipelined pass chosen so: 10 with one field (five waves per
+// SIMD; 12 leave two waiting: 230 against 169 us at 64x64x32, 8: 191), 8 with two (6: 377 against 356).
+static int element_blocks(const SemMesh* m, int nfields) {
+  if (m->regular_fast_path < 0 && element_path(m) == 3) return nfields == 2 ? 8 : 10;
+  return nfields == 2 ? m->blocks_per_cu_adj : m->blocks_per_cu_fwd;
+}
+
 bool sem_interior_active(const SemMesh* m, int nfields) {
+  const int path = element_path(m);
   return m->interior_newmark && m->n_shared < m->nglob && m->nspec_irregular == 0 && !m->anisotropy &&
-         (m->regular_fast_path == 3 || m->regular_fast_path == 5) && m->nslabs == 0 &&
-         !sem_brick_active(m, nfields) && m->d_floc != nullptr;
+         (path == 3 || path == 5) && m->nslabs == 0 && !sem_brick_active(m, nfields) && m->d_floc != nullptr;
 }
 
 void sem_launch_forces(SemMesh* m, int nfields, int kernel_mode, int elem_begin, int elem_count,
@@ -1095,11 +1110,11 @@ void sem_launch_forces(SemMesh* m, int nfields, int kernel_mode, int elem_begin,
   const int sp = m->static_precision;
   const bool an = m->anisotropy != 0;
   hipStream_t s = m->stream;
-  if (gather && m->nspec_irregular == 0 && m->regular_fast_path && kernel_mode != 1) {
+  if (gather && m->nspec_irregular == 0 && element_path(m) && kernel_mode != 1) {
     // regular_fast_path 2: the software-pipelined isotropic pass, 3: the same with two
     // barriers per element (ping-pong LDS buffers)
-    int pipe = m->regular_fast_path;
-    const int bpc = nfields == 2 ? m->blocks_per_cu_adj : m->blocks_per_cu_fwd;
+    int pipe = element_path(m);
+    const int bpc = element_blocks(m, nfields);
     if (pipe == 5) {
       // 5: the ping-pong pass in column-block order on a lattice mesh over the whole mesh,
       // when every XCD's share is whole columns (anything else keeps element order)

@@ -105,7 +105,7 @@ struct SemMesh {
   int approximate_hess_kl = 0;
   int compute_and_store_strain = 0;
   int static_precision = SEM_STATIC_FP32;
-  int regular_fast_path = 1;  // folded-table element pass on all-regular meshes
+  int regular_fast_path = -1;  // element pass (fwat_set_tuning_); -1: the library's choice
   int blocks_per_cu_fwd = 0;  // element-pass workgroups per CU (0: one per element)
   int blocks_per_cu_adj = 8;
   int graph = 0;              // whole-run loops captured into a HIP graph (fwat_set_graph_)
