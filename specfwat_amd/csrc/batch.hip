@@ -38,6 +38,14 @@ constexpr int TPB = 256;
 
 inline int nblk(size_t n) { return (int)((n + TPB - 1) / TPB); }
 
+struct BatchSeismo {
+  int nrec, it, nmax;
+  const int* nstep;
+  const int* riglob;
+  const realw* rh;
+  realw* seis;
+};
+
 struct BatchElemArgs {
   const int* ibool;
   const realw* kappa;
@@ -74,6 +82,8 @@ struct BatchElemArgs {
   double* rho_kl;    // [nglob][E]
   float* rho_part;   // [nglob][E]
   realw fdt;         // field time step
+  int nblk;          // workgroups of the element pass; a forward launch's others take seismograms
+  BatchSeismo se;
 };
 
 __device__ __forceinline__ float bf16f(uint16_t x) { return __uint_as_float((uint32_t)x << 16); }
@@ -118,6 +128,59 @@ __device__ __forceinline__ void store_pt(realw* __restrict__ p, const realw (&x)
     for (int k = 0; k < 3 * E; ++k) p[k] = x[k];
   }
 }
+
+// Seismograms of the forward field, one 128-lane workgroup per (receiver, event), into
+// seis [E][NSTEP_max][nrec][3] row it-1.  They ride with the element pass's launch, which leaves
+// the receivers' points alone (they are shared points); s: 3 * 128 reals of LDS.
+template <int E>
+__device__ __forceinline__ void batch_seismo_block(const BatchSeismo& S, int q, const realw* __restrict__ u, realw* s) {
+  const int r = q / E, ev = q % E, t = threadIdx.x;
+  if (S.it > S.nstep[ev]) return;  // block-uniform
+  realw x = 0, y = 0, z = 0;
+  if (t < 125) {
+    const realw h = S.rh[(size_t)r * 125 + t];
+    const size_t g = (size_t)S.riglob[(size_t)r * 125 + t];
+    const realw* U = u + (g * E + ev) * 3;
+    x = h * U[0]; y = h * U[1]; z = h * U[2];
+  }
+  s[t] = x; s[128 + t] = y; s[256 + t] = z;
+  __syncthreads();
+  for (int w = 64; w > 0; w >>= 1) {
+    if (t < w) { s[t] += s[t + w]; s[128 + t] += s[128 + t + w]; s[256 + t] += s[256 + t + w]; }
+    __syncthreads();
+  }
+  if (t == 0) {
+    realw* o = S.seis + (((size_t)ev * S.nmax + (S.it - 1)) * S.nrec + r) * 3;
+    o[0] = s[0]; o[1] = s[128]; o[2] = s[256];
+  }
+}
+
+// A point's row of 3E floats in pieces of 16 bytes (E a multiple of 4), 8 (E = 2) or 4: the
+// isotropic element pass moves rows between memory and LDS with a lane per piece, so that a wave's
+// access covers whole rows (a lane per row touched 64 rows in 16-byte pieces: 46.5 / 20.1 us for
+// the two- and one-field passes of 8 events on 16x16x8 elements).  In LDS value k of the row of local
+// point p sits at k * SU + p, SU odd so that the pieces of a row fall into different banks.
+template <int E>
+struct EventRow {
+  static constexpr int W = E % 4 == 0 ? 4 : E % 2 == 0 ? 2 : 1, C = 3 * E / W, SU = 129;
+  // piece `at` of the rows at p, into / from LDS
+  __device__ static __forceinline__ void get(const realw* __restrict__ p, size_t at, realw* s) {
+    if constexpr (W == 4) {
+      const float4 v = reinterpret_cast<const float4*>(p)[at];
+      s[0] = v.x; s[SU] = v.y; s[2 * SU] = v.z; s[3 * SU] = v.w;
+    } else if constexpr (W == 2) {
+      const float2 v = reinterpret_cast<const float2*>(p)[at];
+      s[0] = v.x; s[SU] = v.y;
+    } else {
+      s[0] = p[at];
+    }
+  }
+  __device__ static __forceinline__ void put(realw* __restrict__ p, size_t at, const realw* s) {
+    if constexpr (W == 4) reinterpret_cast<float4*>(p)[at] = make_float4(s[0], s[SU], s[2 * SU], s[3 * SU]);
+    else if constexpr (W == 2) reinterpret_cast<float2*>(p)[at] = make_float2(s[0], s[SU]);
+    else p[at] = s[0];
+  }
+};
 
 // Newmark finish of event ev at a point whose only term is one element's: the
 // element pass holds the point's forces f0, f1 and displacements u0, u1; its inverse
@@ -190,11 +253,21 @@ constexpr int batch_elem_waves(int E, int NF) { return NF == 2 ? (E >= 8 ? 3 : 4
 template <int E, int NF, int SP, bool INT>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(INT ? 1 : batch_elem_waves(E, NF))))
 void k_batch_elem(BatchElemArgs A) {
+  using Row = EventRow<E>;
   __shared__ realw s_tab[128];
-  __shared__ realw s_u[NF][E][3][128];
+  __shared__ int s_g[2][125];      // the element's points, alternating from element to element
+  __shared__ uint8_t s_row[125];   // local point of each row of element-local forces
+  __shared__ realw s_u[NF][E][3][Row::SU];
   __shared__ realw s_s[NF][6][128];
   const int t = threadIdx.x;
-  if (t < 125) s_tab[t] = A.tables[t];
+  if (NF == 1 && (int)blockIdx.x >= A.nblk) {  // block-uniform
+    batch_seismo_block<E>(A.se, blockIdx.x - A.nblk, A.u0, &s_s[0][0][0]);
+    return;
+  }
+  if (t < 125) {
+    s_tab[t] = A.tables[t];
+    s_row[sem_floc_slot(t)] = (uint8_t)t;
+  }
   const bool act = t < 125;
   const int tt = act ? t : 124;
   const int I = tt % 5, J = (tt / 5) % 5, K = tt / 25;
@@ -217,15 +290,19 @@ void k_batch_elem(BatchElemArgs A) {
     }
   }
   const int La0 = 5 * J + 25 * K, Lb0 = I + 25 * K, Lc0 = I + 5 * J;
-  const int nb = gridDim.x;
+  const int nb = A.nblk;
   const int x = blockIdx.x & 7, per_xcd = nb >> 3, slot = blockIdx.x >> 3;
   const int chunk = (A.nspec + 7) >> 3;
   const int e_end = min(A.nspec, (x + 1) * chunk);
   const size_t nloc = (size_t)A.nspec * 125;
   const int mask = A.active_mask;
-  for (int e = x * chunk + slot; e < e_end; e += per_xcd) {
+  int b = 0;
+  int ig_next = x * chunk + slot < e_end ? A.ibool[(size_t)(x * chunk + slot) * 125 + tt] : 0;
+  for (int e = x * chunk + slot; e < e_end; e += per_xcd, b ^= 1) {
     const size_t Lg = (size_t)e * 125 + tt;
-    const int iglob = A.ibool[Lg];
+    const int iglob = ig_next;
+    if (act) s_g[b][t] = iglob;
+    if (e + per_xcd < e_end) ig_next = A.ibool[(size_t)(e + per_xcd) * 125 + tt];
     bool src = false;  // uniform over the workgroup
     if (INT)
       for (int k = 0; k < A.n_src; ++k) src |= e == A.src_el[k];
@@ -241,18 +318,14 @@ void k_batch_elem(BatchElemArgs A) {
     }
     const realw lam = kl - (2.0f / 3.0f) * ml;
     const realw m2 = 2.0f * ml;
-    __syncthreads();  // previous element done with s_u
-    if (act) {
+    __syncthreads();  // previous element done with s_u; this one's points in s_g
+    // consecutive lanes take consecutive pieces of the points' rows
 #pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        realw x3[3 * E];
-        load_pt<E>((f == 0 ? A.u0 : A.u1) + (size_t)iglob * (3 * E), x3);
-#pragma unroll
-        for (int ev = 0; ev < E; ++ev) {
-          s_u[f][ev][0][t] = x3[3 * ev];
-          s_u[f][ev][1][t] = x3[3 * ev + 1];
-          s_u[f][ev][2][t] = x3[3 * ev + 2];
-        }
+    for (int f = 0; f < NF; ++f) {
+      const realw* U = f == 0 ? A.u0 : A.u1;
+      for (int q = t; q < 125 * Row::C; q += 128) {
+        const int p = q / Row::C, c = q - p * Row::C;
+        Row::get(U, (size_t)s_g[b][p] * Row::C + c, &s_u[f][0][0][0] + (size_t)c * Row::W * Row::SU + p);
       }
     }
     const bool inner = INT && act && !src && iglob >= A.n_shared;
@@ -336,21 +409,16 @@ void k_batch_elem(BatchElemArgs A) {
       }
       __syncthreads();  // s_s free for the next event
     }
-    const int fs = sem_floc_slot(tt);
     // the 27 inner slots sit at the end of the element row, so leaving the rows of the
     // points finished here out leaves the rest whole (a free-surface element's top
     // face points that have no other term lie mid-row and are stored anyway)
-    if (act && !(inner && fs >= 98)) {
 #pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        realw out[3 * E];
-#pragma unroll
-        for (int ev = 0; ev < E; ++ev) {
-          out[3 * ev] = s_u[f][ev][0][t];
-          out[3 * ev + 1] = s_u[f][ev][1][t];
-          out[3 * ev + 2] = s_u[f][ev][2][t];
-        }
-        store_pt<E>((f == 0 ? A.floc0 : A.floc1) + (Lg - tt + fs) * (3 * E), out);
+    for (int f = 0; f < NF; ++f) {
+      realw* O = f == 0 ? A.floc0 : A.floc1;
+      for (int q = t; q < 125 * Row::C; q += 128) {
+        const int r = q / Row::C, c = q - r * Row::C, p = s_row[r];
+        if (INT && r >= 98 && !src && s_g[b][p] >= A.n_shared) continue;
+        Row::put(O, ((size_t)e * 125 + r) * Row::C + c, &s_u[f][0][0][0] + (size_t)c * Row::W * Row::SU + p);
       }
     }
   }
@@ -368,6 +436,10 @@ __global__ __launch_bounds__(128) void k_batch_elem_aniso(BatchElemArgs A) {
   __shared__ realw s_u[NF][E][3][128];
   __shared__ realw s_s[NF][6][128];
   const int t = threadIdx.x;
+  if (NF == 1 && (int)blockIdx.x >= A.nblk) {  // block-uniform
+    batch_seismo_block<E>(A.se, blockIdx.x - A.nblk, A.u0, &s_s[0][0][0]);
+    return;
+  }
   if (t < 125) s_tab[t] = A.tables[t];
   const bool act = t < 125;
   const int tt = act ? t : 124;
@@ -391,7 +463,7 @@ __global__ __launch_bounds__(128) void k_batch_elem_aniso(BatchElemArgs A) {
     }
   }
   const int La0 = 5 * J + 25 * K, Lb0 = I + 25 * K, Lc0 = I + 5 * J;
-  const int nb = gridDim.x;
+  const int nb = A.nblk;
   const int x = blockIdx.x & 7, per_xcd = nb >> 3, slot = blockIdx.x >> 3;
   const int chunk = (A.nspec + 7) >> 3;
   const int e_end = min(A.nspec, (x + 1) * chunk);
@@ -496,6 +568,17 @@ __global__ __launch_bounds__(128) void k_batch_elem_aniso(BatchElemArgs A) {
   }
 }
 
+// Stacey traction of a face point (coefficients C) for velocity V
+__device__ __forceinline__ void batch_stacey_point(const realw* __restrict__ C, const realw* __restrict__ V, realw& tx,
+                                                   realw& ty, realw& tz) {
+  const realw nx = C[0], ny = C[1], nz = C[2], jw = C[3], rvp = C[4], rvs = C[5];
+  const realw vx = V[0], vy = V[1], vz = V[2];
+  const realw vn = vx * nx + vy * ny + vz * nz;
+  tx = (rvp * vn * nx + rvs * (vx - vn * nx)) * jw;
+  ty = (rvp * vn * ny + rvs * (vy - vn * ny)) * jw;
+  tz = (rvp * vn * nz + rvs * (vz - vn * nz)) * jw;
+}
+
 struct BatchAsmArgs {
   int nglob, nloc, nfp, nrec, nmax, it;
   const int* off;
@@ -510,7 +593,8 @@ struct BatchAsmArgs {
   float* rho_part;     // [nglob][E] fp32 partial sums (null: straight into fp64)
   int kflush;
   const int* nstep;    // [E]
-  const realw* face0;  // [nfp][E][3] traction of field 0 (forward: store row it-1; adjoint: scratch)
+  const realw* fcoef;  // [nfp][8]: the traction of field 0 is taken here (a forward run stores it to
+  realw* face0;        // face0), or null: it is read from face0 [nfp][E][3]
   const realw* face1;  // [nfp][E][3] replayed store row NSTEP_max - it (adjoint)
   const double* stf;   // [E][NSTEP_max]
   const realw* adj;    // [E][NSTEP_max][nrec][3]
@@ -571,7 +655,14 @@ __global__ void k_batch_asm(BatchAsmArgs A) {
       }
     } else if (c < A.nloc + A.nfp) {
       const size_t p = ((size_t)(c - A.nloc) * E + ev) * 3;
-      f0x -= A.face0[p]; f0y -= A.face0[p + 1]; f0z -= A.face0[p + 2];
+      realw tx, ty, tz;
+      if (A.fcoef) {  // from the point's own velocity, stored on the way in a forward run
+        batch_stacey_point(A.fcoef + 8 * (size_t)(c - A.nloc), A.v0 + 3 * q, tx, ty, tz);
+        if (!TWO) store3(A.face0 + p, tx, ty, tz);
+      } else {
+        tx = A.face0[p]; ty = A.face0[p + 1]; tz = A.face0[p + 2];
+      }
+      f0x -= tx; f0y -= ty; f0z -= tz;
       if (TWO) { f1x -= A.face1[p]; f1y -= A.face1[p + 1]; f1z -= A.face1[p + 2]; }
     } else if (c < A.nloc + A.nfp + nsp) {
       const int p = c - A.nloc - A.nfp;
@@ -619,26 +710,18 @@ __global__ void k_batch_asm(BatchAsmArgs A) {
   }
 }
 
-// Stacey traction of field 0, one lane per (face point, event), written to
-// out [nfp][E][3] (forward: the store row of this step; adjoint: scratch)
-__global__ void k_batch_stacey(int nfp, int E, int it, int nmax, int adjoint, const int* __restrict__ nstep,
-                               const int* __restrict__ figlob, const realw* __restrict__ fcoef,
-                               const realw* __restrict__ v, realw* __restrict__ out) {
+// Stacey traction of the forward field, one lane per (face point, event), written to out
+// [nfp][E][3]: the fp16 store, whose scales need the whole step's tractions first (else the
+// assembly takes them)
+__global__ void k_batch_stacey(int nfp, int E, int it, const int* __restrict__ nstep, const int* __restrict__ figlob,
+                               const realw* __restrict__ fcoef, const realw* __restrict__ v, realw* __restrict__ out) {
   const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= (size_t)nfp * E) return;
   const int ev = (int)(q % E), p = (int)(q / E);
-  const int ne = nstep[ev];
-  if (adjoint ? (it <= nmax - ne) : (it > ne)) return;
-  const size_t g = (size_t)figlob[p];
-  const realw* C = fcoef + 8 * (size_t)p;
-  const realw nx = C[0], ny = C[1], nz = C[2], jw = C[3], rvp = C[4], rvs = C[5];
-  const realw* V = v + (g * E + ev) * 3;
-  const realw vx = V[0], vy = V[1], vz = V[2];
-  const realw vn = vx * nx + vy * ny + vz * nz;
-  realw* o = out + 3 * q;
-  o[0] = (rvp * vn * nx + rvs * (vx - vn * nx)) * jw;
-  o[1] = (rvp * vn * ny + rvs * (vy - vn * ny)) * jw;
-  o[2] = (rvp * vn * nz + rvs * (vz - vn * nz)) * jw;
+  if (it > nstep[ev]) return;
+  realw tx, ty, tz;
+  batch_stacey_point(fcoef + 8 * (size_t)p, v + ((size_t)figlob[p] * E + ev) * 3, tx, ty, tz);
+  store3(out + 3 * q, tx, ty, tz);
 }
 
 // Compact Stacey store: a record (one step of one event, nfp*3 values) keeps
@@ -704,32 +787,29 @@ __global__ void k_fill_u32(unsigned int* p, size_t n) {
   if (i < n) p[i] = 0u;
 }
 
-// seismograms of the forward field, one block per (receiver, event), into
-// seis [E][NSTEP_max][nrec][3] row it-1
-__global__ __launch_bounds__(128) void k_batch_seismo(int nrec, int E, int it, int nmax,
-                                                      const int* __restrict__ nstep, const int* __restrict__ riglob,
-                                                      const realw* __restrict__ rh, const realw* __restrict__ u,
-                                                      realw* __restrict__ seis) {
-  __shared__ realw s[3][128];
-  const int r = blockIdx.x / E, ev = blockIdx.x % E, t = threadIdx.x;
-  if (it > nstep[ev]) return;  // block-uniform
-  realw x = 0, y = 0, z = 0;
-  if (t < 125) {
-    const realw h = rh[(size_t)r * 125 + t];
-    const size_t g = (size_t)riglob[(size_t)r * 125 + t];
-    const realw* U = u + (g * E + ev) * 3;
-    x = h * U[0]; y = h * U[1]; z = h * U[2];
-  }
-  s[0][t] = x; s[1][t] = y; s[2][t] = z;
+// per event, out [E][nloc]: the density kernel of every local point, -rho K, and a modulus kernel
+// scaled as save_adjoint_kernels does
+__global__ void k_batch_expand_rho(size_t nloc, int E, const int* __restrict__ ibool, const double* __restrict__ K,
+                                   const realw* __restrict__ rho, double* __restrict__ out) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nloc * E) return;
+  const size_t e = i / nloc, L = i - e * nloc;
+  out[i] = -(double)rho[L] * K[(size_t)ibool[L] * E + e];
+}
+
+__global__ void k_batch_scale(size_t nloc, int E, const double* __restrict__ K, const realw* __restrict__ modulus,
+                              double factor, double* __restrict__ out) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nloc * E) out[i] = K[i] * (factor * (double)modulus[i % nloc]);
+}
+
+// c_ij kernels of one element from rows [21][125] to the caller's [125][21], negated, through LDS
+__global__ __launch_bounds__(256) void k_batch_cij_point_major(const double* __restrict__ K, double* __restrict__ out) {
+  __shared__ double s[2625];
+  const size_t b = (size_t)blockIdx.x * 2625;
+  for (int i = threadIdx.x; i < 2625; i += 256) s[i] = K[b + i];
   __syncthreads();
-  for (int w = 64; w > 0; w >>= 1) {
-    if (t < w) { s[0][t] += s[0][t + w]; s[1][t] += s[1][t + w]; s[2][t] += s[2][t + w]; }
-    __syncthreads();
-  }
-  if (t == 0) {
-    realw* o = seis + (((size_t)ev * nmax + (it - 1)) * nrec + r) * 3;
-    o[0] = s[0][0]; o[1] = s[1][0]; o[2] = s[2][0];
-  }
+  for (int i = threadIdx.x; i < 2625; i += 256) out[b + i] = -s[(i % 21) * 125 + i / 21];
 }
 
 __global__ void k_batch_vshift(size_t n, realw* __restrict__ v, const realw* __restrict__ a, realw dto2) {
@@ -799,7 +879,7 @@ SemBatch* batch_of(long* p) {
 }
 
 template <int E>
-void launch_elem(SemBatch* B, int nf, const int* active, const int* last) {
+void launch_elem(SemBatch* B, int nf, int it, const int* active, const int* last) {
   SemMesh* m = B->m;
   BatchElemArgs A{};
   A.ibool = m->d_ibool; A.kappa = m->d_kappa; A.mu = m->d_mu;
@@ -830,7 +910,9 @@ void launch_elem(SemBatch* B, int nf, const int* active, const int* last) {
   int dev = 0, ncu = 0;
   HIP_CHECK(hipGetDevice(&dev));
   HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  const int nb = std::max(8, std::min((m->nspec + 7) & ~7, (ncu * B->blocks_per_cu + 7) & ~7));
+  A.nblk = std::max(8, std::min((m->nspec + 7) & ~7, (ncu * B->blocks_per_cu + 7) & ~7));
+  if (nf == 1 && m->nrec) A.se = BatchSeismo{m->nrec, it, B->nmax, B->d_nstep, m->d_rec_iglob, m->d_rec_h, B->seis};
+  const int nb = A.nblk + A.se.nrec * E;
   const int sp = m->static_precision;
   hipStream_t s = m->stream;
 #define LB(NF, SP)                                                                \
@@ -852,12 +934,13 @@ void launch_elem(SemBatch* B, int nf, const int* active, const int* last) {
   HIP_CHECK(hipGetLastError());
 }
 
-void elem_pass(SemBatch* B, int nf, const int* active, const int* last) {
+// it: the step (1-based), whose seismograms a forward pass takes
+void elem_pass(SemBatch* B, int nf, int it, const int* active, const int* last) {
   switch (B->E) {
-    case 1: launch_elem<1>(B, nf, active, last); break;
-    case 2: launch_elem<2>(B, nf, active, last); break;
-    case 4: launch_elem<4>(B, nf, active, last); break;
-    case 8: launch_elem<8>(B, nf, active, last); break;
+    case 1: launch_elem<1>(B, nf, it, active, last); break;
+    case 2: launch_elem<2>(B, nf, it, active, last); break;
+    case 4: launch_elem<4>(B, nf, it, active, last); break;
+    case 8: launch_elem<8>(B, nf, it, active, last); break;
     default: SEM_FAIL("batch size %d not supported (1, 2, 4, 8)", B->E);
   }
 }
@@ -879,9 +962,10 @@ void asm_pass(SemBatch* B, bool two, int it) {
   A.n_extra = in ? B->n_extra : 0;
   const size_t row = B->nfp * B->E * 3;
   if (two) {
-    A.face0 = B->face_scratch;
+    A.fcoef = m->d_face_coef;
     A.face1 = B->store_precision ? B->face_replay : B->store + (size_t)(B->nmax - it) * row;
   } else {
+    A.fcoef = B->store_precision ? nullptr : m->d_face_coef;
     A.face0 = B->store_precision ? B->face_scratch : B->store + (size_t)(it - 1) * row;
   }
   const dim3 gr(nblk(((size_t)A.n_main + A.n_extra) * B->E)), bl(TPB);
@@ -900,26 +984,23 @@ void asm_pass(SemBatch* B, bool two, int it) {
   HIP_CHECK(hipGetLastError());
 }
 
-// Stacey terms of this step.  Forward: the traction of field 0 goes to the
-// store row it-1 (fp32 store) or to the scratch, then into the fp16 record
-// it-1 with its scales; adjoint: the adjoint field's traction to the scratch
-// and, with the fp16 store, record NSTEP_max - it unpacked for the replay.
+// Stacey terms of this step that the assembly does not take itself: with the fp16 store the
+// forward field's tractions go to the scratch and into record it-1 with its scales, and record
+// NSTEP_max - it is unpacked for the replay.
 void stacey_pass(SemBatch* B, int it, bool adjoint) {
-  if (!B->nfp) return;
+  if (!B->nfp || !B->store_precision) return;
   SemMesh* m = B->m;
   hipStream_t s = m->stream;
   const int nfp = (int)B->nfp, E = B->E;
   const size_t row = B->nfp * E * 3;
-  const bool compact = B->store_precision != 0;
-  realw* out = (adjoint || compact) ? B->face_scratch : B->store + (size_t)(it - 1) * row;
-  hipLaunchKernelGGL(k_batch_stacey, dim3(nblk(B->nfp * E)), dim3(TPB), 0, s, nfp, E, it, B->nmax, (int)adjoint,
-                     B->d_nstep, m->d_face_iglob, m->d_face_coef, B->v, out);
-  if (compact && !adjoint) {
+  if (!adjoint) {
+    hipLaunchKernelGGL(k_batch_stacey, dim3(nblk(B->nfp * E)), dim3(TPB), 0, s, nfp, E, it, B->d_nstep, m->d_face_iglob,
+                       m->d_face_coef, B->v, B->face_scratch);
     unsigned int* mx = B->store_max + (size_t)(it - 1) * E;
     hipLaunchKernelGGL(k_batch_face_absmax, dim3(nblk(B->nfp * E)), dim3(TPB), 0, s, nfp, E, B->face_scratch, mx);
     hipLaunchKernelGGL(k_batch_store_pack, dim3(nblk(B->nfp * E)), dim3(TPB), 0, s, nfp, E, B->face_scratch, mx,
                        B->store16 + (size_t)(it - 1) * row);
-  } else if (compact && adjoint) {
+  } else {
     const size_t r = (size_t)(B->nmax - it);
     hipLaunchKernelGGL(k_batch_store_unpack, dim3(nblk(B->nfp * E)), dim3(TPB), 0, s, nfp, E, B->store16 + r * row,
                        B->store_max + r * E, B->face_replay);
@@ -1123,12 +1204,9 @@ void fwat_batch_forward_(long* Batch_pointer, int* timed) {
       last[e] = it == B->nstep[e];
     }
     if (tm) tm->mark(it, 0, s);
-    elem_pass(B, 1, active, last);
+    elem_pass(B, 1, it, active, last);
     if (tm) tm->mark(it, 1, s);
     stacey_pass(B, it, false);
-    if (m->nrec)
-      hipLaunchKernelGGL(k_batch_seismo, dim3(m->nrec * E), dim3(128), 0, s, m->nrec, E, it, N, B->d_nstep,
-                         m->d_rec_iglob, m->d_rec_h, B->u, B->seis);
     if (tm) tm->mark(it, 2, s);
     asm_pass(B, false, it);
     if (tm) tm->mark(it, 3, s);
@@ -1215,7 +1293,7 @@ void fwat_batch_adjoint_(long* Batch_pointer, int* timed) {
     }
     B->kflush = kb <= 1 || it % kb == 0 || it == N;  // every event is active at it == N
     if (tm) tm->mark(it, 0, s);
-    elem_pass(B, 2, active, last);
+    elem_pass(B, 2, it, active, last);
     if (tm) tm->mark(it, 1, s);
     stacey_pass(B, it, true);
     if (tm) tm->mark(it, 2, s);
@@ -1249,25 +1327,20 @@ void fwat_batch_kernels_(long* Batch_pointer, realw* h_rhostore, double* h_rho_k
   if (B->aniso) SEM_FAIL("anisotropic batch: its kernels come from fwat_batch_kernels_ani_");
   if (!B->mu_kl) SEM_FAIL("fwat_batch_adjoint_ has not run");
   const int E = B->E;
-  const size_t nloc = (size_t)m->nspec * 125, ng = (size_t)m->nglob;
-  std::vector<double> rg((size_t)E * ng);
-  std::vector<int> ib(nloc);
-  std::vector<float> kap(nloc), mu(nloc);
+  const size_t nloc = (size_t)m->nspec * 125, n = (size_t)E * nloc;
   hipStream_t s = m->stream;
-  HIP_CHECK(hipMemcpyAsync(rg.data(), B->rho_kl, rg.size() * 8, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(h_mu_kl, B->mu_kl, (size_t)E * nloc * 8, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(h_kappa_kl, B->kappa_kl, (size_t)E * nloc * 8, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(ib.data(), m->d_ibool, nloc * 4, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(kap.data(), m->d_kappa, nloc * 4, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(mu.data(), m->d_mu, nloc * 4, hipMemcpyDeviceToHost, s));
+  // scaled on the device, one array after the other through one buffer
+  realw* d_rho = dev_upload(h_rhostore, nloc, s);
+  double* tmp = dev_alloc<double>(n);
+  hipLaunchKernelGGL(k_batch_expand_rho, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, m->d_ibool, B->rho_kl, d_rho, tmp);
+  HIP_CHECK(hipMemcpyAsync(h_rho_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_batch_scale, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, B->mu_kl, m->d_mu, -2.0, tmp);
+  HIP_CHECK(hipMemcpyAsync(h_mu_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_batch_scale, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, B->kappa_kl, m->d_kappa, -1.0, tmp);
+  HIP_CHECK(hipMemcpyAsync(h_kappa_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
-  for (int e = 0; e < E; ++e)
-    for (size_t L = 0; L < nloc; ++L) {
-      const size_t q = (size_t)e * nloc + L;
-      h_rho_kl[q] = -(double)h_rhostore[L] * rg[(size_t)ib[L] * E + e];
-      h_mu_kl[q] *= -2.0 * (double)mu[L];
-      h_kappa_kl[q] *= -(double)kap[L];
-    }
+  dev_free(tmp);
+  dev_free(d_rho);
 }
 
 // Kernels of an anisotropic batch per event: rho_kl (NGLLX,NGLLY,NGLLZ,NSPEC_AB,nevents) scaled by
@@ -1279,23 +1352,19 @@ void fwat_batch_kernels_ani_(long* Batch_pointer, realw* h_rhostore, double* h_r
   if (!B->aniso) SEM_FAIL("isotropic batch: its kernels come from fwat_batch_kernels_");
   if (!B->cijkl_kl) SEM_FAIL("fwat_batch_adjoint_ has not run");
   const int E = B->E;
-  const size_t nloc = (size_t)m->nspec * 125, ng = (size_t)m->nglob;
-  std::vector<double> rg((size_t)E * ng), ck(nloc * 21);
-  std::vector<int> ib(nloc);
+  const size_t nloc = (size_t)m->nspec * 125, n = (size_t)E * nloc;
   hipStream_t s = m->stream;
-  HIP_CHECK(hipMemcpyAsync(rg.data(), B->rho_kl, rg.size() * 8, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(ib.data(), m->d_ibool, nloc * 4, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  realw* d_rho = dev_upload(h_rhostore, nloc, s);
+  double* tmp = dev_alloc<double>(std::max(n, nloc * 21));
+  hipLaunchKernelGGL(k_batch_expand_rho, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, m->d_ibool, B->rho_kl, d_rho, tmp);
+  HIP_CHECK(hipMemcpyAsync(h_rho_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
   for (int e = 0; e < E; ++e) {
-    HIP_CHECK(hipMemcpyAsync(ck.data(), B->cijkl_kl + (size_t)e * nloc * 21, ck.size() * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    double* out = h_cijkl_kl + (size_t)e * nloc * 21;
-    for (size_t el = 0; el < (size_t)m->nspec; ++el)
-      for (int q = 0; q < 21; ++q)
-        for (int L = 0; L < 125; ++L) out[(el * 125 + L) * 21 + q] = -ck[(el * 21 + q) * 125 + L];
-    for (size_t L = 0; L < nloc; ++L)
-      h_rho_kl[(size_t)e * nloc + L] = -(double)h_rhostore[L] * rg[(size_t)ib[L] * E + e];
+    hipLaunchKernelGGL(k_batch_cij_point_major, dim3(m->nspec), dim3(256), 0, s, B->cijkl_kl + (size_t)e * nloc * 21, tmp);
+    HIP_CHECK(hipMemcpyAsync(h_cijkl_kl + (size_t)e * nloc * 21, tmp, nloc * 21 * 8, hipMemcpyDeviceToHost, s));
   }
+  HIP_CHECK(hipStreamSynchronize(s));
+  dev_free(tmp);
+  dev_free(d_rho);
 }
 
 // element / assembly pass time of the last timed batch run (ms) and step counts
