@@ -10,7 +10,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ["prepare.hip", "forces.hip", "timeloop.hip", "brick.hip", "smooth_pde.hip", "batch.hip", "postproc.hip",
-           "optimize.hip", "measure.hip"]
+           "optimize.hip", "measure.hip", "transfer.hip"]
 OUT = os.path.join(HERE, "libspecfwat_hip.so")
 
 HIPCC_FLAGS = [

@@ -1313,9 +1313,7 @@ void fwat_batch_seismograms_(long* Batch_pointer, realw* h_seis) {
   SemBatch* B = batch_of(Batch_pointer);
   SemMesh* m = B->m;
   if (!m->nrec) return;
-  HIP_CHECK(hipMemcpyAsync(h_seis, B->seis, sizeof(realw) * (size_t)B->E * B->nmax * m->nrec * 3,
-                           hipMemcpyDeviceToHost, m->stream));
-  HIP_CHECK(hipStreamSynchronize(m->stream));
+  sem_to_host(h_seis, B->seis, sizeof(realw) * (size_t)B->E * B->nmax * m->nrec * 3, m->stream);
 }
 
 // Scaled kernels per event: rho_kl, mu_kl, kappa_kl (NGLLX,NGLLY,NGLLZ,NSPEC_AB,nevents), fp64,
@@ -1333,12 +1331,11 @@ void fwat_batch_kernels_(long* Batch_pointer, realw* h_rhostore, double* h_rho_k
   realw* d_rho = dev_upload(h_rhostore, nloc, s);
   double* tmp = dev_alloc<double>(n);
   hipLaunchKernelGGL(k_batch_expand_rho, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, m->d_ibool, B->rho_kl, d_rho, tmp);
-  HIP_CHECK(hipMemcpyAsync(h_rho_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
+  sem_to_host(h_rho_kl, tmp, n * 8, s);
   hipLaunchKernelGGL(k_batch_scale, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, B->mu_kl, m->d_mu, -2.0, tmp);
-  HIP_CHECK(hipMemcpyAsync(h_mu_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
+  sem_to_host(h_mu_kl, tmp, n * 8, s);
   hipLaunchKernelGGL(k_batch_scale, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, B->kappa_kl, m->d_kappa, -1.0, tmp);
-  HIP_CHECK(hipMemcpyAsync(h_kappa_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  sem_to_host(h_kappa_kl, tmp, n * 8, s);
   dev_free(tmp);
   dev_free(d_rho);
 }
@@ -1357,12 +1354,11 @@ void fwat_batch_kernels_ani_(long* Batch_pointer, realw* h_rhostore, double* h_r
   realw* d_rho = dev_upload(h_rhostore, nloc, s);
   double* tmp = dev_alloc<double>(std::max(n, nloc * 21));
   hipLaunchKernelGGL(k_batch_expand_rho, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, m->d_ibool, B->rho_kl, d_rho, tmp);
-  HIP_CHECK(hipMemcpyAsync(h_rho_kl, tmp, n * 8, hipMemcpyDeviceToHost, s));
+  sem_to_host(h_rho_kl, tmp, n * 8, s);
   for (int e = 0; e < E; ++e) {
     hipLaunchKernelGGL(k_batch_cij_point_major, dim3(m->nspec), dim3(256), 0, s, B->cijkl_kl + (size_t)e * nloc * 21, tmp);
-    HIP_CHECK(hipMemcpyAsync(h_cijkl_kl + (size_t)e * nloc * 21, tmp, nloc * 21 * 8, hipMemcpyDeviceToHost, s));
+    sem_to_host(h_cijkl_kl + (size_t)e * nloc * 21, tmp, nloc * 21 * 8, s);
   }
-  HIP_CHECK(hipStreamSynchronize(s));
   dev_free(tmp);
   dev_free(d_rho);
 }

@@ -1974,6 +1974,52 @@ __global__ void k_fill_f32m(size_t n, float* __restrict__ x) {
 
 double g_meas_ms = 0.0;
 
+// Device scratch of one call, cut from a few large blocks that are given back together: giving back
+// a block of 100 MB or more takes 0.23 ms, and a call has a dozen such arrays.
+class Scratch {
+  std::vector<void*> blocks_;
+  char* at_ = nullptr;
+  size_t left_ = 0;
+
+ public:
+  Scratch() = default;
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  ~Scratch() {
+    for (void* p : blocks_) HIP_CHECK(hipFree(p));
+  }
+  template <class T>
+  T* alloc(size_t n) {
+    if (n == 0) return nullptr;
+    const size_t bytes = (n * sizeof(T) + 255) & ~(size_t)255;
+    if (bytes > left_) {
+      left_ = std::max(bytes * 8, (size_t)1 << 20);  // room for arrays like this one
+      if (left_ > (size_t)1 << 30) left_ = std::max(bytes, (size_t)1 << 30);
+      void* p = nullptr;
+      if (left_ > bytes && hipMalloc(&p, left_) != hipSuccess) {
+        (void)hipGetLastError();  // little memory left: this array alone
+        p = nullptr;
+      }
+      if (!p) {
+        left_ = bytes;
+        HIP_CHECK(hipMalloc(&p, left_));
+      }
+      blocks_.push_back(p);
+      at_ = (char*)p;
+    }
+    T* p = reinterpret_cast<T*>(at_);
+    at_ += bytes;
+    left_ -= bytes;
+    return p;
+  }
+  template <class T>
+  T* upload(const T* h, size_t n, hipStream_t s) {
+    T* p = alloc<T>(n);
+    if (n) HIP_CHECK(hipMemcpyAsync(p, h, n * sizeof(T), hipMemcpyHostToDevice, s));
+    return p;
+  }
+};
+
 // window_taper's weights (signal.f90:419-491) for a window of npts samples
 void taper_weights_into(int npts, double pct, int type, double* w);
 
@@ -2267,7 +2313,7 @@ void fwat_waveform_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* ob
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipEventRecord(e1, s));
   std::vector<double> mr(2 * (size_t)nw * T);
-  HIP_CHECK(hipMemcpyAsync(adj, d_adj, n * sizeof(float), hipMemcpyDeviceToHost, s));
+  sem_to_host(adj, d_adj, n * sizeof(float), s);
   HIP_CHECK(hipMemcpyAsync(mr.data(), d_mr, mr.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0.0f;
@@ -2379,14 +2425,15 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   const size_t n = (size_t)N * T;
   hipStream_t s;
   HIP_CHECK(hipStreamCreate(&s));
+  Scratch scratch;
   hipEvent_t e0, e1;
   HIP_CHECK(hipEventCreate(&e0));
   HIP_CHECK(hipEventCreate(&e1));
-  float* d_obs = dev_upload(obs, n, s);
-  float* d_syn = dev_upload(syn, n, s);
-  float* d_adj = dev_alloc<float>(n);
-  int* d_ish = dev_alloc<int>(T);
-  double* d_out = dev_alloc<double>(8 * (size_t)nw * T);
+  float* d_obs = scratch.upload(obs, n, s);
+  float* d_syn = scratch.upload(syn, n, s);
+  float* d_adj = scratch.alloc<float>(n);
+  int* d_ish = scratch.alloc<int>(T);
+  double* d_out = scratch.alloc<double>(8 * (size_t)nw * T);
   int maxnl = 0;
   std::vector<int> nbs(nw), nls(nw);
   std::vector<std::vector<double>> tws(nw);
@@ -2398,10 +2445,10 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     wmin = std::min(wmin, std::min(windows[2 * w], windows[2 * w + 1]));
     wmax = std::max(wmax, std::max(windows[2 * w], windows[2 * w + 1]));
   }
-  double* d_D = dev_alloc<double>((size_t)T * maxnl);
-  double* d_S = dev_alloc<double>((size_t)T * maxnl);
-  double* d_tw = dev_alloc<double>(maxnl);
-  double* d_A = dev_alloc<double>((size_t)T * maxnl);
+  double* d_D = scratch.alloc<double>((size_t)T * maxnl);
+  double* d_S = scratch.alloc<double>((size_t)T * maxnl);
+  double* d_tw = scratch.alloc<double>(maxnl);
+  double* d_A = scratch.alloc<double>((size_t)T * maxnl);
   CcShift shift(T, nls, s);
   HIP_CHECK(hipEventRecord(e0, s));
   hipLaunchKernelGGL(k_fill_f32m, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, d_adj);
@@ -2427,8 +2474,8 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     int fnb = 0, fnl = 0;
     window_range(wmin, wmax, *dt, N, fnb, fnl);
     taper_weights(fnl, *taper_percentage, *itaper_type, fw);
-    d_fw = dev_upload(fw.data(), fw.size(), s);
-    d_sos = dev_upload(sos, 6 * (size_t)*nsect, s);
+    d_fw = scratch.upload(fw.data(), fw.size(), s);
+    d_sos = scratch.upload(sos, 6 * (size_t)*nsect, s);
     launch_sos(s, N, T, *nsect, d_sos, d_adj);
     hipLaunchKernelGGL(k_window_final, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, N, T, fnb, fnl, d_fw,
                        d_adj);
@@ -2436,7 +2483,7 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipEventRecord(e1, s));
   std::vector<double> out(8 * (size_t)nw * T);
-  HIP_CHECK(hipMemcpyAsync(adj, d_adj, n * sizeof(float), hipMemcpyDeviceToHost, s));
+  sem_to_host(adj, d_adj, n * sizeof(float), s);
   HIP_CHECK(hipMemcpyAsync(out.data(), d_out, out.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0.0f;
@@ -2451,8 +2498,6 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     }
     misfits[t] = m;
   }
-  dev_free(d_obs); dev_free(d_syn); dev_free(d_adj); dev_free(d_ish); dev_free(d_out); dev_free(d_D); dev_free(d_S);
-  dev_free(d_tw); dev_free(d_fw); dev_free(d_sos); dev_free(d_A);
   shift.free_all();
   HIP_CHECK(hipEventDestroy(e0));
   HIP_CHECK(hipEventDestroy(e1));
@@ -2584,7 +2629,7 @@ void fwat_mt_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipEventRecord(ev1, s));
   std::vector<double> out(10 * (size_t)nw * T);
-  HIP_CHECK(hipMemcpyAsync(adj, d_adj, n * sizeof(float), hipMemcpyDeviceToHost, s));
+  sem_to_host(adj, d_adj, n * sizeof(float), s);
   HIP_CHECK(hipMemcpyAsync(out.data(), d_out, out.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0.0f;
@@ -2700,7 +2745,7 @@ void fwat_ep_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipEventRecord(ev1, s));
   std::vector<double> out(8 * (size_t)nw * T);
-  HIP_CHECK(hipMemcpyAsync(adj, d_adj, n * sizeof(float), hipMemcpyDeviceToHost, s));
+  sem_to_host(adj, d_adj, n * sizeof(float), s);
   HIP_CHECK(hipMemcpyAsync(out.data(), d_out, out.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0.0f;
@@ -2752,25 +2797,26 @@ void fwat_win_sel_batch_(int* nstep, int* ntrace, double* dt, realw* obs, realw*
   const size_t n = (size_t)N * T;
   hipStream_t s;
   HIP_CHECK(hipStreamCreate(&s));
+  Scratch scratch;
   hipEvent_t ev0, ev1;
   HIP_CHECK(hipEventCreate(&ev0));
   HIP_CHECK(hipEventCreate(&ev1));
-  float* d_obs = dev_upload(obs, n, s);
-  float* d_syn = dev_upload(syn, n, s);
-  double* d_tp = dev_upload(tp, (size_t)T, s);
-  double* d_dist = dev_upload(dist, (size_t)T, s);
-  double* d_wt = dev_upload(wt.data(), wt.size(), s);
-  float* d_obsT = dev_alloc<float>(n);
-  float* d_synT = dev_alloc<float>(n);
-  double* d_Dn = dev_alloc<double>(n);
-  double* d_Sn = dev_alloc<double>(n);
-  double* d_noise = dev_alloc<double>(T);
-  double* d_ts = dev_alloc<double>((size_t)nw * T);
-  double* d_cc = dev_alloc<double>((size_t)nw * T);
-  int* d_ish = dev_alloc<int>((size_t)nw * T);
-  int* d_nwin = dev_alloc<int>(T);
-  double* d_win = dev_alloc<double>(2 * (size_t)*maxwin * T);
-  unsigned char* d_good = dev_alloc<unsigned char>((size_t)nw * T);
+  float* d_obs = scratch.upload(obs, n, s);
+  float* d_syn = scratch.upload(syn, n, s);
+  double* d_tp = scratch.upload(tp, (size_t)T, s);
+  double* d_dist = scratch.upload(dist, (size_t)T, s);
+  double* d_wt = scratch.upload(wt.data(), wt.size(), s);
+  float* d_obsT = scratch.alloc<float>(n);
+  float* d_synT = scratch.alloc<float>(n);
+  double* d_Dn = scratch.alloc<double>(n);
+  double* d_Sn = scratch.alloc<double>(n);
+  double* d_noise = scratch.alloc<double>(T);
+  double* d_ts = scratch.alloc<double>((size_t)nw * T);
+  double* d_cc = scratch.alloc<double>((size_t)nw * T);
+  int* d_ish = scratch.alloc<int>((size_t)nw * T);
+  int* d_nwin = scratch.alloc<int>(T);
+  double* d_win = scratch.alloc<double>(2 * (size_t)*maxwin * T);
+  unsigned char* d_good = scratch.alloc<unsigned char>((size_t)nw * T);
   // phase splitting: envelope transform on nf = 2 ** exponent(real(nstep)) points
   int nfe = 0, Me = 0, logMe = 0;
   double *d_env = nullptr, *d_stl = nullptr;
@@ -2787,10 +2833,10 @@ void fwat_win_sel_batch_(int* nstep, int* ntrace, double* dt, realw* obs, realw*
       twh[2 * j] = (double)std::cos(a);
       twh[2 * j + 1] = (double)std::sin(a);
     }
-    d_twe = reinterpret_cast<double2*>(dev_upload(twh.data(), twh.size(), s));
-    d_env = dev_alloc<double>(n);
-    d_stl = dev_alloc<double>(n);
-    d_g01 = dev_alloc<double2>(2 * (size_t)T * (Me + 1));
+    d_twe = reinterpret_cast<double2*>(scratch.upload(twh.data(), twh.size(), s));
+    d_env = scratch.alloc<double>(n);
+    d_stl = scratch.alloc<double>(n);
+    d_g01 = scratch.alloc<double2>(2 * (size_t)T * (Me + 1));
   }
   HIP_CHECK(hipEventRecord(ev0, s));
   const dim3 ttiles((unsigned)((T + 63) / 64), (unsigned)((N + 63) / 64));
@@ -2821,10 +2867,6 @@ void fwat_win_sel_batch_(int* nstep, int* ntrace, double* dt, realw* obs, realw*
   float ms = 0.0f;
   HIP_CHECK(hipEventElapsedTime(&ms, ev0, ev1));
   g_meas_ms = ms;
-  dev_free(d_obs); dev_free(d_syn); dev_free(d_tp); dev_free(d_dist); dev_free(d_wt); dev_free(d_obsT);
-  dev_free(d_synT); dev_free(d_Dn); dev_free(d_Sn); dev_free(d_noise); dev_free(d_ts); dev_free(d_cc); dev_free(d_ish);
-  dev_free(d_nwin); dev_free(d_win); dev_free(d_good); dev_free(d_env); dev_free(d_stl); dev_free(d_g01);
-  dev_free(d_twe);
   for (int t = 0; t < T; ++t)
     if (nwin[t] < 0) SEM_FAIL("fwat_win_sel_batch_: trace %d has more than %d good groups", t, WS_MAXG);
   HIP_CHECK(hipEventDestroy(ev0));
@@ -2895,8 +2937,8 @@ void fwat_conv_adjoint_batch_(int* nstep, int* nrec, double* dt, realw* dat_r, r
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipEventRecord(ev1, s));
   std::vector<double> out(2 * (size_t)R);
-  HIP_CHECK(hipMemcpyAsync(adj_r, d_ar_out, n * sizeof(float), hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipMemcpyAsync(adj_z, d_az_out, n * sizeof(float), hipMemcpyDeviceToHost, s));
+  sem_to_host(adj_r, d_ar_out, n * sizeof(float), s);
+  sem_to_host(adj_z, d_az_out, n * sizeof(float), s);
   HIP_CHECK(hipMemcpyAsync(out.data(), d_out, out.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
   float ms = 0.0f;

@@ -286,6 +286,9 @@ inline T* dev_alloc(size_t n) {
   return p;
 }
 
+// copy to ordinary host memory, complete on return; large ones through several threads (transfer.hip)
+void sem_to_host(void* host, const void* dev, size_t bytes, hipStream_t s);
+
 template <class T>
 inline T* dev_upload(const T* h, size_t n, hipStream_t s) {
   T* p = dev_alloc<T>(n);

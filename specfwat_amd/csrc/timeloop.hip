@@ -935,9 +935,7 @@ void compute_seismograms_cuda_(long* Mesh_pointer, int* it) {
 void transfer_seismograms_from_device_(long* Mesh_pointer, realw* h_seismograms) {
   SemMesh* m = sem_mesh(Mesh_pointer);
   if (m->nrec == 0) return;
-  HIP_CHECK(hipMemcpyAsync(h_seismograms, m->d_seismograms, sizeof(realw) * (size_t)m->nstep * m->nrec * 3,
-                           hipMemcpyDeviceToHost, m->stream));
-  HIP_CHECK(hipStreamSynchronize(m->stream));
+  sem_to_host(h_seismograms, m->d_seismograms, sizeof(realw) * (size_t)m->nstep * m->nrec * 3, m->stream);
 }
 
 // Kernel accumulation of one adjoint step from the stored strains
@@ -970,15 +968,13 @@ void transfer_kernels_el_to_host_dp_(long* Mesh_pointer, double* h_rho_kl, doubl
   double* tmp = dev_alloc<double>(nloc);
   hipLaunchKernelGGL(k_expand_glob, dim3(nblk(nloc)), dim3(TPB), 0, s, m->nspec, m->d_ibool,
                      m->d_rho_kl_glob, -1.0, m->d_rho, tmp);
-  HIP_CHECK(hipMemcpyAsync(h_rho_kl, tmp, nloc * 8, hipMemcpyDeviceToHost, s));
-  HIP_CHECK(hipStreamSynchronize(s));
+  sem_to_host(h_rho_kl, tmp, nloc * 8, s);
   if (!m->anisotropic_kl) {
     // scaled on the device: the host loop over both arrays took as long as 40 adjoint steps (64x64x32)
     hipLaunchKernelGGL(k_scale_kernel, dim3(nblk(nloc)), dim3(TPB), 0, s, nloc, m->d_mu_kl, m->d_mu, -2.0, tmp);
-    HIP_CHECK(hipMemcpyAsync(h_mu_kl, tmp, nloc * 8, hipMemcpyDeviceToHost, s));
+    sem_to_host(h_mu_kl, tmp, nloc * 8, s);
     hipLaunchKernelGGL(k_scale_kernel, dim3(nblk(nloc)), dim3(TPB), 0, s, nloc, m->d_kappa_kl, m->d_kappa, -1.0, tmp);
-    HIP_CHECK(hipMemcpyAsync(h_kappa_kl, tmp, nloc * 8, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    sem_to_host(h_kappa_kl, tmp, nloc * 8, s);
   }
   dev_free(tmp);
 }
@@ -1004,8 +1000,7 @@ void transfer_kernels_ani_to_host_dp_(long* Mesh_pointer, double* h_cijkl_kl, in
   const size_t nloc = (size_t)m->nspec * 125;
   double* tmp = dev_alloc<double>(nloc * 21);
   hipLaunchKernelGGL(k_cij_point_major, dim3(m->nspec), dim3(256), 0, m->stream, m->d_cijkl_kl, tmp);
-  HIP_CHECK(hipMemcpyAsync(h_cijkl_kl, tmp, nloc * 21 * 8, hipMemcpyDeviceToHost, m->stream));
-  HIP_CHECK(hipStreamSynchronize(m->stream));
+  sem_to_host(h_cijkl_kl, tmp, nloc * 21 * 8, m->stream);
   dev_free(tmp);
 }
 
@@ -1018,8 +1013,7 @@ void transfer_kernels_hess_el_tohost_dp_(long* Mesh_pointer, double* h_hess_kl, 
   double* tmp = dev_alloc<double>(nloc);
   hipLaunchKernelGGL(k_expand_glob, dim3(nblk(nloc)), dim3(TPB), 0, m->stream, m->nspec, m->d_ibool,
                      m->d_hess_kl_glob, 1.0, (const realw*)nullptr, tmp);
-  HIP_CHECK(hipMemcpyAsync(h_hess_kl, tmp, nloc * 8, hipMemcpyDeviceToHost, m->stream));
-  HIP_CHECK(hipStreamSynchronize(m->stream));
+  sem_to_host(h_hess_kl, tmp, nloc * 8, m->stream);
   dev_free(tmp);
 }
 

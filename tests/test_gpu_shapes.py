@@ -1,0 +1,126 @@
+"""Kernels at the sizes and inputs where their tiles, remainders and fast paths can go wrong,
+against the oracle or the plain statement of the same computation."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from specfwat_amd import misfit
+from specfwat_amd.mesh import BoxMesh
+from specfwat_amd.solver import ElasticRun
+from specfwat_amd.sources import Receivers, Sources
+from test_gpu_parity import KERN_TOL, SEIS_TOL, make_case, oracle_of, rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,dt,T,len_fac", [
+    ("slow", 0.01, 0.8, 1.0), ("slow", 0.005, 1.0, 1.6), ("fast", 0.02, 2.0, 2.0), ("quiet", 0.02, 2.0, 2.56),
+    ("square", 0.02, 2.0, 2.0), ("zero", 0.02, 2.0, 2.0), ("long", 0.002, 2.0, 4.0)])
+def test_sliding_lags_with_many_candidates(kind, dt, T, len_fac):
+    """Window selection where single precision cannot tell the lags apart: periods of hundreds of
+    samples (neighbouring lags differ by less than the sums' rounding), quiet stretches 1e-9 below
+    the trace's maximum, exact ties (square waves) and data that are zero; windows of 81, 321,
+    201, 257 and 4,001 samples.  The same windows as the oracle, which sums every lag in double."""
+    rng = np.random.default_rng(3)
+    nstep, nrec = (4101, 1) if kind == "long" else (2400, 2)
+    print(f"sliding lags: {kind}, {int(len_fac * T / dt) + 1} samples", flush=True)
+    t = np.arange(nstep) * dt
+    span = nstep * dt
+    obs, syn = np.zeros((nstep, nrec, 3), np.float32), np.zeros((nstep, nrec, 3), np.float32)
+    tp, dist = (np.array([0.3, 0.25]) * span)[:nrec], (np.array([2.0, 2.2]) * span)[:nrec]
+    for r in range(nrec):
+        for c in range(3):
+            f, env = {"slow": (0.12, 0.06), "long": (8.0, 0.25)}.get(kind, (0.5, 0.25))
+            w = lambda s: np.exp(-((t - 0.55 * span - s) * env) ** 2) * np.sin(2 * np.pi * f * (t - s))
+            if kind == "square":
+                w = lambda s: np.sign(np.sin(2 * np.pi * f * (t - np.round(s / dt) * dt) + 1e-3))
+            syn[:, r, c] = w(0.0)
+            obs[:, r, c] = w(0.04 * (r + 1)) + 1e-3 * rng.standard_normal(nstep) * (kind == "fast")
+            if kind == "quiet":
+                obs[:nstep // 2, r, c] *= 1e-9
+                syn[:nstep // 2, r, c] *= 1e-9
+    if kind == "zero":
+        obs[:, 0] = 0
+        obs[:nstep // 2, 1] = 0
+    cfg = dict(sliding_win_len_fac=len_fac, min_peaks_troughs=1, min_snr_window=0.1, min_win_len_fac=0.05)
+    got = misfit.select_windows(obs, syn, dt, 0.0, tp, dist, T, **cfg)
+    n = 0
+    for r in range(nrec):
+        for c in range(3):
+            ref, _, _ = orc.win_sel(obs[:, r, c], syn[:, r, c], dt, 0.0, tp[r], dist[r], T, **cfg)
+            np.testing.assert_array_equal(got[3 * r + c], ref)
+            n += len(ref)
+    assert n > 0 or kind in ("zero", "square")
+    print(f"windows: {n}", flush=True)
+
+
+@pytest.mark.parametrize("nl", [128, 129, 1024, 1025, 4096, 4097, 8192, 8193])
+def test_correlation_shift_by_transforms(nl):
+    """xcorr_shift at both ends of the transform path's range and of its lengths (nl 128 and 8193
+    take the direct sums), with ties: a periodic window, whose best lags' sums differ by the
+    taper only, a square wave and zero data.  The shifts of the oracle's direct sums."""
+    nstep, dt = nl + 7, 0.01
+    rng = np.random.default_rng(nl)
+    t = np.arange(nstep)
+    obs, syn = np.zeros((nstep, 2, 3), np.float32), np.zeros((nstep, 2, 3), np.float32)
+    wave = np.exp(-((t - 0.5 * nl) / (0.1 * nl)) ** 2) * np.sin(2 * np.pi * t / (0.07 * nl))
+    shift = max(1, min(nl // 40, 300))
+    for k, (o, s) in enumerate([(np.roll(wave, shift), wave), (1e-12 * np.roll(wave, -shift), wave),
+                                (np.sin(2 * np.pi * t / 16.0), np.sin(2 * np.pi * (t - 3) / 16.0)),
+                                (np.sign(np.sin(2 * np.pi * t / 32 + 0.1)), np.sign(np.sin(2 * np.pi * (t - 4) / 32 + 0.1))),
+                                (rng.standard_normal(nstep), rng.standard_normal(nstep)), (0 * t, wave)]):
+        obs[:, k // 3, k % 3], syn[:, k // 3, k % 3] = o, s
+    win = [[0.03, 0.03 + nl * dt + 0.001]]
+    print(f"correlation of {nl} samples", flush=True)
+    _, _, meas = misfit.event_cc_adjoint_sources(obs, syn, dt, win, imeas=11)
+    for k in range(6):
+        _, _, o = orc.cc_adjoint(obs[:, k // 3, k % 3], syn[:, k // 3, k % 3], dt, win, imeas=11)
+        if k == 5:  # zero data: the error and the coefficient are not numbers; the shift is the first lag
+            assert meas[k, 0, 7] == 1 - (int(win[0][1] / dt) - int(win[0][0] / dt))
+            continue
+        assert meas[k, 0, 4] == pytest.approx(o["tshift"][0], abs=1e-12), k
+
+
+@pytest.mark.parametrize("nrec", [1, 3, 4, 5, 9])
+def test_many_receivers_in_one_element(nrec):
+    """Every receiver in one element on an absorbing side: a point's row then ends in nrec receiver
+    terms, read four at a time, after its face and source terms; forward and adjoint runs against
+    the FP64 oracle, with the tractions taken inside the assembly."""
+    c = make_case(nex=4, ney=3, nez=3, seed=60 + nrec, nstep=140)
+    m = c["mesh"]
+    rng = np.random.default_rng(nrec)
+    c["rxyz"] = np.stack([rng.uniform(0.02, 0.23, nrec) * m.lx, rng.uniform(0.02, 0.31, nrec) * m.ly, np.zeros(nrec)], axis=1)
+    c["sxyz"] = [[0.12 * m.lx, 0.2 * m.ly, -0.15 * m.lz]]
+    o = oracle_of(c, 64)
+    obs = o.forward(save=True)
+    adj = (0.5 * obs).astype(np.float32)
+    ko = o.adjoint(adj)
+    src, rec = Sources(m, c["sxyz"], c["mt"], c["f0"]), Receivers(m, c["rxyz"])
+    assert len(set(rec.ispec)) == 1
+    f = ElasticRun(m, c["rho"], c["vp"], c["vs"], src, rec, c["dt"], c["nstep"], 1, True)
+    f.iterate_time()
+    assert rel(f.seismograms(), obs) < SEIS_TOL
+    a = ElasticRun(m, c["rho"], c["vp"], c["vs"], src, rec, c["dt"], c["nstep"], 3, False)
+    a.take_forward(f)
+    a.set_adjoint_sources(adj)
+    a.iterate_time()
+    k = a.kernels()
+    for n in ("rho_kl", "mu_kl", "kappa_kl"):
+        assert rel(k[n], ko[n]) < KERN_TOL, n
+    f.close()
+    a.close()
+
+
+@pytest.mark.parametrize("nrec", [341, 342, 347, 683])
+def test_large_results_arrive_whole(nrec):
+    """Adjoint sources of 4,096 samples, 48 KiB a receiver: from 16 MiB on results are copied in
+    pieces by several threads; below, at and above that size, with ragged last pieces.  The traces
+    repeat those of seven receivers, so each has to equal its part of the small call's result."""
+    n, dt = 4096, 0.05
+    rng = np.random.default_rng(nrec)
+    obs, syn = (rng.standard_normal((n, 7, 3)).astype(np.float32) for _ in range(2))
+    q = np.arange(nrec) % 7
+    small = misfit.event_adjoint_sources(obs, syn, dt, [[1.0, 200.0]])[1]
+    large = misfit.event_adjoint_sources(obs[:, q], syn[:, q], dt, [[1.0, 200.0]])[1]
+    assert np.abs(small).max() > 0
+    np.testing.assert_array_equal(large, small[:, q])
