@@ -15,8 +15,9 @@
 // Differences in mechanism (not in result): the reference scatters with
 // atomics into ddat, launches 4-5 kernels per diffusion step (memset, two
 // phase launches, apply_mass, keep_pml) and exchanges halos over MPI; here
-// the element pass writes element-local terms and one gather launch per step
-// sums them per point in element order (the reference CPU loop's order, no
+// the element pass finishes the points that belong to one element only and
+// writes element-local terms of the others, one gather launch per step sums
+// those per point in element order (the reference CPU loop's order, no
 // atomics, run-to-run reproducible) fused with dat += rvol * ddat, the
 // element phases are merged (single GPU), and up to 24 fields share one
 // geometry read with the fields innermost in HBM ([nglob][fields]).
@@ -25,6 +26,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace {
 
@@ -36,175 +38,236 @@ inline unsigned sm_blocks(size_t n) { return (unsigned)((n + SM_TPB - 1) / SM_TP
 struct SmoothArgs {
   const int* ibool;       // 0-based [nspec][125]
   const int* irregular;   // [nspec]
-  const realw* jinv9;     // [nirr][9][125]
+  const realw* jinv9;     // [9][nirr][125], as the caller's nine arrays
+  size_t jstride;         // nirr * 125
   const realw* jac;       // [nspec][125]  (jacobian_all)
   const realw* rot;       // [nspec][3][125] when spherical
   const realw* tables;    // hprimeT[25] hprimewgll[25] wgllwgll_yz[25] _xz[25] _xy[25]
-  const realw* dat;       // [nglob][NFP]
-  realw* dloc;            // [nspec][125][NFP] element-local -(weak-form stiffness term)
+  const realw* rvol;      // [nglob]
+  realw* dat;             // [nglob][NFP]
+  realw* dloc;            // [nspec][125][NFP] element-local -(weak-form stiffness term), rows by sem_floc_slot
   int nspec, nfield;
+  int n_shared;           // points from here on belong to one element
   int nblocks_padded;
   realw cv, ch, xix_regular;
+  realw cxh, cxv;         // ch and cv times xix_regular^2
   int is_sph;
   int faithful;
 };
 
-// Element pass: one element per 128-lane workgroup; every lane loads the NFP
-// field values of its point in one contiguous read, the fields are then
-// processed one after the other out of LDS (geometry read once for all), and
-// each lane writes its NFP element-local results in one contiguous write.
+// Rows of NFP values per point in pieces of 16 bytes when NFP is a multiple of 4, else of 4 bytes.
+template <int W>
+struct SmoothPiece {
+  using T = realw;
+  __device__ static __forceinline__ T zero() { return 0.0f; }
+  __device__ static __forceinline__ T fma_s(T x, realw h, T y) { return fmaf(x, h, y); }
+  __device__ static __forceinline__ T mul_s(T x, realw h) { return x * h; }
+};
+template <>
+struct SmoothPiece<4> {
+  using T = float4;
+  __device__ static __forceinline__ T zero() { return make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
+  __device__ static __forceinline__ T fma_s(T x, realw h, T y) {
+    return make_float4(fmaf(x.x, h, y.x), fmaf(x.y, h, y.y), fmaf(x.z, h, y.z), fmaf(x.w, h, y.w));
+  }
+  __device__ static __forceinline__ T mul_s(T x, realw h) { return make_float4(x.x * h, x.y * h, x.z * h, x.w * h); }
+};
 template <int NFP>
+struct SmoothRow {
+  static constexpr int W = NFP % 4 == 0 ? 4 : 1, C = NFP / W;  // values per piece, pieces per row
+};
+
+// Element pass: one element per 128-lane workgroup.  The rows of the element's points go to LDS
+// by consecutive lanes taking consecutive pieces of a row (a wave's access then covers eleven
+// 96-byte rows whole at 24 fields; a lane per row touches 64 rows in 16-byte pieces), the fields
+// are then processed a piece (four fields) at a time between two barriers, geometry read once for
+// all, and the element-local terms leave LDS the same way, into rows in the order of sem_floc_slot.
+//   * Points of one element only (numbered last, [n_shared, nglob)) have no other term: their
+//     diffusion step dat += rvol * term is taken here and nothing of them is stored (27 of an
+//     element's 125 rows), in place, since no other element reads them.
+//   * REG: axis-aligned cubes with the diagonal map, whose fluxes are one factor per direction.
+// LDS holds the pieces as they are: gfx950 reads 16 bytes a lane at twice the rate of 4
+// (5.7e7 LDS cycles a launch with one value per lane and read, 4.4e7 with pieces).  Rows of 1 to 3 values
+// are moved by the lane of their point, which needs no second trip through LDS.
+// 32x32x16 cubes, 21 fields: 119 us a step with a lane per row, one field between two barriers and
+// every row stored, 118 us with a third of the gather's work done here (the gather 94 -> 46 us);
+// LDS and arithmetic are each busy half of the time.
+template <int NFP, bool REG>
 __global__ __launch_bounds__(128) void k_smooth_elem(SmoothArgs A) {
+  constexpr int W = SmoothRow<NFP>::W, C = SmoothRow<NFP>::C;
+  using P = SmoothPiece<W>;
+  using T = typename P::T;
+  constexpr int SU = 131;  // pieces c and c + 1 of a point 12 banks apart: rows go in and out without conflicts
   __shared__ realw s_tab[128];
-  __shared__ realw s_u[NFP][128];
-  __shared__ realw s_t[3][128];
+  __shared__ int s_g[125];
+  __shared__ uint8_t s_row[125];  // local point of each row
+  __shared__ T s_u[C * SU];       // piece c of local point p at c * SU + p
+  __shared__ T s_t[3][128];
   const int t = threadIdx.x;
-  if (t < 125) s_tab[t] = A.tables[t];
   const int e = xcd_remap(blockIdx.x, A.nblocks_padded);
   if (e >= A.nspec) return;  // block-uniform
-  const bool act = t < 125;
-  const int tt = act ? t : 124;
+  const int tt = min(t, 124);
   const int I = tt % 5, J = (tt / 5) % 5, K = tt / 25;
-  __syncthreads();
-  // mxm_opt{x,y,z} of the reference: u(l,J,K) * hprimeT[I*5+l], etc.
-  realw hpI[5], hpJ[5], hpK[5], hwI[5], hwJ[5], hwK[5];
-#pragma unroll
-  for (int l = 0; l < 5; ++l) {
-    hpI[l] = s_tab[I * 5 + l];
-    hpJ[l] = s_tab[J * 5 + l];
-    hpK[l] = s_tab[K * 5 + l];
-    hwI[l] = s_tab[25 + I * 5 + l];
-    hwJ[l] = s_tab[25 + J * 5 + l];
-    hwK[l] = s_tab[25 + K * 5 + l];
+  const size_t L0 = (size_t)e * 125, Lg = L0 + tt;
+  if (t < 125) {
+    s_tab[t] = A.tables[t];
+    if constexpr (W == 4) {
+      s_g[t] = A.ibool[Lg];
+      s_row[sem_floc_slot(t)] = (uint8_t)t;
+    }
   }
-  const realw fac1 = s_tab[50 + K * 5 + J];
-  const realw fac2 = s_tab[75 + K * 5 + I];
-  const realw fac3 = s_tab[100 + J * 5 + I];
-  const size_t Lg = (size_t)e * 125 + tt;
-  const int iglob = A.ibool[Lg];
-  const int ir = A.irregular[e];
-  realw xix, xiy, xiz, etx, ety, etz, gax, gay, gaz;
-  if (ir) {
-    const realw* G = A.jinv9 + (size_t)(ir - 1) * 1125 + tt;
-    xix = G[0]; xiy = G[125]; xiz = G[250];
-    etx = G[375]; ety = G[500]; etz = G[625];
-    gax = G[750]; gay = G[875]; gaz = G[1000];
-  } else if (A.faithful) {
-    xix = xiy = xiz = etx = ety = etz = gax = gay = gaz = A.xix_regular;
-  } else {
-    xix = ety = gaz = A.xix_regular;
-    xiy = xiz = etx = etz = gax = gay = 0.0f;
-  }
+  // geometry, requested with the points
   const realw jl = A.jac[Lg];
-  realw rx = 0, ry = 0, rz = 0;
-  if (A.is_sph) {
-    rx = A.rot[(size_t)e * 375 + tt];
-    ry = A.rot[(size_t)e * 375 + 125 + tt];
-    rz = A.rot[(size_t)e * 375 + 250 + tt];
-  }
-  if (act) {
-    const realw* D = A.dat + (size_t)iglob * NFP;
-    if constexpr (NFP % 4 == 0) {
+  realw g[REG ? 1 : 3][3], r[3] = {0.0f, 0.0f, 1.0f};
+  if constexpr (!REG) {
+    const int ir = A.irregular[e];
+    if (ir) {
+      const realw* Gm = A.jinv9 + (size_t)(ir - 1) * 125 + tt;
 #pragma unroll
-      for (int k = 0; k < NFP / 4; ++k) {
-        const float4 v = reinterpret_cast<const float4*>(D)[k];
-        s_u[4 * k][t] = v.x; s_u[4 * k + 1][t] = v.y; s_u[4 * k + 2][t] = v.z; s_u[4 * k + 3][t] = v.w;
-      }
+      for (int q = 0; q < 9; ++q) g[q / 3][q % 3] = Gm[q * A.jstride];
     } else {
 #pragma unroll
-      for (int k = 0; k < NFP; ++k) s_u[k][t] = D[k];
+      for (int q = 0; q < 9; ++q) g[q / 3][q % 3] = A.faithful || q % 4 == 0 ? A.xix_regular : 0.0f;
     }
+    if (A.is_sph)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) r[c] = A.rot[(size_t)e * 375 + 125 * c + tt];
+  }
+  T* dat = reinterpret_cast<T*>(A.dat);
+  const int own = A.ibool[Lg];
+  if constexpr (W == 1) {
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      if (t < 125) s_u[c * SU + t] = dat[(size_t)own * C + c];
   }
   __syncthreads();
-  const realw cv = A.cv, ch = A.ch;
-#pragma unroll 1
-  for (int f = 0; f < A.nfield; ++f) {
-    realw t1 = 0, t2 = 0, t3 = 0;
+  if constexpr (W == 4)
+    for (int q = t; q < 125 * C; q += 128) {
+      const int p = q / C, c = q - p * C;
+      s_u[c * SU + p] = dat[(size_t)s_g[p] * C + c];
+    }
+  // mxm_opt{x,y,z} of the reference: u(l,J,K) * hprimeT[I*5+l], etc.; the quadrature factor and
+  // the sign are folded into the second tables
+  realw hpI[5], hpJ[5], hpK[5], hwI[5], hwJ[5], hwK[5];
+  {
+    const realw fac1 = -s_tab[50 + K * 5 + J], fac2 = -s_tab[75 + K * 5 + I], fac3 = -s_tab[100 + J * 5 + I];
 #pragma unroll
     for (int l = 0; l < 5; ++l) {
-      t1 += s_u[f][l + 5 * J + 25 * K] * hpI[l];
-      t2 += s_u[f][I + 5 * l + 25 * K] * hpJ[l];
-      t3 += s_u[f][I + 5 * J + 25 * l] * hpK[l];
+      hpI[l] = s_tab[I * 5 + l];
+      hpJ[l] = s_tab[J * 5 + l];
+      hpK[l] = s_tab[K * 5 + l];
+      hwI[l] = s_tab[25 + I * 5 + l] * fac1;
+      hwJ[l] = s_tab[25 + J * 5 + l] * fac2;
+      hwK[l] = s_tab[25 + K * 5 + l] * fac3;
     }
-    const realw dx = t1 * xix + t2 * etx + t3 * gax;
-    const realw dy = t1 * xiy + t2 * ety + t3 * gay;
-    const realw dz = t1 * xiz + t2 * etz + t3 * gaz;
-    realw f1, f2, f3;
-    if (A.is_sph) {
-      const realw rd = rx * dx + ry * dy + rz * dz;
-      f1 = ((cv - ch) * (rx * xix + ry * xiy + rz * xiz) * rd + ch * (xix * dx + xiy * dy + xiz * dz)) * jl;
-      f2 = ((cv - ch) * (rx * etx + ry * ety + rz * etz) * rd + ch * (etx * dx + ety * dy + etz * dz)) * jl;
-      f3 = ((cv - ch) * (rx * gax + ry * gay + rz * gaz) * rd + ch * (gax * dx + gay * dy + gaz * dz)) * jl;
-    } else {
-      f1 = ((cv - ch) * xiz * dz + ch * (xix * dx + xiy * dy + xiz * dz)) * jl;
-      f2 = ((cv - ch) * etz * dz + ch * (etx * dx + ety * dy + etz * dz)) * jl;
-      f3 = ((cv - ch) * gaz * dz + ch * (gax * dx + gay * dy + gaz * dz)) * jl;
-    }
-    if (act) { s_t[0][t] = f1; s_t[1][t] = f2; s_t[2][t] = f3; }
-    __syncthreads();  // fluxes complete; every lane is done reading s_u[f]
-    realw n1 = 0, n2 = 0, n3 = 0;
-#pragma unroll
-    for (int l = 0; l < 5; ++l) {
-      n1 += s_t[0][l + 5 * J + 25 * K] * hwI[l];
-      n2 += s_t[1][I + 5 * l + 25 * K] * hwJ[l];
-      n3 += s_t[2][I + 5 * J + 25 * l] * hwK[l];
-    }
-    if (act) s_u[f][t] = -(fac1 * n1 + fac2 * n2 + fac3 * n3);  // own slot only
-    __syncthreads();  // s_t free for the next field
   }
-  if (act) {
-    realw* O = A.dloc + Lg * NFP;
-    if constexpr (NFP % 4 == 0) {
+  // The fluxes are f_a = sum_b M[a][b] t_b with M = J (ch g_a . g_b + (cv - ch) (g_a . r)(g_b . r)),
+  // g_a the gradient of reference coordinate a and r the vertical (z, or rot when spherical)
+  realw M[3][3] = {};
+  if constexpr (REG) {
+    M[0][0] = M[1][1] = A.cxh * jl;
+    M[2][2] = A.cxv * jl;
+  } else {
+    const realw cv = A.cv, ch = A.ch;
+    realw v[3];
 #pragma unroll
-      for (int k = 0; k < NFP / 4; ++k)
-        reinterpret_cast<float4*>(O)[k] = make_float4(s_u[4 * k][t], s_u[4 * k + 1][t], s_u[4 * k + 2][t], s_u[4 * k + 3][t]);
+    for (int a = 0; a < 3; ++a) v[a] = r[0] * g[a][0] + r[1] * g[a][1] + r[2] * g[a][2];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b)
+        M[a][b] = jl * (ch * (g[a][0] * g[b][0] + g[a][1] * g[b][1] + g[a][2] * g[b][2]) + (cv - ch) * v[a] * v[b]);
+  }
+  const int La0 = 5 * J + 25 * K, Lb0 = I + 25 * K, Lc0 = I + 5 * J;
+  if constexpr (W == 4) __syncthreads();
+  T* dloc = reinterpret_cast<T*>(A.dloc);
+#pragma unroll 1
+  for (int c = 0; c < C; ++c) {
+    T* U = s_u + c * SU;
+    T t1 = P::zero(), t2 = P::zero(), t3 = P::zero();
+#pragma unroll
+    for (int l = 0; l < 5; ++l) {
+      t1 = P::fma_s(U[La0 + l], hpI[l], t1);
+      t2 = P::fma_s(U[Lb0 + 5 * l], hpJ[l], t2);
+      t3 = P::fma_s(U[Lc0 + 25 * l], hpK[l], t3);
+    }
+    if constexpr (REG) {
+      s_t[0][t] = P::mul_s(t1, M[0][0]);
+      s_t[1][t] = P::mul_s(t2, M[1][1]);
+      s_t[2][t] = P::mul_s(t3, M[2][2]);
     } else {
 #pragma unroll
-      for (int k = 0; k < NFP; ++k) O[k] = s_u[k][t];
+      for (int a = 0; a < 3; ++a)
+        s_t[a][t] = P::fma_s(t3, M[a][2], P::fma_s(t2, M[a][1], P::mul_s(t1, M[a][0])));
+    }
+    __syncthreads();  // fluxes complete; every lane is done reading this piece of s_u
+    T d = P::zero();
+#pragma unroll
+    for (int l = 0; l < 5; ++l) {
+      d = P::fma_s(s_t[0][La0 + l], hwI[l], d);
+      d = P::fma_s(s_t[1][Lb0 + 5 * l], hwJ[l], d);
+      d = P::fma_s(s_t[2][Lc0 + 25 * l], hwK[l], d);
+    }
+    if constexpr (W == 1) {
+      if (t < 125) {
+        if (own >= A.n_shared) dat[(size_t)own * C + c] = P::fma_s(d, A.rvol[own], U[t]);
+        else dloc[(L0 + sem_floc_slot(t)) * C + c] = d;
+      }
+      if (c + 1 < C) __syncthreads();  // s_t free for the next value
+    } else {
+      if (t < 125) U[t] = d;  // own slot only
+      __syncthreads();        // s_t free for the next piece; the terms are in s_u
+    }
+  }
+  if constexpr (W == 1) return;
+  for (int q = t; q < 125 * C; q += 128) {
+    const int row = q / C, c = q - row * C;
+    const int p = s_row[row], ig = s_g[p];
+    const T v = s_u[c * SU + p];
+    if (ig >= A.n_shared) {
+      T* D = dat + (size_t)ig * C + c;
+      *D = P::fma_s(v, A.rvol[ig], *D);
+    } else {
+      dloc[(L0 + row) * C + c] = v;
     }
   }
 }
 
-// ddat(g) = sum of the element-local terms of g in element order (the
-// reference CPU loop's accumulation order); dat += rvol * ddat.  One lane per
-// point carrying all NFP fields: each contribution is one contiguous
-// NFP-float row (16-byte vectors), and the dat update is a contiguous
-// read-modify-write of the point's row.
+// ddat(g) = sum of the element-local terms of g in element order (the reference CPU loop's
+// accumulation order); dat += rvol * ddat, for the points of more than one element.  One lane per
+// piece of a point's row, so consecutive lanes read and write whole rows (32x32x16 cubes, 21
+// fields: 94 us a step with a lane per row over all points; bound by the rows' traffic).
 template <int NFP>
-__global__ void k_smooth_gather(int nglob, const int* __restrict__ off, const int* __restrict__ idx,
+__global__ void k_smooth_gather(int npts, const int* __restrict__ off, const int* __restrict__ idx,
                                 const realw* __restrict__ dloc, const realw* __restrict__ rvol,
                                 realw* __restrict__ dat) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= nglob) return;
-  realw d[NFP];
-#pragma unroll
-  for (int f = 0; f < NFP; ++f) d[f] = 0.0f;
+  constexpr int W = SmoothRow<NFP>::W, C = SmoothRow<NFP>::C;
+  const size_t h = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (h >= (size_t)npts * C) return;
+  const int g = (int)(h / C), c = (int)(h - (size_t)g * C);
   const int k1 = off[g + 1];
-  for (int k = off[g]; k < k1; ++k) {
-    const realw* P = dloc + (size_t)idx[k] * NFP;
-    if constexpr (NFP % 4 == 0) {
-#pragma unroll
-      for (int q = 0; q < NFP / 4; ++q) {
-        const float4 v = reinterpret_cast<const float4*>(P)[q];
-        d[4 * q] += v.x; d[4 * q + 1] += v.y; d[4 * q + 2] += v.z; d[4 * q + 3] += v.w;
-      }
-    } else {
-#pragma unroll
-      for (int f = 0; f < NFP; ++f) d[f] += P[f];
-    }
-  }
   const realw r = rvol[g];
-  realw* D = dat + (size_t)g * NFP;
-  if constexpr (NFP % 4 == 0) {
-#pragma unroll
-    for (int q = 0; q < NFP / 4; ++q) {
-      float4 v = reinterpret_cast<const float4*>(D)[q];
-      v.x += r * d[4 * q]; v.y += r * d[4 * q + 1]; v.z += r * d[4 * q + 2]; v.w += r * d[4 * q + 3];
-      reinterpret_cast<float4*>(D)[q] = v;
+  if constexpr (W == 4) {
+    const float4* P = reinterpret_cast<const float4*>(dloc) + c;
+    float4* D = reinterpret_cast<float4*>(dat) + h;
+    const float4 v = *D;
+    float4 d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int k = off[g];
+    for (; k + 1 < k1; k += 2) {  // both rows requested before either is added
+      const float4 a = P[(size_t)idx[k] * C], b = P[(size_t)idx[k + 1] * C];
+      d.x += a.x; d.y += a.y; d.z += a.z; d.w += a.w;
+      d.x += b.x; d.y += b.y; d.z += b.z; d.w += b.w;
     }
+    if (k < k1) {
+      const float4 a = P[(size_t)idx[k] * C];
+      d.x += a.x; d.y += a.y; d.z += a.z; d.w += a.w;
+    }
+    *D = make_float4(fmaf(r, d.x, v.x), fmaf(r, d.y, v.y), fmaf(r, d.z, v.z), fmaf(r, d.w, v.w));
   } else {
-#pragma unroll
-    for (int f = 0; f < NFP; ++f) D[f] += r * d[f];
+    const realw v = dat[h];
+    realw d = 0.0f;
+    for (int k = off[g]; k < k1; ++k) d += dloc[(size_t)idx[k] * C + c];
+    dat[h] = fmaf(r, d, v);
   }
 }
 
@@ -216,19 +279,22 @@ __global__ void k_keep_pml(int npml, int nfield, int nfp, const int* __restrict_
   for (int f = 0; f < nfield; ++f) dat[(size_t)pml_iglob[q] * nfp + f] = pml_val[(size_t)f * npml + q];
 }
 
-// [nfield][nglob] <-> [nglob][nfp]
-__global__ void k_to_point_major(int nglob, int nfield, int nfp, const realw* __restrict__ a, realw* __restrict__ b) {
-  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (size_t)nglob * nfp) return;
-  const int g = (int)(q / nfp), f = (int)(q % nfp);
-  b[q] = f < nfield ? a[(size_t)f * nglob + g] : 0.0f;
+// [nfield][nglob] <-> [nglob][nfp], the rows in library numbering; a lane per point, so that the
+// caller's side is contiguous over the lanes
+__global__ void k_to_point_major(int nglob, int nfield, int nfp, const int* __restrict__ perm,
+                                 const realw* __restrict__ a, realw* __restrict__ b) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= nglob) return;
+  realw* B = b + (size_t)perm[g] * nfp;
+  for (int f = 0; f < nfp; ++f) B[f] = f < nfield ? a[(size_t)f * nglob + g] : 0.0f;
 }
 
-__global__ void k_to_field_major(int nglob, int nfield, int nfp, const realw* __restrict__ b, realw* __restrict__ a) {
-  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (size_t)nglob * nfield) return;
-  const int f = (int)(q / nglob), g = (int)(q % nglob);
-  a[q] = b[(size_t)g * nfp + f];
+__global__ void k_to_field_major(int nglob, int nfield, int nfp, const int* __restrict__ perm,
+                                 const realw* __restrict__ b, realw* __restrict__ a) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= nglob) return;
+  const realw* B = b + (size_t)perm[g] * nfp;
+  for (int f = 0; f < nfield; ++f) a[(size_t)f * nglob + g] = B[f];
 }
 
 int g_smooth_faithful = 1;
@@ -239,6 +305,8 @@ int padded_fields(int nf) { return nf <= 3 ? nf : ((nf + 3) / 4) * 4; }
 
 struct SmoothPlan {
   int nspec = 0, nglob = 0, nirr = 0, npml = 0, nfield = 0, nfp = 1;
+  int n_shared = 0;         // points of more than one element come first, in the caller's order
+  int* d_perm = nullptr;    // caller's point -> library point
   int* d_ibool = nullptr;
   int* d_irr = nullptr;
   realw* d_jinv9 = nullptr;
@@ -260,7 +328,7 @@ struct SmoothPlan {
 void plan_free(SmoothPlan& p) {
   dev_free(p.d_ibool); dev_free(p.d_irr); dev_free(p.d_jinv9); dev_free(p.d_jac); dev_free(p.d_rot);
   dev_free(p.d_tables); dev_free(p.d_rvol); dev_free(p.d_off); dev_free(p.d_idx); dev_free(p.d_dat);
-  dev_free(p.d_dloc); dev_free(p.d_io); dev_free(p.d_pml_iglob); dev_free(p.d_pml_val);
+  dev_free(p.d_dloc); dev_free(p.d_io); dev_free(p.d_pml_iglob); dev_free(p.d_pml_val); dev_free(p.d_perm);
   if (p.stream) HIP_CHECK(hipStreamDestroy(p.stream));
   p = SmoothPlan();
 }
@@ -268,7 +336,7 @@ void plan_free(SmoothPlan& p) {
 // elem_ms / update_ms of a timed run: the element and gather launches of every
 // stride-th step (at most about 256 steps) timed by their dispatch timestamps,
 // scaled to all nstep steps
-template <int NFP>
+template <int NFP, bool REG>
 void launch_steps(SmoothPlan& p, const SmoothArgs& a, int nstep, bool timed) {
   const int stride = std::max(1, nstep / 256), nsamp = (nstep + stride - 1) / stride;
   std::vector<hipEvent_t> ev;
@@ -280,10 +348,10 @@ void launch_steps(SmoothPlan& p, const SmoothArgs& a, int nstep, bool timed) {
     const bool tm = timed && it % stride == 0;
     const size_t q = 4 * (size_t)(it / stride);
     if (tm) sem_arm_launch_events(ev[q], ev[q + 1]);
-    SEM_LAUNCH(k_smooth_elem<NFP>, dim3(a.nblocks_padded), dim3(128), 0, p.stream, a);
+    SEM_LAUNCH((k_smooth_elem<NFP, REG>), dim3(a.nblocks_padded), dim3(128), 0, p.stream, a);
     if (tm) sem_arm_launch_events(ev[q + 2], ev[q + 3]);
-    SEM_LAUNCH(k_smooth_gather<NFP>, dim3(sm_blocks((size_t)p.nglob)), dim3(SM_TPB), 0, p.stream, p.nglob,
-               p.d_off, p.d_idx, p.d_dloc, p.d_rvol, p.d_dat);
+    SEM_LAUNCH(k_smooth_gather<NFP>, dim3(std::max(1u, sm_blocks((size_t)p.n_shared * SmoothRow<NFP>::C))), dim3(SM_TPB),
+               0, p.stream, p.n_shared, p.d_off, p.d_idx, p.d_dloc, p.d_rvol, p.d_dat);
     if (p.npml > 0)
       hipLaunchKernelGGL(k_keep_pml, dim3((p.npml + SM_TPB - 1) / SM_TPB), dim3(SM_TPB), 0, p.stream, p.npml,
                          p.nfield, p.nfp, p.d_pml_iglob, p.d_pml_val, p.d_dat);
@@ -305,26 +373,37 @@ void launch_steps(SmoothPlan& p, const SmoothArgs& a, int nstep, bool timed) {
   }
 }
 
+template <bool REG>
+void launch_fields(SmoothPlan& p, const SmoothArgs& a, int nstep, bool timed) {
+  switch (p.nfp) {
+    case 1: launch_steps<1, REG>(p, a, nstep, timed); break;
+    case 2: launch_steps<2, REG>(p, a, nstep, timed); break;
+    case 3: launch_steps<3, REG>(p, a, nstep, timed); break;
+    case 4: launch_steps<4, REG>(p, a, nstep, timed); break;
+    case 8: launch_steps<8, REG>(p, a, nstep, timed); break;
+    case 12: launch_steps<12, REG>(p, a, nstep, timed); break;
+    case 16: launch_steps<16, REG>(p, a, nstep, timed); break;
+    case 20: launch_steps<20, REG>(p, a, nstep, timed); break;
+    case 24: launch_steps<24, REG>(p, a, nstep, timed); break;
+    default: SEM_FAIL("smooth: %d padded fields not supported", p.nfp);
+  }
+}
+
 void run_steps(SmoothPlan& p, int nstep, realw cv, realw ch, realw xix_regular, int is_sph, bool timed) {
   SmoothArgs a{};
-  a.ibool = p.d_ibool; a.irregular = p.d_irr; a.jinv9 = p.d_jinv9; a.jac = p.d_jac; a.rot = p.d_rot;
-  a.tables = p.d_tables; a.dat = p.d_dat; a.dloc = p.d_dloc;
+  a.ibool = p.d_ibool; a.irregular = p.d_irr; a.jinv9 = p.d_jinv9; a.jstride = (size_t)p.nirr * 125; a.jac = p.d_jac; a.rot = p.d_rot;
+  a.tables = p.d_tables; a.rvol = p.d_rvol; a.dat = p.d_dat; a.dloc = p.d_dloc;
+  a.n_shared = p.n_shared;
+  a.cxh = (realw)((double)ch * xix_regular * xix_regular);
+  a.cxv = (realw)((double)cv * xix_regular * xix_regular);
   a.nspec = p.nspec; a.nfield = p.nfield;
   a.nblocks_padded = xcd_pad(p.nspec);
   a.cv = cv; a.ch = ch; a.xix_regular = xix_regular; a.is_sph = is_sph; a.faithful = g_smooth_faithful;
   p.elem_ms = p.update_ms = 0;
-  switch (p.nfp) {
-    case 1: launch_steps<1>(p, a, nstep, timed); break;
-    case 2: launch_steps<2>(p, a, nstep, timed); break;
-    case 3: launch_steps<3>(p, a, nstep, timed); break;
-    case 4: launch_steps<4>(p, a, nstep, timed); break;
-    case 8: launch_steps<8>(p, a, nstep, timed); break;
-    case 12: launch_steps<12>(p, a, nstep, timed); break;
-    case 16: launch_steps<16>(p, a, nstep, timed); break;
-    case 20: launch_steps<20>(p, a, nstep, timed); break;
-    case 24: launch_steps<24>(p, a, nstep, timed); break;
-    default: SEM_FAIL("smooth: %d padded fields not supported", p.nfp);
-  }
+  // cubes with the diagonal map everywhere: one flux factor per direction (faithful mode and
+  // irregular or spherical meshes need the whole map)
+  if (p.nirr == 0 && !g_smooth_faithful && !is_sph) launch_fields<true>(p, a, nstep, timed);
+  else launch_fields<false>(p, a, nstep, timed);
 }
 
 // Build the device plan from the reference's host arrays.
@@ -343,27 +422,48 @@ void plan_build(SmoothPlan& p, int nspec, int nglob, int nirr, int is_sph, const
     if (g < 0 || g >= nglob) SEM_FAIL("smooth_pde: ibool(%zu)=%d outside 1..%d", L, g + 1, nglob);
     ib[L] = g;
   }
+  // library numbering: points of more than one element first, in the caller's order, then the
+  // others element by element
+  std::vector<uint8_t> touch(nglob, 0);
+  for (size_t L = 0; L < nloc; ++L) touch[ib[L]] = (uint8_t)std::min(2, touch[ib[L]] + 1);
+  std::vector<int> perm(nglob, -1);
+  int n = 0;
+  for (int g = 0; g < nglob; ++g)
+    if (touch[g] != 1) perm[g] = n++;
+  p.n_shared = n;
+  for (size_t L = 0; L < nloc; ++L)
+    if (touch[ib[L]] == 1) perm[ib[L]] = n++;
+  for (size_t L = 0; L < nloc; ++L) ib[L] = perm[ib[L]];
+  p.d_perm = dev_upload(perm.data(), perm.size(), s);
   p.d_ibool = dev_upload(ib.data(), nloc, s);
-  // CSR point -> local points in increasing local index (element order)
+  // CSR shared point -> element rows in element order, by their place in the rows
   if (nloc >= (size_t)INT32_MAX) SEM_FAIL("smooth: too many local points for 32-bit CSR indices");
   {
-    std::vector<int> off((size_t)nglob + 1, 0), idx(nloc);
-    for (size_t L = 0; L < nloc; ++L) off[(size_t)ib[L] + 1]++;
-    for (int g = 0; g < nglob; ++g) off[g + 1] += off[g];
-    std::vector<int> fill(off.begin(), off.end() - 1);
-    for (size_t L = 0; L < nloc; ++L) idx[fill[ib[L]]++] = (int)L;
+    int slot[125];
+    for (int L = 0; L < 125; ++L) slot[L] = sem_floc_slot(L);
+    std::vector<int> off((size_t)p.n_shared + 1, 0);
+    for (size_t L = 0; L < nloc; ++L)
+      if (ib[L] < p.n_shared) off[(size_t)ib[L] + 1]++;
+    for (int g = 0; g < p.n_shared; ++g) off[g + 1] += off[g];
+    std::vector<int> fill(off.begin(), off.end() - 1), idx((size_t)off[p.n_shared]);
+    for (int e = 0; e < nspec; ++e)
+      for (int L = 0; L < 125; ++L) {
+        const int g = ib[(size_t)e * 125 + L];
+        if (g < p.n_shared) idx[fill[g]++] = e * 125 + slot[L];
+      }
     p.d_off = dev_upload(off.data(), off.size(), s);
     p.d_idx = dev_upload(idx.data(), idx.size(), s);
+    HIP_CHECK(hipStreamSynchronize(s));
   }
   std::vector<int> irr(irregular, irregular + nspec);
   for (int e = 0; e < nspec; ++e)
     if (irr[e] < 0 || irr[e] > nirr) SEM_FAIL("smooth_pde: irregular_element_number(%d)=%d outside 0..%d", e + 1, irr[e], nirr);
   p.d_irr = dev_upload(irr.data(), (size_t)nspec, s);
   if (nirr > 0) {
-    std::vector<realw> j9((size_t)nirr * 1125);
-    for (size_t e = 0; e < (size_t)nirr; ++e)
-      for (int c = 0; c < 9; ++c) std::memcpy(&j9[(e * 9 + c) * 125], &jin[c][e * 125], 125 * sizeof(realw));
-    p.d_jinv9 = dev_upload(j9.data(), j9.size(), s);
+    const size_t nj = (size_t)nirr * 125;
+    p.d_jinv9 = dev_alloc<realw>(9 * nj);
+    for (int c = 0; c < 9; ++c)
+      HIP_CHECK(hipMemcpyAsync(p.d_jinv9 + c * nj, jin[c], nj * sizeof(realw), hipMemcpyHostToDevice, s));
   }
   p.d_jac = dev_upload(jaco, nloc, s);
   if (is_sph) {
@@ -383,20 +483,22 @@ void plan_build(SmoothPlan& p, int nspec, int nglob, int nirr, int is_sph, const
     tab[100 + q] = wxy[q];
   }
   p.d_tables = dev_upload(tab, 125, s);
-  p.d_rvol = dev_upload(rvol, (size_t)nglob, s);
+  std::vector<realw> rv(nglob);
+  for (int g = 0; g < nglob; ++g) rv[perm[g]] = rvol[g];
+  p.d_rvol = dev_upload(rv.data(), (size_t)nglob, s);
   p.d_dat = dev_alloc<realw>((size_t)nglob * p.nfp);
   p.d_dloc = dev_alloc<realw>(nloc * p.nfp);
   p.d_io = dev_alloc<realw>((size_t)nglob * nfield);
   // PML points in element order (last writer of a shared point wins, as the
   // reference's sequential CPU loop)
-  std::vector<int> piglob;
+  std::vector<int> piglob;  // in the caller's point order, as smooth_pde_cuda_ lists the values
   if (is_CPML) {
     std::vector<int> last(nglob, -1);
     for (int e = 0; e < nspec; ++e)
       if (is_CPML[e])
         for (int L = 0; L < 125; ++L) last[ib[(size_t)e * 125 + L]] = e * 125 + L;
     for (int g = 0; g < nglob; ++g)
-      if (last[g] >= 0) piglob.push_back(g);
+      if (last[perm[g]] >= 0) piglob.push_back(perm[g]);
   }
   p.npml = (int)piglob.size();
   if (p.npml) {
@@ -411,18 +513,17 @@ void plan_build(SmoothPlan& p, int nspec, int nglob, int nirr, int is_sph, const
 void upload_fields(SmoothPlan& p, const realw* dat_glob) {
   const size_t n = (size_t)p.nglob * p.nfield;
   HIP_CHECK(hipMemcpyAsync(p.d_io, dat_glob, n * sizeof(realw), hipMemcpyHostToDevice, p.stream));
-  hipLaunchKernelGGL(k_to_point_major, dim3(sm_blocks((size_t)p.nglob * p.nfp)), dim3(SM_TPB), 0, p.stream, p.nglob,
-                     p.nfield, p.nfp, p.d_io, p.d_dat);
+  hipLaunchKernelGGL(k_to_point_major, dim3(sm_blocks((size_t)p.nglob)), dim3(SM_TPB), 0, p.stream, p.nglob, p.nfield,
+                     p.nfp, p.d_perm, p.d_io, p.d_dat);
   HIP_CHECK(hipGetLastError());
 }
 
 void download_fields(SmoothPlan& p, realw* dat_glob) {
   const size_t n = (size_t)p.nglob * p.nfield;
-  hipLaunchKernelGGL(k_to_field_major, dim3(sm_blocks(n)), dim3(SM_TPB), 0, p.stream, p.nglob, p.nfield, p.nfp,
-                     p.d_dat, p.d_io);
+  hipLaunchKernelGGL(k_to_field_major, dim3(sm_blocks((size_t)p.nglob)), dim3(SM_TPB), 0, p.stream, p.nglob, p.nfield,
+                     p.nfp, p.d_perm, p.d_dat, p.d_io);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(dat_glob, p.d_io, n * sizeof(realw), hipMemcpyDeviceToHost, p.stream));
-  HIP_CHECK(hipStreamSynchronize(p.stream));
+  sem_to_host(dat_glob, p.d_io, n * sizeof(realw), p.stream);
 }
 
 double g_last_elem_ms = 0.0, g_last_update_ms = 0.0;

@@ -111,6 +111,23 @@ def test_many_receivers_in_one_element(nrec):
     a.close()
 
 
+@pytest.mark.parametrize("mesh,perturb,nfield", [((1, 1, 1), 0.0, 4), ((3, 1, 2), 0.0, 1), ((3, 2, 2), 0.1, 6),
+                                                 ((5, 3, 2), 0.0, 21), ((5, 3, 2), 0.1, 24), ((3, 3, 3), 0.0, 25)])
+def test_smoothing_of_any_number_of_fields(mesh, perturb, nfield):
+    """Diffusion steps of 1 to 25 fields (whole and ragged groups of four, rows of one value and of
+    16-byte pieces, a second run for the 25th) on cubes and deformed elements, down to one element,
+    all of whose points the element pass finishes; against the loop restatement field by field."""
+    from specfwat_amd.smooth import smooth_batch
+    print(f"smoothing {nfield} fields on {mesh}, perturb {perturb}", flush=True)
+    m = BoxMesh(*mesh, *(1000.0 * v for v in mesh), perturb=perturb)
+    rng = np.random.default_rng(nfield)
+    fields = rng.standard_normal((nfield, m.nspec, 125)).astype(np.float32)
+    out = smooth_batch(m, fields, 800.0, 400.0, faithful=False)[0]
+    for q in {0, nfield // 2, nfield - 1}:
+        _, ref, _ = orc.smooth_pde(m.smooth_arrays(), fields[q].ravel(), 800.0, 400.0, m.distance_min_glob(), faithful=False)
+        assert rel(out[q], ref) < 1e-5, q  # 32-bit steps, the bar of the other smoothing tests
+
+
 @pytest.mark.parametrize("nrec", [341, 342, 347, 683])
 def test_large_results_arrive_whole(nrec):
     """Adjoint sources of 4,096 samples, 48 KiB a receiver: from 16 MiB on results are copied in
