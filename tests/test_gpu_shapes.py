@@ -141,3 +141,19 @@ def test_large_results_arrive_whole(nrec):
     large = misfit.event_adjoint_sources(obs[:, q], syn[:, q], dt, [[1.0, 200.0]])[1]
     assert np.abs(small).max() > 0
     np.testing.assert_array_equal(large, small[:, q])
+
+
+@pytest.mark.parametrize("nstep", [31, 32, 33, 63, 64, 65, 97, 129])
+def test_adjoint_filter_at_block_edges(nstep):
+    """The bandpass walks blocks of 32 samples, the next one loaded ahead, its second section one
+    sample behind: series that end at, before and after a block; against the oracle trace by trace."""
+    dt = 0.05
+    rng = np.random.default_rng(nstep)
+    obs, syn = (rng.standard_normal((nstep, 11, 3)).astype(np.float32) for _ in range(2))
+    win = [[0.0, nstep * dt]]
+    _, adj = misfit.event_adjoint_sources(obs, syn, dt, win, min_period=0.4, max_period=12.0)
+    for r in range(11):
+        for c in range(3):
+            _, a, _, _ = orc.waveform_adjoint(obs[:, r, c], syn[:, r, c], dt, win)
+            a = orc.filter_adj(a, dt, np.float32(1 / 12.0), np.float32(1 / 0.4), win)
+            assert np.abs(adj[:, r, c] - a).max() <= 1e-6 * np.abs(a).max(), (r, c)  # single precision, as its other tests
