@@ -375,8 +375,7 @@ void k_batch_elem(BatchElemArgs A) {
             const realw prod = (ea0 - t3a) * (eb0 - t3b) + (ea1 - t3a) * (eb1 - t3b) + (ea2 - t3a) * (eb2 - t3b) +
                                2.0f * (ea3 * eb3 + ea4 * eb4 + ea5 * eb5);
             const size_t kq = (size_t)ev * nloc + Lg;
-            kernel_acc(A.mu_kl, A.mu_part, kq, prod, A.dt, A.kflush != 0);
-            kernel_acc(A.kappa_kl, A.kappa_part, kq, tra * trb, A.dt, A.kflush != 0);
+            kernel_acc_pair(A.mu_kl, A.mu_part, prod, A.kappa_kl, A.kappa_part, tra * trb, kq, A.dt, A.kflush != 0);
           }
         }
         const realw ltr = lam * (duxdx + duydy + duzdz);
@@ -512,16 +511,17 @@ __global__ __launch_bounds__(128) void k_batch_elem_aniso(BatchElemArgs A) {
           } else if (act) {
             const realw vb[6] = {e1, e2, e3, 2.0f * (0.5f * e4), 2.0f * (0.5f * e5), 2.0f * (0.5f * e6)};
             const size_t k0 = (size_t)ev * nloc21 + (size_t)e * 21 * 125 + t;
+            realw pr[21];
             int q = 0;
 #pragma unroll
             for (int P = 0; P < 6; ++P)
 #pragma unroll
               for (int Q = P; Q < 6; ++Q) {
-                realw pr = va[P] * vb[Q];
-                if (Q > P) pr += va[Q] * vb[P];
-                kernel_acc(A.cijkl_kl, A.cij_part, k0 + (size_t)q * 125, pr, A.dt, A.kflush != 0);
+                pr[q] = va[P] * vb[Q];
+                if (Q > P) pr[q] += va[Q] * vb[P];
                 ++q;
               }
+            kernel_acc_n<21>(A.cijkl_kl, A.cij_part, k0, 125, pr, A.dt, A.kflush != 0);
           }
         }
         asm volatile("" ::: "memory");

@@ -229,22 +229,22 @@ __global__ __launch_bounds__(128) void k_forces(ForceArgs A) {
           const realw prod = (ea[0] - t3a) * (eb0 - t3b) + (ea[1] - t3a) * (eb1 - t3b) +
                              (ea[2] - t3a) * (eb2 - t3b) +
                              2.0f * (ea[3] * eb3 + ea[4] * eb4 + ea[5] * eb5);
-          kernel_acc(A.mu_kl, A.mu_part, Lg, prod, A.dt, A.kflush != 0);
-          kernel_acc(A.kappa_kl, A.kappa_part, Lg, tra * trb, A.dt, A.kflush != 0);
+          kernel_acc_pair(A.mu_kl, A.mu_part, prod, A.kappa_kl, A.kappa_part, tra * trb, Lg, A.dt, A.kflush != 0);
         } else {
           const realw va[6] = {ea[0], ea[1], ea[2], 2.0f * ea[5], 2.0f * ea[4], 2.0f * ea[3]};
           const realw vb[6] = {eb0, eb1, eb2, 2.0f * eb5, 2.0f * eb4, 2.0f * eb3};
           const size_t k0 = (size_t)ispec * 21 * 125 + t;
+          realw pr[21];
           int q = 0;
 #pragma unroll
           for (int P = 0; P < 6; ++P)
 #pragma unroll
             for (int Q = P; Q < 6; ++Q) {
-              realw pr = va[P] * vb[Q];
-              if (Q > P) pr += va[Q] * vb[P];
-              kernel_acc(A.cijkl_kl, A.cij_part, k0 + (size_t)q * 125, pr, A.dt, A.kflush != 0);
+              pr[q] = va[P] * vb[Q];
+              if (Q > P) pr[q] += va[Q] * vb[P];
               ++q;
             }
+          kernel_acc_n<21>(A.cijkl_kl, A.cij_part, k0, 125, pr, A.dt, A.kflush != 0);
         }
       }
     }
@@ -322,16 +322,20 @@ __global__ __launch_bounds__(128) void k_forces(ForceArgs A) {
 //     wgllwgll(..) of the output point, and LDS holds the six stress
 //     components only (the flux of direction d is row d of sigma);
 //   * the three directions accumulate into one register per component.
+// Both fields of an adjoint step share the two barriers of an element: their points are requested
+// together and the moduli or c_ij read once.  24x24x12 with 21 c_ij and their kernels: 65 us field
+// after field, 54 with the kernels' partial sums requested together (kernel_acc_n), 47 so; 305 B a
+// point at 5.6 TB/s, near the memory's rate.
 // Workgroups are persistent: each loops over its share of an XCD-contiguous
 // run of elements, so the table set-up is paid once per workgroup.
 template <int NF, bool ANISO, int KMODE, int SP>
 __device__ __forceinline__ void forces_reg_body(const ForceArgs& A) {
   __shared__ realw s_tab[128];
-  __shared__ realw s_u[3][128];
-  __shared__ realw s_s[6][128];
+  __shared__ realw s_u[NF][3][128];
+  __shared__ realw s_s[NF][6][128];
   const int t = threadIdx.x;
   if (NF == 1 && (int)blockIdx.x >= A.nblk) {  // block-uniform
-    sem_seismo_block(A.se, blockIdx.x - A.nblk, &s_u[0][0]);
+    sem_seismo_block(A.se, blockIdx.x - A.nblk, &s_u[0][0][0]);
     return;
   }
   if (t < 125) s_tab[t] = A.tables[t];
@@ -382,75 +386,74 @@ __device__ __forceinline__ void forces_reg_body(const ForceArgs& A) {
     } else {
       C = A.cij + (size_t)e * 21 * 125 + tt;
     }
-    realw ea[6];
+    realw st[NF][6];  // strains of the fields: xx yy zz 2xy 2xz 2yz
+    if (act) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const realw* U = (f == 0 ? A.u0 : A.u1) + 3 * (size_t)iglob;
+        s_u[f][0][t] = U[0];
+        s_u[f][1][t] = U[1];
+        s_u[f][2][t] = U[2];
+      }
+    }
+    __syncthreads();
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      const realw* U = f == 0 ? A.u0 : A.u1;
-      realw* Floc = f == 0 ? A.floc0 : A.floc1;
-      __syncthreads();  // previous element / field done with s_u and s_s
-      if (act) {
-        s_u[0][t] = U[3 * (size_t)iglob];
-        s_u[1][t] = U[3 * (size_t)iglob + 1];
-        s_u[2][t] = U[3 * (size_t)iglob + 2];
-      }
-      __syncthreads();
       realw duxdx = 0, duydx = 0, duzdx = 0, duxdy = 0, duydy = 0, duzdy = 0, duxdz = 0, duydz = 0, duzdz = 0;
 #pragma unroll
       for (int l = 0; l < 5; ++l) {
         const int La = La0 + l, Lb = Lb0 + 5 * l, Lc = Lc0 + 25 * l;
-        duxdx += s_u[0][La] * hpI[l]; duydx += s_u[1][La] * hpI[l]; duzdx += s_u[2][La] * hpI[l];
-        duxdy += s_u[0][Lb] * hpJ[l]; duydy += s_u[1][Lb] * hpJ[l]; duzdy += s_u[2][Lb] * hpJ[l];
-        duxdz += s_u[0][Lc] * hpK[l]; duydz += s_u[1][Lc] * hpK[l]; duzdz += s_u[2][Lc] * hpK[l];
+        duxdx += s_u[f][0][La] * hpI[l]; duydx += s_u[f][1][La] * hpI[l]; duzdx += s_u[f][2][La] * hpI[l];
+        duxdy += s_u[f][0][Lb] * hpJ[l]; duydy += s_u[f][1][Lb] * hpJ[l]; duzdy += s_u[f][2][Lb] * hpJ[l];
+        duxdz += s_u[f][0][Lc] * hpK[l]; duydz += s_u[f][1][Lc] * hpK[l]; duzdz += s_u[f][2][Lc] * hpK[l];
       }
-      const realw exy2 = duxdy + duydx, exz2 = duzdx + duxdz, eyz2 = duzdy + duydz;
-      if (KMODE == 2) {
-        if (f == 0) {
-          ea[0] = duxdx; ea[1] = duydy; ea[2] = duzdz;
-          ea[3] = 0.5f * exy2; ea[4] = 0.5f * exz2; ea[5] = 0.5f * eyz2;
-        } else if (act) {
-          const realw eb0 = duxdx, eb1 = duydy, eb2 = duzdz;
-          const realw eb3 = 0.5f * exy2, eb4 = 0.5f * exz2, eb5 = 0.5f * eyz2;
-          if (!ANISO) {
-            const realw tra = ea[0] + ea[1] + ea[2], trb = eb0 + eb1 + eb2;
-            const realw t3a = tra / 3.0f, t3b = trb / 3.0f;
-            const realw prod = (ea[0] - t3a) * (eb0 - t3b) + (ea[1] - t3a) * (eb1 - t3b) +
-                               (ea[2] - t3a) * (eb2 - t3b) +
-                               2.0f * (ea[3] * eb3 + ea[4] * eb4 + ea[5] * eb5);
-            kernel_acc(A.mu_kl, A.mu_part, Lg, prod, A.dt, A.kflush != 0);
-            kernel_acc(A.kappa_kl, A.kappa_part, Lg, tra * trb, A.dt, A.kflush != 0);
-          } else {
-            const realw va[6] = {ea[0], ea[1], ea[2], 2.0f * ea[5], 2.0f * ea[4], 2.0f * ea[3]};
-            const realw vb[6] = {eb0, eb1, eb2, 2.0f * eb5, 2.0f * eb4, 2.0f * eb3};
-            const size_t k0 = (size_t)e * 21 * 125 + t;
-            int q = 0;
+      st[f][0] = duxdx; st[f][1] = duydy; st[f][2] = duzdz;
+      st[f][3] = duxdy + duydx; st[f][4] = duzdx + duxdz; st[f][5] = duzdy + duydz;
+    }
+    if (KMODE == 2 && act) {
+      // strains st[f] = xx yy zz 2xy 2xz 2yz
+      const realw ea3 = 0.5f * st[0][3], ea4 = 0.5f * st[0][4], ea5 = 0.5f * st[0][5];
+      const realw eb3 = 0.5f * st[NF - 1][3], eb4 = 0.5f * st[NF - 1][4], eb5 = 0.5f * st[NF - 1][5];
+      if (!ANISO) {
+        const realw tra = st[0][0] + st[0][1] + st[0][2], trb = st[NF - 1][0] + st[NF - 1][1] + st[NF - 1][2];
+        const realw t3a = tra / 3.0f, t3b = trb / 3.0f;
+        const realw prod = (st[0][0] - t3a) * (st[NF - 1][0] - t3b) + (st[0][1] - t3a) * (st[NF - 1][1] - t3b) +
+                           (st[0][2] - t3a) * (st[NF - 1][2] - t3b) +
+                           2.0f * (ea3 * eb3 + ea4 * eb4 + ea5 * eb5);
+        kernel_acc_pair(A.mu_kl, A.mu_part, prod, A.kappa_kl, A.kappa_part, tra * trb, Lg, A.dt, A.kflush != 0);
+      } else {
+        const realw va[6] = {st[0][0], st[0][1], st[0][2], 2.0f * ea5, 2.0f * ea4, 2.0f * ea3};
+        const realw vb[6] = {st[NF - 1][0], st[NF - 1][1], st[NF - 1][2], 2.0f * eb5, 2.0f * eb4, 2.0f * eb3};
+        const size_t k0 = (size_t)e * 21 * 125 + t;
+        realw pr[21];
+        int q = 0;
 #pragma unroll
-            for (int P = 0; P < 6; ++P)
+        for (int P = 0; P < 6; ++P)
 #pragma unroll
-              for (int Q = P; Q < 6; ++Q) {
-                realw pr = va[P] * vb[Q];
-                if (Q > P) pr += va[Q] * vb[P];
-                kernel_acc(A.cijkl_kl, A.cij_part, k0 + (size_t)q * 125, pr, A.dt, A.kflush != 0);
-                ++q;
-              }
+          for (int Q = P; Q < 6; ++Q) {
+            pr[q] = va[P] * vb[Q];
+            if (Q > P) pr[q] += va[Q] * vb[P];
+            ++q;
           }
-        }
+        kernel_acc_n<21>(A.cijkl_kl, A.cij_part, k0, 125, pr, A.dt, A.kflush != 0);
       }
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const realw e1 = st[f][0], e2 = st[f][1], e3 = st[f][2], e4 = st[f][5], e5 = st[f][4], e6 = st[f][3];
       realw sxx, syy, szz, sxy, sxz, syz;
       if (!ANISO) {
         const realw lam = kl - (2.0f / 3.0f) * ml;
         const realw m2 = 2.0f * ml;
-        const realw ltr = lam * (duxdx + duydy + duzdz);
-        sxx = ltr + m2 * duxdx;
-        syy = ltr + m2 * duydy;
-        szz = ltr + m2 * duzdz;
-        sxy = ml * exy2;
-        sxz = ml * exz2;
-        syz = ml * eyz2;
+        const realw ltr = lam * (e1 + e2 + e3);
+        sxx = ltr + m2 * e1;
+        syy = ltr + m2 * e2;
+        szz = ltr + m2 * e3;
+        sxy = ml * e6;
+        sxz = ml * e5;
+        syz = ml * e4;
       } else {
-        const realw e1 = duxdx, e2 = duydy, e3 = duzdz, e4 = eyz2, e5 = exz2, e6 = exy2;
-        // load the 21 c_ij here for each field (cache hits the second time) instead of
-        // keeping them live across both fields: 144 -> fewer VGPRs, more waves per SIMD
-        asm volatile("" ::: "memory");
+        // c index (P,Q), P<=Q, upper-triangle row-major: 11 12 13 14 15 16 22 .. 66
         const realw c11 = C[0], c12 = C[125], c13 = C[250], c14 = C[375], c15 = C[500], c16 = C[625];
         const realw c22 = C[750], c23 = C[875], c24 = C[1000], c25 = C[1125], c26 = C[1250];
         const realw c33 = C[1375], c34 = C[1500], c35 = C[1625], c36 = C[1750];
@@ -464,19 +467,23 @@ __device__ __forceinline__ void forces_reg_body(const ForceArgs& A) {
         sxy = c16 * e1 + c26 * e2 + c36 * e3 + c46 * e4 + c56 * e5 + c66 * e6;
       }
       if (act) {
-        s_s[0][t] = sxx; s_s[1][t] = syy; s_s[2][t] = szz;
-        s_s[3][t] = sxy; s_s[4][t] = sxz; s_s[5][t] = syz;
+        s_s[f][0][t] = sxx; s_s[f][1][t] = syy; s_s[f][2][t] = szz;
+        s_s[f][3][t] = sxy; s_s[f][4][t] = sxz; s_s[f][5][t] = syz;
       }
-      __syncthreads();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
       realw fx = 0, fy = 0, fz = 0;
 #pragma unroll
       for (int l = 0; l < 5; ++l) {
         const int La = La0 + l, Lb = Lb0 + 5 * l, Lc = Lc0 + 25 * l;
         // direction x: row x of sigma at (l,J,K); y: row y at (I,l,K); z: row z at (I,J,l)
-        fx += s_s[0][La] * hwI[l]; fy += s_s[3][La] * hwI[l]; fz += s_s[4][La] * hwI[l];
-        fx += s_s[3][Lb] * hwJ[l]; fy += s_s[1][Lb] * hwJ[l]; fz += s_s[5][Lb] * hwJ[l];
-        fx += s_s[4][Lc] * hwK[l]; fy += s_s[5][Lc] * hwK[l]; fz += s_s[2][Lc] * hwK[l];
+        fx += s_s[f][0][La] * hwI[l]; fy += s_s[f][3][La] * hwI[l]; fz += s_s[f][4][La] * hwI[l];
+        fx += s_s[f][3][Lb] * hwJ[l]; fy += s_s[f][1][Lb] * hwJ[l]; fz += s_s[f][5][Lb] * hwJ[l];
+        fx += s_s[f][4][Lc] * hwK[l]; fy += s_s[f][5][Lc] * hwK[l]; fz += s_s[f][2][Lc] * hwK[l];
       }
+      realw* Floc = f == 0 ? A.floc0 : A.floc1;
       if (act) {
         realw* F = Floc + 3 * (Lg - tt + (A.grouped ? sem_floc_slot(tt) : tt));
         F[0] = fx;

@@ -327,6 +327,36 @@ __device__ __forceinline__ void kernel_acc(double* __restrict__ K, float* __rest
   }
 }
 
+// The same for the pair mu, kappa and for N densities whose integrals lie `stride` apart.  One uniform
+// branch around all of them: with the branch inside, each sum is a load, a wait
+// and a store of its own, N latencies one after the other.
+__device__ __forceinline__ void kernel_acc_pair(double* __restrict__ K0, float* __restrict__ part0, float x0,
+                                                double* __restrict__ K1, float* __restrict__ part1, float x1,
+                                                size_t i, double dt, bool flush) {
+  if (part0 && !flush) {
+    const float p0 = part0[i], p1 = part1[i];
+    part0[i] = p0 + x0;
+    part1[i] = p1 + x1;
+  } else {
+    kernel_acc(K0, part0, i, x0, dt, flush);
+    kernel_acc(K1, part1, i, x1, dt, flush);
+  }
+}
+template <int N>
+__device__ __forceinline__ void kernel_acc_n(double* __restrict__ K, float* __restrict__ part, size_t i, int stride,
+                                             const float (&x)[N], double dt, bool flush) {
+  if (part && !flush) {
+    float p[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) p[q] = part[i + (size_t)q * stride];
+#pragma unroll
+    for (int q = 0; q < N; ++q) part[i + (size_t)q * stride] = p[q] + x[q];
+  } else {
+#pragma unroll
+    for (int q = 0; q < N; ++q) kernel_acc(K, part, i + (size_t)q * stride, x[q], dt, flush);
+  }
+}
+
 // One field's contributions to the Newmark update of a point (assembly passes).
 struct AsmField {
   const realw* floc;
