@@ -102,7 +102,9 @@ __global__ __launch_bounds__(128) void k_smooth_elem(SmoothArgs A) {
   __shared__ int s_g[125];
   __shared__ uint8_t s_row[125];  // local point of each row
   __shared__ T s_u[C * SU];       // piece c of local point p at c * SU + p
-  __shared__ T s_t[3][128];
+  constexpr int NB = C <= 2 ? 2 : 1;  // two halves of the fluxes in turn save a barrier a piece; with
+                                      // more pieces their LDS costs waves (six: 120 -> 135 us)
+  __shared__ T s_t[NB][3][128];
   const int t = threadIdx.x;
   const int e = xcd_remap(blockIdx.x, A.nblocks_padded);
   if (e >= A.nspec) return;  // block-uniform
@@ -191,35 +193,36 @@ __global__ __launch_bounds__(128) void k_smooth_elem(SmoothArgs A) {
       t2 = P::fma_s(U[Lb0 + 5 * l], hpJ[l], t2);
       t3 = P::fma_s(U[Lc0 + 25 * l], hpK[l], t3);
     }
+    auto& S = s_t[NB == 2 ? c & 1 : 0];
     if constexpr (REG) {
-      s_t[0][t] = P::mul_s(t1, M[0][0]);
-      s_t[1][t] = P::mul_s(t2, M[1][1]);
-      s_t[2][t] = P::mul_s(t3, M[2][2]);
+      S[0][t] = P::mul_s(t1, M[0][0]);
+      S[1][t] = P::mul_s(t2, M[1][1]);
+      S[2][t] = P::mul_s(t3, M[2][2]);
     } else {
 #pragma unroll
       for (int a = 0; a < 3; ++a)
-        s_t[a][t] = P::fma_s(t3, M[a][2], P::fma_s(t2, M[a][1], P::mul_s(t1, M[a][0])));
+        S[a][t] = P::fma_s(t3, M[a][2], P::fma_s(t2, M[a][1], P::mul_s(t1, M[a][0])));
     }
     __syncthreads();  // fluxes complete; every lane is done reading this piece of s_u
     T d = P::zero();
 #pragma unroll
     for (int l = 0; l < 5; ++l) {
-      d = P::fma_s(s_t[0][La0 + l], hwI[l], d);
-      d = P::fma_s(s_t[1][Lb0 + 5 * l], hwJ[l], d);
-      d = P::fma_s(s_t[2][Lc0 + 25 * l], hwK[l], d);
+      d = P::fma_s(S[0][La0 + l], hwI[l], d);
+      d = P::fma_s(S[1][Lb0 + 5 * l], hwJ[l], d);
+      d = P::fma_s(S[2][Lc0 + 25 * l], hwK[l], d);
     }
     if constexpr (W == 1) {
       if (t < 125) {
         if (own >= A.n_shared) dat[(size_t)own * C + c] = P::fma_s(d, A.rvol[own], U[t]);
         else dloc[(L0 + sem_floc_slot(t)) * C + c] = d;
       }
-      if (c + 1 < C) __syncthreads();  // s_t free for the next value
-    } else {
-      if (t < 125) U[t] = d;  // own slot only
-      __syncthreads();        // s_t free for the next piece; the terms are in s_u
+    } else if (t < 125) {
+      U[t] = d;  // own slot only
     }
+    if (NB == 1 && c + 1 < C) __syncthreads();  // the fluxes are read
   }
   if constexpr (W == 1) return;
+  __syncthreads();  // the terms are in s_u
   for (int q = t; q < 125 * C; q += 128) {
     const int row = q / C, c = q - row * C;
     const int p = s_row[row], ig = s_g[p];
@@ -236,7 +239,8 @@ __global__ __launch_bounds__(128) void k_smooth_elem(SmoothArgs A) {
 // ddat(g) = sum of the element-local terms of g in element order (the reference CPU loop's
 // accumulation order); dat += rvol * ddat, for the points of more than one element.  One lane per
 // piece of a point's row, so consecutive lanes read and write whole rows (32x32x16 cubes, 21
-// fields: 94 us a step with a lane per row over all points; bound by the rows' traffic).
+// fields: 94 us a step with a lane per row over all points, 45 now; one field 11 us with a row at
+// a time, 8 in groups; bound by the rows' traffic, and for few fields by the chain offset, index, row).
 template <int NFP>
 __global__ void k_smooth_gather(int npts, const int* __restrict__ off, const int* __restrict__ idx,
                                 const realw* __restrict__ dloc, const realw* __restrict__ rvol,
@@ -246,29 +250,28 @@ __global__ void k_smooth_gather(int npts, const int* __restrict__ off, const int
   if (h >= (size_t)npts * C) return;
   const int g = (int)(h / C), c = (int)(h - (size_t)g * C);
   const int k1 = off[g + 1];
+  int k = off[g];
   const realw r = rvol[g];
-  if constexpr (W == 4) {
-    const float4* P = reinterpret_cast<const float4*>(dloc) + c;
-    float4* D = reinterpret_cast<float4*>(dat) + h;
-    const float4 v = *D;
-    float4 d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    int k = off[g];
-    for (; k + 1 < k1; k += 2) {  // both rows requested before either is added
-      const float4 a = P[(size_t)idx[k] * C], b = P[(size_t)idx[k + 1] * C];
-      d.x += a.x; d.y += a.y; d.z += a.z; d.w += a.w;
-      d.x += b.x; d.y += b.y; d.z += b.z; d.w += b.w;
-    }
-    if (k < k1) {
-      const float4 a = P[(size_t)idx[k] * C];
-      d.x += a.x; d.y += a.y; d.z += a.z; d.w += a.w;
-    }
-    *D = make_float4(fmaf(r, d.x, v.x), fmaf(r, d.y, v.y), fmaf(r, d.z, v.z), fmaf(r, d.w, v.w));
-  } else {
-    const realw v = dat[h];
-    realw d = 0.0f;
-    for (int k = off[g]; k < k1; ++k) d += dloc[(size_t)idx[k] * C + c];
-    dat[h] = fmaf(r, d, v);
-  }
+  using P = SmoothPiece<W>;
+  using T = typename P::T;
+  const T* rows = reinterpret_cast<const T*>(dloc) + c;
+  T* D = reinterpret_cast<T*>(dat) + h;
+  const T v = *D;
+  T d = P::zero();
+  // four, two and one rows at a time, all of a group requested before the first is added
+  auto add = [&](auto n) {
+    constexpr int M = decltype(n)::value;
+    T a[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) a[m] = rows[(size_t)idx[k + m] * C];
+#pragma unroll
+    for (int m = 0; m < M; ++m) d = P::fma_s(a[m], 1.0f, d);
+    k += M;
+  };
+  while (k + 3 < k1) add(std::integral_constant<int, 4>());
+  if (k + 1 < k1) add(std::integral_constant<int, 2>());
+  if (k < k1) add(std::integral_constant<int, 1>());
+  *D = P::fma_s(d, r, v);
 }
 
 // pin PML points: dat(iglob) = dat_bak(local), in element/point order
@@ -416,41 +419,39 @@ void plan_build(SmoothPlan& p, int nspec, int nglob, int nirr, int is_sph, const
   hipStream_t s = p.stream;
   p.nspec = nspec; p.nglob = nglob; p.nirr = nirr; p.nfield = nfield; p.nfp = padded_fields(nfield);
   const size_t nloc = (size_t)nspec * 125;
-  std::vector<int> ib(nloc);
+  if (nloc >= (size_t)INT32_MAX) SEM_FAIL("smooth: too many local points for 32-bit CSR indices");
+  std::vector<int> ib(nloc), touch(nglob, 0);
   for (size_t L = 0; L < nloc; ++L) {
     int g = ibool[L] - 1;
     if (g < 0 || g >= nglob) SEM_FAIL("smooth_pde: ibool(%zu)=%d outside 1..%d", L, g + 1, nglob);
     ib[L] = g;
+    ++touch[g];
   }
   // library numbering: points of more than one element first, in the caller's order, then the
-  // others element by element
-  std::vector<uint8_t> touch(nglob, 0);
-  for (size_t L = 0; L < nloc; ++L) touch[ib[L]] = (uint8_t)std::min(2, touch[ib[L]] + 1);
+  // others element by element; CSR shared point -> element rows in element order, by their place
+  // in the rows, in the same pass over the elements
   std::vector<int> perm(nglob, -1);
-  int n = 0;
-  for (int g = 0; g < nglob; ++g)
-    if (touch[g] != 1) perm[g] = n++;
-  p.n_shared = n;
-  for (size_t L = 0; L < nloc; ++L)
-    if (touch[ib[L]] == 1) perm[ib[L]] = n++;
-  for (size_t L = 0; L < nloc; ++L) ib[L] = perm[ib[L]];
-  p.d_perm = dev_upload(perm.data(), perm.size(), s);
-  p.d_ibool = dev_upload(ib.data(), nloc, s);
-  // CSR shared point -> element rows in element order, by their place in the rows
-  if (nloc >= (size_t)INT32_MAX) SEM_FAIL("smooth: too many local points for 32-bit CSR indices");
   {
-    int slot[125];
+    std::vector<int> off(1, 0);
+    off.reserve(nglob + 1);
+    for (int g = 0; g < nglob; ++g)
+      if (touch[g] != 1) {
+        perm[g] = (int)off.size() - 1;
+        off.push_back(off.back() + touch[g]);
+      }
+    p.n_shared = (int)off.size() - 1;
+    int slot[125], n = p.n_shared;
     for (int L = 0; L < 125; ++L) slot[L] = sem_floc_slot(L);
-    std::vector<int> off((size_t)p.n_shared + 1, 0);
-    for (size_t L = 0; L < nloc; ++L)
-      if (ib[L] < p.n_shared) off[(size_t)ib[L] + 1]++;
-    for (int g = 0; g < p.n_shared; ++g) off[g + 1] += off[g];
     std::vector<int> fill(off.begin(), off.end() - 1), idx((size_t)off[p.n_shared]);
     for (int e = 0; e < nspec; ++e)
       for (int L = 0; L < 125; ++L) {
-        const int g = ib[(size_t)e * 125 + L];
-        if (g < p.n_shared) idx[fill[g]++] = e * 125 + slot[L];
+        int& g = ib[(size_t)e * 125 + L];
+        if (touch[g] == 1) perm[g] = n++;
+        else idx[fill[perm[g]]++] = e * 125 + slot[L];
+        g = perm[g];
       }
+    p.d_perm = dev_upload(perm.data(), perm.size(), s);
+    p.d_ibool = dev_upload(ib.data(), nloc, s);
     p.d_off = dev_upload(off.data(), off.size(), s);
     p.d_idx = dev_upload(idx.data(), idx.size(), s);
     HIP_CHECK(hipStreamSynchronize(s));
