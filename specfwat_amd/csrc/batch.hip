@@ -375,7 +375,8 @@ void k_batch_elem(BatchElemArgs A) {
             const realw prod = (ea0 - t3a) * (eb0 - t3b) + (ea1 - t3a) * (eb1 - t3b) + (ea2 - t3a) * (eb2 - t3b) +
                                2.0f * (ea3 * eb3 + ea4 * eb4 + ea5 * eb5);
             const size_t kq = (size_t)ev * nloc + Lg;
-            kernel_acc_pair(A.mu_kl, A.mu_part, prod, A.kappa_kl, A.kappa_part, tra * trb, kq, A.dt, A.kflush != 0);
+            kernel_acc(A.mu_kl, A.mu_part, kq, prod, A.dt, A.kflush != 0);
+            kernel_acc(A.kappa_kl, A.kappa_part, kq, tra * trb, A.dt, A.kflush != 0);
           }
         }
         const realw ltr = lam * (duxdx + duydy + duzdz);

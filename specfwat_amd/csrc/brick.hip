@@ -161,7 +161,8 @@ __global__ __launch_bounds__(128) void k_brick(BrickArgs A) {
             const realw prod = (ea[0] - t3a) * (eb0 - t3b) + (ea[1] - t3a) * (eb1 - t3b) +
                                (ea[2] - t3a) * (eb2 - t3b) +
                                2.0f * (ea[3] * eb3 + ea[4] * eb4 + ea[5] * eb5);
-            kernel_acc_pair(A.mu_kl, A.mu_part, prod, A.kappa_kl, A.kappa_part, tra * trb, Lg, A.dt, A.kflush != 0);
+            kernel_acc(A.mu_kl, A.mu_part, Lg, prod, A.dt, A.kflush != 0);
+            kernel_acc(A.kappa_kl, A.kappa_part, Lg, tra * trb, A.dt, A.kflush != 0);
           }
         }
         const realw ltr = lam * (duxdx + duydy + duzdz);

@@ -229,7 +229,8 @@ __global__ __launch_bounds__(128) void k_forces(ForceArgs A) {
           const realw prod = (ea[0] - t3a) * (eb0 - t3b) + (ea[1] - t3a) * (eb1 - t3b) +
                              (ea[2] - t3a) * (eb2 - t3b) +
                              2.0f * (ea[3] * eb3 + ea[4] * eb4 + ea[5] * eb5);
-          kernel_acc_pair(A.mu_kl, A.mu_part, prod, A.kappa_kl, A.kappa_part, tra * trb, Lg, A.dt, A.kflush != 0);
+          kernel_acc(A.mu_kl, A.mu_part, Lg, prod, A.dt, A.kflush != 0);
+          kernel_acc(A.kappa_kl, A.kappa_part, Lg, tra * trb, A.dt, A.kflush != 0);
         } else {
           const realw va[6] = {ea[0], ea[1], ea[2], 2.0f * ea[5], 2.0f * ea[4], 2.0f * ea[3]};
           const realw vb[6] = {eb0, eb1, eb2, 2.0f * eb5, 2.0f * eb4, 2.0f * eb3};
@@ -420,7 +421,8 @@ __device__ __forceinline__ void forces_reg_body(const ForceArgs& A) {
         const realw prod = (st[0][0] - t3a) * (st[NF - 1][0] - t3b) + (st[0][1] - t3a) * (st[NF - 1][1] - t3b) +
                            (st[0][2] - t3a) * (st[NF - 1][2] - t3b) +
                            2.0f * (ea3 * eb3 + ea4 * eb4 + ea5 * eb5);
-        kernel_acc_pair(A.mu_kl, A.mu_part, prod, A.kappa_kl, A.kappa_part, tra * trb, Lg, A.dt, A.kflush != 0);
+        kernel_acc(A.mu_kl, A.mu_part, Lg, prod, A.dt, A.kflush != 0);
+        kernel_acc(A.kappa_kl, A.kappa_part, Lg, tra * trb, A.dt, A.kflush != 0);
       } else {
         const realw va[6] = {st[0][0], st[0][1], st[0][2], 2.0f * ea5, 2.0f * ea4, 2.0f * ea3};
         const realw vb[6] = {st[NF - 1][0], st[NF - 1][1], st[NF - 1][2], 2.0f * eb5, 2.0f * eb4, 2.0f * eb3};
