@@ -1549,13 +1549,14 @@ __global__ void __launch_bounds__(256) k_ws_prep(int nstep, double dt, double t0
 // the trace's time range [tstart, tend], and the neighbours its time-shift jump rule looks at
 // (nint(jump / dt) on either side and the one before), with two samples to spare.  The rest of
 // the trace, before the first arrival and after the slowest one, is never asked for: 31 % of
-// 9,800 window starts remain at 10,000 samples of 4 ms and a 12 s range.
+// 9,800 window starts remain at 10,000 samples of 4 ms and a 12 s range.  A negative jump_fac
+// switches the jump rule off: the rule then looks at no neighbour, the time range stays.
 __device__ __forceinline__ int2 ws_needed(int t, int nlen, int nw, double dt, double t0, double min_period,
                                           double min_velocity, double jump_fac, const double* __restrict__ tp,
                                           const double* __restrict__ dist) {
   const double tstart = tp[t] - min_period * 1.5 + t0;
   const double tend = dist[t] / min_velocity + min_period * 1.5 + t0;
-  const double nj = round(jump_fac * min_period / dt) + 3.0, half = (double)nlen / 2.0;
+  const double nj = fmax(round(jump_fac * min_period / dt), 0.0) + 3.0, half = (double)nlen / 2.0;
   const double lo = floor(tstart / dt - half) - nj, hi = ceil(tend / dt - half) + nj;
   // clamped as doubles; a NaN bound keeps its end of the trace
   return make_int2((int)fmin(fmax(lo, 0.0), (double)nw), (int)fmax(fmin(hi, (double)(nw - 1)), -1.0));

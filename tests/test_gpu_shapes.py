@@ -157,3 +157,28 @@ def test_adjoint_filter_at_block_edges(nstep):
             _, a, _, _ = orc.waveform_adjoint(obs[:, r, c], syn[:, r, c], dt, win)
             a = orc.filter_adj(a, dt, np.float32(1 / 12.0), np.float32(1 / 0.4), win)
             assert np.abs(adj[:, r, c] - a).max() <= 1e-6 * np.abs(a).max(), (r, c)  # single precision, as its other tests
+
+
+@pytest.mark.parametrize("jump_fac", [-2.0, -0.3, 0.0, 0.1, 3.0])
+def test_windows_with_any_jump_rule(jump_fac):
+    """The window starts that are computed are those the selection reads: the time range and the
+    jump rule's reach, none for a negative factor (the rule is off) and up to the whole trace.  The
+    first trace's range ends inside the signal on both sides, so windows reach to its ends."""
+    nstep, dt, T = 3000, 0.02, 2.0
+    print(f"jump factor {jump_fac}", flush=True)
+    t = np.arange(nstep) * dt
+    obs, syn = np.zeros((nstep, 2, 3), np.float32), np.zeros((nstep, 2, 3), np.float32)
+    for r in range(2):
+        for c in range(3):
+            syn[:, r, c] = np.sin(2 * np.pi * (0.5 * t + (0.002 + 0.001 * c) * t * t))
+            obs[:, r, c] = np.roll(syn[:, r, c], 3 + 2 * c)
+    tp, dist = np.array([18.0, 3.0]), np.array([2.4 * 42.0, 2.4 * 60.0])
+    cfg = dict(jump_fac=jump_fac, min_peaks_troughs=1, min_snr_window=0.1, min_win_len_fac=0.5)
+    got = misfit.select_windows(obs, syn, dt, 0.0, tp, dist, T, **cfg)
+    n = 0
+    for r in range(2):
+        for c in range(3):
+            ref, _, _ = orc.win_sel(obs[:, r, c], syn[:, r, c], dt, 0.0, tp[r], dist[r], T, **cfg)
+            np.testing.assert_array_equal(got[3 * r + c], ref)
+            n += len(ref)
+    assert n > 0
