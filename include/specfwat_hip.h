@@ -423,6 +423,10 @@ void fwat_waveform_adjoint_batch_noalloc_(int *nstep, int *ntrace, double *dt, r
 void fwat_cc_adjoint_batch_(int *nstep, int *ntrace, double *dt, realw *obs, realw *syn, int *nwin,
                             double *windows, double *taper_percentage, int *itaper_type, int *imeas,
                             double *cfg, int *nsect, realw *sos, double *misfits, double *meas, realw *adj);
+/* No counterpart in the reference, host only: the correlations of windows of 129 to 8192 samples sort
+ * their lags by transforms, and those within margin * |d| |s| of the largest value are compared by
+ * their direct sums; margin covers the rounding of both */
+void fwat_cc_lag_margin_(int *nl, double *margin);
 /* multitaper traveltime (imeas 13) / amplitude (14) measurement of every trace with the reference's
  * fall back to the cross-correlation measurement: MTTTMisfit%calc_adjoint_source
  * (src/preproc/adjoint_sources/mt_tt_misfit.f90:29-791 with utils/dpss.f90:137-262 and

@@ -115,6 +115,7 @@ SIGNATURES = {
     "fwat_waveform_adjoint_last_time_": "d",
     "fwat_waveform_adjoint_batch_noalloc_": "iidPPiDdiiFPPPl",
     "fwat_cc_adjoint_batch_": "iidFFiDdiiDiFDDF",
+    "fwat_cc_lag_margin_": "iD",
     "fwat_mt_adjoint_batch_": "iidFFiDdiiDiFDDF",
     "fwat_ep_adjoint_batch_": "iidFFiDdidiFDDF",
     "fwat_win_sel_batch_": "iidFFdDDdDiID",

@@ -640,11 +640,19 @@ __global__ void k_twiddles(int nf, double2* __restrict__ tw) {
   tw[j] = make_double2(cn, sn);
 }
 
+// How far below the largest transform value, in units of |d| |s|, a lag whose direct sum is the
+// largest can lie.  A transform's rounding is at most about 5 log2(nf) u of its 2-norm (u = 2^-53;
+// windows scaled by powers of two into [-1, 1]): two times |d| |s| for the spectra, sqrt(nl) |d| |s|
+// for the inverse.  A direct sum of nl products is off by at most nl u |d| |s| itself.  Both twice,
+// for the two lags compared.
+__host__ __device__ inline double cc_lag_margin(int nl, int logM) {
+  const double transform = 5.0 * (logM + 1) * (2.0 + sqrt((double)nl)) + 16.0, direct = (double)nl + 4.0;
+  return 2.0 * (transform + direct) * 1.1102230246251565e-16;
+}
+
 // xcorr_shift by transforms: one workgroup per trace, the full correlation of its two windows as
 // the inverse transform of D conj(S) on nf >= 2 nl - 1 points in LDS (nf / 2 complex values), and
-// the lag of its first maximum.  A transform's rounding is at most about 5 log2(nf) u of its
-// 2-norm (u = 2^-53; windows scaled by powers of two into [-1, 1]): two times |d| |s| for the
-// spectra, sqrt(nl) |d| |s| for the inverse.  Lags within twice their sum of the largest value are
+// the lag of its first maximum.  Lags within cc_lag_margin of the largest value are
 // summed again as the reference sums them and compared, so the lag is the one of the direct sums
 // (k_cc_corr) in every case.  Real windows have one lag left and
 // sum nothing.  nl^2 products become nf log2(nf): two windows of 5,000 and 6,000 samples of
@@ -710,8 +718,7 @@ __global__ void __launch_bounds__(NT) k_cc_corr_fft(int nl, int nf, int logM, co
   double best = -INFINITY;
   for (int m = lane; m < nlag; m += NT) best = fmax(best, value(m));
   best = mt_bmax<NT>(best, red);
-  const double bound =
-      2.0 * (5.0 * (logM + 1) * (2.0 + sqrt((double)nl)) + 16.0) * 1.1102230246251565e-16 * sqrt(nd * ns);
+  const double bound = cc_lag_margin(nl, logM) * sqrt(nd * ns);
   const double thr = odd || !(bound < INFINITY) ? -INFINITY : best - bound;
   double count = 0.0;
   int only = 0x7fffffff;
@@ -2446,6 +2453,15 @@ void fwat_waveform_adjoint_batch_noalloc_(int* nstep, int* ntrace, double* dt, r
   hipLaunchKernelGGL(k_trace_misfits, dim3(nb), dim3(MTPB), 0, s, T, nw, d_mr, d_misfits, d_residuals);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(s));
+}
+
+// Margin of the transform path's lags for windows of nl samples, in units of |d| |s| (host only):
+// a lag further than this below the largest transform value cannot have the largest direct sum.
+void fwat_cc_lag_margin_(int* nl, double* margin) {
+  if (!CcShift::fft(*nl)) SEM_FAIL("fwat_cc_lag_margin_: windows of %d samples take the direct sums", *nl);
+  int logM = 0;
+  while ((2 << logM) < CcShift::points(*nl)) ++logM;
+  *margin = cc_lag_margin(*nl, logM);
 }
 
 // cc_tt_misfit.f90 CCTTMisfit%calc_adjoint_source for every trace: imeas 11

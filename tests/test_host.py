@@ -240,3 +240,16 @@ def test_fixed_window_types():
     np.testing.assert_allclose(w, [[-2.0, 21.0], [35.0, 47.9]])
     with pytest.raises(ValueError):
         misfit.fixed_windows(1, 1000, 0.05, 2.0)
+
+
+@pytest.mark.parametrize("nl", [129, 1000, 4096, 4097, 6000, 8192])
+def test_lag_margin_covers_transforms_and_direct_sums(nl):
+    """A lag left out of the direct sums must not be able to win them: the margin holds the rounding
+    of two transform values (5 log2(nf) u of a 2-norm each for the spectra's |d| |s|, twice, and for
+    the inverse, at most sqrt(nl) |d| |s|) and of two direct sums of nl products (nl u |d| |s|)."""
+    u, log_nf = 2.0 ** -53, int(np.ceil(np.log2(2 * nl - 1)))
+    out = np.zeros(1)
+    _lib.call("fwat_cc_lag_margin_", nl, out)
+    margin = out[0]
+    assert margin >= 2 * u * (5 * log_nf * (2 + np.sqrt(nl)) + nl)
+    assert margin < 1e-11  # far below the gap between the lags of a real window
