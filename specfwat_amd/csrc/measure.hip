@@ -244,6 +244,27 @@ __device__ __forceinline__ double lag_sum(int mm, int nlen, const double* dw, co
   return c;
 }
 
+// the sums of lag indices mb .. mb + 3 (mb a multiple of four) as lag_sum takes them, together: one
+// read of each window for four products
+__device__ __forceinline__ void lag_sum4(int mb, int nlen, const double* dw, const double* sw, double (&c)[4]) {
+  const int lo = mb - (nlen - 1) > 0 ? mb - (nlen - 1) : 0, hi = mb + 3 < nlen - 1 ? mb + 3 : nlen - 1;
+  const int off = nlen - 1 - mb;
+  const auto at = [&](int k) { return k >= 0 && k < nlen ? sw[k] : 0.0; };
+  double r0 = at(lo + off), r1 = at(lo + off - 1), r2 = at(lo + off - 2), r3 = at(lo + off - 3);
+  c[0] = c[1] = c[2] = c[3] = 0.0;
+  for (int j = lo; j <= hi; ++j) {
+    const double dv = dw[j];
+    c[0] = c[0] + dv * r0;
+    c[1] = c[1] + dv * r1;
+    c[2] = c[2] + dv * r2;
+    c[3] = c[3] + dv * r3;
+    r3 = r2;
+    r2 = r1;
+    r1 = r0;
+    r0 = at(j + 1 + off);
+  }
+}
+
 // xcorr_shift, first stage: workgroup (trace, block of 1024 lags, 4 consecutive
 // lags per lane) of the full correlation; d and the matching stretch of s come
 // through LDS in chunks of 1024 samples taken in increasing i1, so each lag's
@@ -656,7 +677,8 @@ __host__ __device__ inline double cc_lag_margin(int nl, int logM) {
 // summed again as the reference sums them and compared, so the lag is the one of the direct sums
 // (k_cc_corr) in every case.  Real windows have one lag left and
 // sum nothing.  nl^2 products become nf log2(nf): two windows of 5,000 and 6,000 samples of
-// 1,200 traces 9.7 ms by direct sums.  G: nf / 2 + 1 spectrum values per trace.
+// 1,200 traces 9.7 ms by direct sums.  Windows with a value that is not finite have no transform:
+// every lag is summed as k_cc_corr does.  G: nf / 2 + 1 spectrum values per trace.
 template <int NT>
 __global__ void __launch_bounds__(NT) k_cc_corr_fft(int nl, int nf, int logM, const double2* __restrict__ tw,
                                                     const double* __restrict__ D, const double* __restrict__ S,
@@ -679,67 +701,81 @@ __global__ void __launch_bounds__(NT) k_cc_corr_fft(int nl, int nf, int logM, co
   sm = mt_bmax<NT>(sm, red);
   const bool odd = mt_bmax<NT>(bad, red) != 0.0;
   const int de = dm > 0.0 && !odd ? ilogb(dm) + 1 : 0, se = sm > 0.0 && !odd ? ilogb(sm) + 1 : 0;
-  double nd = 0.0, ns = 0.0;
-  for (int j = lane; j < nl; j += NT) {
-    const double a = ldexp(d[j], -de), b = ldexp(s[j], -se);
-    nd += a * a;
-    ns += b * b;
-  }
-  nd = mt_bsum<NT>(nd, red);
-  ns = mt_bsum<NT>(ns, red);
-  const auto spectrum = [&](int k) {
-    if (k == 0 || k == M) {
-      const double2 z = cbuf[0];
-      return make_double2(k == 0 ? z.x + z.y : z.x - z.y, 0.0);
-    }
-    return mt_half(cbuf[k], cbuf[M - k], tw[k]);
-  };
-  mt_load_real<NT>(cbuf, M, logM, nl, [&](int n) { return ldexp(d[n], -de); });
-  mt_fft<NT>(cbuf, M, logM, nf, tw, false);
-  for (int k = lane; k <= M; k += NT) g[k] = spectrum(k);
-  __syncthreads();
-  mt_load_real<NT>(cbuf, M, logM, nl, [&](int n) { return ldexp(s[n], -se); });
-  mt_fft<NT>(cbuf, M, logM, nf, tw, false);
-  for (int k = lane; k <= M; k += NT) {
-    const double2 X = spectrum(k);
-    g[k] = cmul(g[k], make_double2(X.x, -X.y));
-  }
-  __syncthreads();
-  for (int k = lane; k < M; k += NT) cbuf[__brev((unsigned)k) >> shb] = mt_repack(g[k], g[M - k], tw[k]);
-  __syncthreads();
-  mt_fft<NT>(cbuf, M, logM, nf, tw, true);
-  // lag index m: lag l = m + 1 - nl at sample l (l >= 0) or nf + l
   const int nlag = 2 * nl - 1;
-  const auto value = [&](int m) {
-    const int l = m + 1 - nl, n = l >= 0 ? l : nf + l;
-    const double2 z = cbuf[n >> 1];
-    return ((n & 1) ? z.y : z.x) / M;
-  };
-  double best = -INFINITY;
-  for (int m = lane; m < nlag; m += NT) best = fmax(best, value(m));
-  best = mt_bmax<NT>(best, red);
-  const double bound = cc_lag_margin(nl, logM) * sqrt(nd * ns);
-  const double thr = odd || !(bound < INFINITY) ? -INFINITY : best - bound;
-  double count = 0.0;
-  int only = 0x7fffffff;
-  for (int m = lane; m < nlag; m += NT)
-    if (!(value(m) < thr)) {
-      count += 1.0;
-      only = min(only, m);
-    }
-  count = mt_bsum<NT>(count, red);
   double bv = -INFINITY;
   int bm = 0x7fffffff;
-  if (!odd && (nd == 0.0 || ns == 0.0)) {
-    bm = 0;  // every sum is zero: the first lag
-  } else if (count == 1.0) {
-    bm = only;
+  if (odd) {  // block-uniform
+    // every lag by its direct sum, four a lane, both windows in LDS (2 nl <= nf doubles)
+    double* dw = reinterpret_cast<double*>(cbuf);
+    double* sw = dw + nl;
+    for (int j = lane; j < nl; j += NT) { dw[j] = d[j]; sw[j] = s[j]; }
+    __syncthreads();
+    for (int mb = 4 * lane; mb < nlag; mb += 4 * NT) {
+      double c[4];
+      lag_sum4(mb, nl, dw, sw, c);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (mb + q < nlag && c[q] > bv) { bv = c[q]; bm = mb + q; }
+    }
   } else {
+    double nd = 0.0, ns = 0.0;
+    for (int j = lane; j < nl; j += NT) {
+      const double a = ldexp(d[j], -de), b = ldexp(s[j], -se);
+      nd += a * a;
+      ns += b * b;
+    }
+    nd = mt_bsum<NT>(nd, red);
+    ns = mt_bsum<NT>(ns, red);
+    const auto spectrum = [&](int k) {
+      if (k == 0 || k == M) {
+        const double2 z = cbuf[0];
+        return make_double2(k == 0 ? z.x + z.y : z.x - z.y, 0.0);
+      }
+      return mt_half(cbuf[k], cbuf[M - k], tw[k]);
+    };
+    mt_load_real<NT>(cbuf, M, logM, nl, [&](int n) { return ldexp(d[n], -de); });
+    mt_fft<NT>(cbuf, M, logM, nf, tw, false);
+    for (int k = lane; k <= M; k += NT) g[k] = spectrum(k);
+    __syncthreads();
+    mt_load_real<NT>(cbuf, M, logM, nl, [&](int n) { return ldexp(s[n], -se); });
+    mt_fft<NT>(cbuf, M, logM, nf, tw, false);
+    for (int k = lane; k <= M; k += NT) {
+      const double2 X = spectrum(k);
+      g[k] = cmul(g[k], make_double2(X.x, -X.y));
+    }
+    __syncthreads();
+    for (int k = lane; k < M; k += NT) cbuf[__brev((unsigned)k) >> shb] = mt_repack(g[k], g[M - k], tw[k]);
+    __syncthreads();
+    mt_fft<NT>(cbuf, M, logM, nf, tw, true);
+    // lag index m: lag l = m + 1 - nl at sample l (l >= 0) or nf + l
+    const auto value = [&](int m) {
+      const int l = m + 1 - nl, n = l >= 0 ? l : nf + l;
+      const double2 z = cbuf[n >> 1];
+      return ((n & 1) ? z.y : z.x) / M;
+    };
+    double best = -INFINITY;
+    for (int m = lane; m < nlag; m += NT) best = fmax(best, value(m));
+    best = mt_bmax<NT>(best, red);
+    const double thr = best - cc_lag_margin(nl, logM) * sqrt(nd * ns);
+    double count = 0.0;
+    int only = 0x7fffffff;
     for (int m = lane; m < nlag; m += NT)
       if (!(value(m) < thr)) {
-        const double c = lag_sum(m, nl, d, s);
-        if (c > bv || (c == bv && m < bm)) { bv = c; bm = m; }
+        count += 1.0;
+        only = min(only, m);
       }
+    count = mt_bsum<NT>(count, red);
+    if (nd == 0.0 || ns == 0.0) {
+      bm = 0;  // every sum is zero: the first lag
+    } else if (count == 1.0) {
+      bm = only;
+    } else {
+      for (int m = lane; m < nlag; m += NT)
+        if (!(value(m) < thr)) {
+          const double c = lag_sum(m, nl, d, s);
+          if (c > bv || (c == bv && m < bm)) { bv = c; bm = m; }
+        }
+    }
   }
   red[lane] = bv;
   ri[lane] = bm;
@@ -1609,9 +1645,18 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
   float* cs = reinterpret_cast<float*>(sw + nq);  // fp32 sums of lag index 0 .. 2 nlen - 2
   float* df = cs + 2 * nq;
   float* sf = df + nq;  // s[x mod nlen] at sf[x + nq + 4], x = -nq - 4 .. nq + 3
+  const int nlag = 2 * nlen - 1;
+  const auto first_max = [](double bv, int bm) {  // the lanes' first maximum
+    for (int o = 32; o > 0; o >>= 1) {
+      const double v2 = __shfl_xor(bv, o);
+      const int m2 = __shfl_xor(bm, o);
+      if (v2 > bv || (v2 == bv && m2 < bm)) { bv = v2; bm = m2; }
+    }
+    return bm;
+  };
   float dm = 0.0f, sm = 0.0f;
-  bool odd = false;  // a value that is not finite
   {
+    bool odd = false;  // a value that is not finite
     const double* d = Dn + (size_t)t * nstep + i;
     const double* s = Sn + (size_t)t * nstep + i;
     double dmx = 0.0, smx = 0.0;
@@ -1627,10 +1672,28 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
       dmx = fmax(dmx, __shfl_xor(dmx, o));
       smx = fmax(smx, __shfl_xor(smx, o));
     }
-    odd = __any(odd);
-    // powers of two: the scaled windows' largest magnitudes lie in [1/2, 1)
-    const int de = dmx > 0.0 && !odd ? ilogb(dmx) + 1 : 0, se = smx > 0.0 && !odd ? ilogb(smx) + 1 : 0;
     __threadfence_block();
+    if (__any(odd)) {  // no scale: every lag by its direct sum, four a lane, the longest sums (the middle lags') first
+      const int nb = (nlag + 3) / 4, mid = nb / 2;
+      double bv = -INFINITY;
+      int bm = 0x7fffffff;
+      for (int r = lane; r <= nb; r += 64) {
+        const int b = r & 1 ? mid - (r + 1) / 2 : mid + r / 2;
+        if (b < 0 || b >= nb) continue;
+        double c[4];
+        lag_sum4(4 * b, nlen, dw, sw, c);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int m = 4 * b + q;
+          if (m < nlag && (c[q] > bv || (c[q] == bv && m < bm))) { bv = c[q]; bm = m; }
+        }
+      }
+      bm = first_max(bv, bm);
+      if (lane == 0) ish_out[(size_t)t * nw + i] = bm + 1 - nlen;
+      return;
+    }
+    // powers of two: the scaled windows' largest magnitudes lie in [1/2, 1)
+    const int de = dmx > 0.0 ? ilogb(dmx) + 1 : 0, se = smx > 0.0 ? ilogb(smx) + 1 : 0;
     for (int j = lane; j < nq; j += 64) {
       const float v = j < nlen ? (float)ldexp(dw[j], -de) : 0.0f;
       df[j] = v;
@@ -1648,7 +1711,6 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
     }
   }
   __threadfence_block();  // LDS of this wavefront, written and read by its own lanes
-  const int nlag = 2 * nlen - 1;
   float best = -INFINITY;
   for (int r = lane; 4 * r < nlen; r += 64) {
     const int mb = 4 * r;
@@ -1687,7 +1749,7 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
   // error of a sum: (nlen + 3) roundings of at most |d| |s| (two of the scaled inputs, nq of the
   // running sum), twice for the differences, twice for two sums compared, 1/16 to spare
   const float bound = 4.25f * (float)(nq + 8) * 5.9604645e-8f * sqrtf(dm * sm);
-  const float thr = odd || !(bound < INFINITY) ? -INFINITY : best - bound;
+  const float thr = best - bound;
   int count = 0, only = 0;
   for (int m0 = 0; m0 < nlag; m0 += 64) {
     const unsigned long long w = __ballot(m0 + lane < nlag && !(cs[min(m0 + lane, nlag - 1)] < thr));
@@ -1695,7 +1757,7 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
     count += __builtin_popcountll(w);
   }
   int bm = only;
-  if (!odd && (dm == 0.0f || sm == 0.0f)) {
+  if (dm == 0.0f || sm == 0.0f) {
     bm = 0;  // every sum is zero: the first lag
   } else if (count != 1) {
     double bv = -INFINITY;
@@ -1705,11 +1767,7 @@ __global__ void __launch_bounds__(256) k_ws_sliding(int nstep, int nlen, int nw,
         const double c = lag_sum(m, nlen, dw, sw);
         if (c > bv || (c == bv && m < bm)) { bv = c; bm = m; }
       }
-    for (int o = 32; o > 0; o >>= 1) {
-      const double v2 = __shfl_xor(bv, o);
-      const int m2 = __shfl_xor(bm, o);
-      if (v2 > bv || (v2 == bv && m2 < bm)) { bv = v2; bm = m2; }
-    }
+    bm = first_max(bv, bm);
   }
   if (lane == 0) ish_out[(size_t)t * nw + i] = bm + 1 - nlen;
 }

@@ -182,3 +182,90 @@ def test_windows_with_any_jump_rule(jump_fac):
             np.testing.assert_array_equal(got[3 * r + c], ref)
             n += len(ref)
     assert n > 0
+
+
+def _direct_shift(d, s):
+    """The first maximum of every lag's direct sum, the lags in fours over the union of their ranges
+    (a sample that is not a number makes a zero product one too); None when no sum is above -inf."""
+    n, best, at = len(d), -np.inf, None
+    pad = np.concatenate([np.zeros(3), s, np.zeros(3)])
+    with np.errstate(invalid="ignore"):
+        for mb in range(0, 2 * n - 1, 4):
+            lo, hi = max(0, mb - n + 1), min(n - 1, mb + 3)
+            for m in range(mb, min(mb + 4, 2 * n - 1)):
+                c = np.cumsum(d[lo:hi + 1] * pad[lo + n - 1 - m + 3:hi + n - 1 - m + 4])[-1]
+                if c > best:
+                    best, at = c, m + 1 - n
+    return at
+
+
+@pytest.mark.filterwarnings("ignore:invalid value")
+@pytest.mark.parametrize("nl", [128, 129, 517, 2049])
+def test_correlation_shift_of_data_that_are_not_finite(nl):
+    """Windows with NaN or infinite samples, whose transforms say nothing: the shift is the direct
+    sums' in every path (nl 128 has no other); a window of NaN only is not selected."""
+    nstep, dt = nl + 7, 0.01
+    rng = np.random.default_rng(nl)
+    obs, syn = (rng.standard_normal((nstep, 3, 3)).astype(np.float32) for _ in range(2))
+    a, b = 4 + nl // 5, 4 + (7 * nl) // 8
+    obs[a, 0, 0], obs[b, 0, 1], syn[a, 0, 2] = np.nan, np.inf, -np.inf
+    syn[b, 1, 0], obs[a, 1, 1], obs[b, 1, 1] = np.nan, np.nan, np.nan
+    obs[4, 1, 2], syn[nl + 2, 1, 2] = np.nan, np.inf
+    obs[:, 2, 0] = np.nan
+    win = [[0.03, 0.03 + nl * dt + 0.001]]
+    print(f"correlation of {nl} samples that are not finite", flush=True)
+    _, adj, meas = misfit.event_cc_adjoint_sources(obs, syn, dt, win, imeas=11)
+    first, _, n = misfit.get_window_info(win[0], dt)
+    first -= 1
+    assert n == nl
+    tw = misfit.window_taper(np.ones(n), 0.05, 1)
+    for k in range(9):
+        d, s = (x[first:first + n, k // 3, k % 3].astype(np.float64) * tw for x in (obs, syn))
+        ref = _direct_shift(d, s)
+        if k == 6:
+            assert ref is None and meas[k, 0, 6] == 0 and not adj[:, 2, 0].any()
+        else:
+            assert meas[k, 0, 7] == ref, k
+
+
+@pytest.mark.filterwarnings("ignore:invalid value")
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_windows_of_data_that_are_not_finite(bad):
+    """Window starts whose samples are not all finite take every lag's direct sum: their shifts decide
+    by the jump rule which starts beside them stay good.  The oracle's shifts and coefficients
+    of the clean trace, with those starts' shifts put in, give the windows."""
+    nstep, dt, T, thr, max_shift = 1700, 0.02, 2.0, 0.8, 0.3
+    t = np.arange(nstep) * dt
+    obs, syn = np.zeros((nstep, 1, 3), np.float32), np.zeros((nstep, 1, 3), np.float32)
+    for c in range(3):
+        syn[:, 0, c] = np.sin(2 * np.pi * (0.5 * t + 0.002 * t * t))
+        obs[:, 0, c] = np.roll(syn[:, 0, c], 3 + c)
+    hit = (800, 0 if np.isnan(bad) else 1), (1003, 2)  # (sample, component) of obs; the second pair of syn when NaN
+    clean = obs.copy(), syn.copy()
+    obs[hit[0][0], 0, hit[0][1]] = bad
+    (syn if np.isnan(bad) else obs)[hit[1][0], 0, hit[1][1]] = bad
+    tp, dist, jump_fac = 6.0, 2.4 * 28.0, 0.1
+    print(f"windows with {bad}", flush=True)
+    got = misfit.select_windows(obs, syn, dt, 0.0, np.array([tp]), np.array([dist]), T, min_peaks_troughs=0,
+                                min_snr_window=0.0, min_energy_ratio=1e9, min_win_len_fac=0.5, jump_fac=jump_fac)
+    nlen = int(2.0 * T / dt) + 1
+    tw, nw = misfit.window_taper(np.ones(nlen), 1.0, 1), nstep - nlen
+    tc = (np.arange(nw) + nlen / 2.0) * dt
+    nj, n = int(jump_fac * T / dt + 0.5), 0
+    for c in range(3):
+        _, cc, ts = orc.win_sel(clean[0][:, 0, c], clean[1][:, 0, c], dt, 0.0, tp, dist, T, min_peaks_troughs=0)
+        d, s = (x[:, 0, c].astype(np.float64) / np.abs(clean[1][:, 0, c]).max() for x in (obs, syn))
+        for i in range(nw):
+            if not (np.isfinite(d[i:i + nlen]).all() and np.isfinite(s[i:i + nlen]).all()):
+                dw, sw = d[i:i + nlen] * tw, s[i:i + nlen] * tw
+                k = _direct_shift(dw, sw)
+                x, y = (dw[k:], sw[:nlen - k]) if k >= 0 else (dw[:k], sw[-k:])  # what overlaps after the shift
+                cc[i], ts[i] = (x * y).sum() / np.sqrt((x * x).sum() * (y * y).sum()), k * dt
+        good = (cc > thr) & (np.abs(ts) < max_shift * T) & (tc >= tp - 1.5 * T) & (tc <= dist / 2.4 + 1.5 * T)
+        for i in np.flatnonzero(np.abs(np.diff(ts)) > jump_fac * T) + 1:
+            good[max(0, i - nj):i + nj + 1] = False
+        edge = np.flatnonzero(np.diff(np.concatenate([[0], good.astype(int), [0]])))
+        ref = [(tc[a], tc[b - 1]) for a, b in zip(edge[::2], edge[1::2]) if (b - 1 - a) * dt >= 0.5 * T]
+        np.testing.assert_array_equal(got[c], np.array(ref).reshape(-1, 2))
+        n += len(ref)
+    assert n >= 4
