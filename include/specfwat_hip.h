@@ -220,6 +220,9 @@ void fwat_floc_row_layout_(int *slot);
  * host's launch rate); captured runs are not timed.  Replaces the per-step launches of
  * iterate_time (prepare_fwd.f90:364); no counterpart in the reference. */
 void fwat_set_graph_(long *Mesh_pointer, int *on);
+/* device memory (bytes, default 256 MiB) that the c_ij kernels of a handle, and all kernels of a
+ * batch on it, take at a time on their way to the host; fewer when the device is full */
+void fwat_set_readout_bytes_(long *Mesh_pointer, int *bytes);
 /* Host-only (no device work): the gather-assembly CSR the preparation entry points build for
  * these arrays -- for every point its element terms in the order of SPECFEM's CPU element loop
  * over phase_ispec_inner_elastic (outer elements, then inner; the loop shape of

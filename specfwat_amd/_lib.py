@@ -70,6 +70,7 @@ SIGNATURES = {
     "fwat_set_floc_layout_": "Li",
     "fwat_floc_row_layout_": "I",
     "fwat_set_graph_": "Li",
+    "fwat_set_readout_bytes_": "Li",
     "fwat_assembly_csr_": "iiIiIIiIiIiIiiII",
     "fwat_set_slabs_": "Li",
     "fwat_batch_create_": "LLiIfFID",

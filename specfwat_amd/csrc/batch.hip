@@ -788,29 +788,22 @@ __global__ void k_fill_u32(unsigned int* p, size_t n) {
   if (i < n) p[i] = 0u;
 }
 
-// per event, out [E][nloc]: the density kernel of every local point, -rho K, and a modulus kernel
-// scaled as save_adjoint_kernels does
-__global__ void k_batch_expand_rho(size_t nloc, int E, const int* __restrict__ ibool, const double* __restrict__ K,
+// local points [L0, L0 + n) of every event, out [E][n]: the density kernel, -rho K (rho: those points'),
+// and a modulus kernel scaled as save_adjoint_kernels does
+__global__ void k_batch_expand_rho(size_t L0, size_t n, int E, const int* __restrict__ ibool, const double* __restrict__ K,
                                    const realw* __restrict__ rho, double* __restrict__ out) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nloc * E) return;
-  const size_t e = i / nloc, L = i - e * nloc;
-  out[i] = -(double)rho[L] * K[(size_t)ibool[L] * E + e];
+  if (i >= n * E) return;
+  const size_t e = i / n, l = i - e * n;
+  out[i] = -(double)rho[l] * K[(size_t)ibool[L0 + l] * E + e];
 }
 
-__global__ void k_batch_scale(size_t nloc, int E, const double* __restrict__ K, const realw* __restrict__ modulus,
-                              double factor, double* __restrict__ out) {
+__global__ void k_batch_scale(size_t L0, size_t n, size_t nloc, int E, const double* __restrict__ K,
+                              const realw* __restrict__ modulus, double factor, double* __restrict__ out) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nloc * E) out[i] = K[i] * (factor * (double)modulus[i % nloc]);
-}
-
-// c_ij kernels of one element from rows [21][125] to the caller's [125][21], negated, through LDS
-__global__ __launch_bounds__(256) void k_batch_cij_point_major(const double* __restrict__ K, double* __restrict__ out) {
-  __shared__ double s[2625];
-  const size_t b = (size_t)blockIdx.x * 2625;
-  for (int i = threadIdx.x; i < 2625; i += 256) s[i] = K[b + i];
-  __syncthreads();
-  for (int i = threadIdx.x; i < 2625; i += 256) out[b + i] = -s[(i % 21) * 125 + i / 21];
+  if (i >= n * E) return;
+  const size_t e = i / n, L = L0 + (i - e * n);
+  out[i] = K[e * nloc + L] * (factor * (double)modulus[L]);
 }
 
 __global__ void k_batch_vshift(size_t n, realw* __restrict__ v, const realw* __restrict__ a, realw dto2) {
@@ -1027,6 +1020,36 @@ void ensure_store(SemBatch* B) {
     const size_t ns = (size_t)B->nmax * B->E;
     hipLaunchKernelGGL(k_fill_u32, dim3(nblk(ns)), dim3(TPB), 0, s, B->store_max, ns);
   }
+}
+
+// Kernels of every event to the host, scaled on the device, as many points at a time as the read-out
+// may take memory for: the density's and (mu not null) the moduli's, [E][nloc] each.
+void batch_points_to_host(SemBatch* B, const realw* h_rhostore, double* rho, double* mu, double* kappa) {
+  SemMesh* m = B->m;
+  hipStream_t s = m->stream;
+  const size_t E = (size_t)B->E, nloc = (size_t)m->nspec * 125;
+  size_t most = 0;
+  double* tmp = (double*)sem_readout_alloc(nloc, E * sizeof(double) + sizeof(realw), m->readout_bytes, &most);
+  realw* d_rho = (realw*)(tmp + E * most);
+  for (size_t L0 = 0; L0 < nloc; L0 += most) {
+    const size_t n = std::min(most, nloc - L0);
+    const auto out = [&](double* host) {
+      HIP_CHECK(hipGetLastError());
+      if (n == nloc) sem_to_host(host, tmp, E * n * sizeof(double), s);
+      else
+        for (size_t e = 0; e < E; ++e) sem_to_host(host + e * nloc + L0, tmp + e * n, n * sizeof(double), s);
+    };
+    HIP_CHECK(hipMemcpyAsync(d_rho, h_rhostore + L0, n * sizeof(realw), hipMemcpyHostToDevice, s));
+    const dim3 gr(nblk(n * E)), bl(TPB);
+    hipLaunchKernelGGL(k_batch_expand_rho, gr, bl, 0, s, L0, n, (int)E, m->d_ibool, B->rho_kl, d_rho, tmp);
+    out(rho);
+    if (!mu) continue;
+    hipLaunchKernelGGL(k_batch_scale, gr, bl, 0, s, L0, n, nloc, (int)E, B->mu_kl, m->d_mu, -2.0, tmp);
+    out(mu);
+    hipLaunchKernelGGL(k_batch_scale, gr, bl, 0, s, L0, n, nloc, (int)E, B->kappa_kl, m->d_kappa, -1.0, tmp);
+    out(kappa);
+  }
+  dev_free(tmp);
 }
 
 // element / assembly pass times summed over the sampled steps of a timed run
@@ -1322,23 +1345,9 @@ void fwat_batch_seismograms_(long* Batch_pointer, realw* h_seis) {
 void fwat_batch_kernels_(long* Batch_pointer, realw* h_rhostore, double* h_rho_kl, double* h_mu_kl,
                          double* h_kappa_kl) {
   SemBatch* B = batch_of(Batch_pointer);
-  SemMesh* m = B->m;
   if (B->aniso) SEM_FAIL("anisotropic batch: its kernels come from fwat_batch_kernels_ani_");
   if (!B->mu_kl) SEM_FAIL("fwat_batch_adjoint_ has not run");
-  const int E = B->E;
-  const size_t nloc = (size_t)m->nspec * 125, n = (size_t)E * nloc;
-  hipStream_t s = m->stream;
-  // scaled on the device, one array after the other through one buffer
-  realw* d_rho = dev_upload(h_rhostore, nloc, s);
-  double* tmp = dev_alloc<double>(n);
-  hipLaunchKernelGGL(k_batch_expand_rho, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, m->d_ibool, B->rho_kl, d_rho, tmp);
-  sem_to_host(h_rho_kl, tmp, n * 8, s);
-  hipLaunchKernelGGL(k_batch_scale, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, B->mu_kl, m->d_mu, -2.0, tmp);
-  sem_to_host(h_mu_kl, tmp, n * 8, s);
-  hipLaunchKernelGGL(k_batch_scale, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, B->kappa_kl, m->d_kappa, -1.0, tmp);
-  sem_to_host(h_kappa_kl, tmp, n * 8, s);
-  dev_free(tmp);
-  dev_free(d_rho);
+  batch_points_to_host(B, h_rhostore, h_rho_kl, h_mu_kl, h_kappa_kl);
 }
 
 // Kernels of an anisotropic batch per event: rho_kl (NGLLX,NGLLY,NGLLZ,NSPEC_AB,nevents) scaled by
@@ -1349,19 +1358,8 @@ void fwat_batch_kernels_ani_(long* Batch_pointer, realw* h_rhostore, double* h_r
   SemMesh* m = B->m;
   if (!B->aniso) SEM_FAIL("isotropic batch: its kernels come from fwat_batch_kernels_");
   if (!B->cijkl_kl) SEM_FAIL("fwat_batch_adjoint_ has not run");
-  const int E = B->E;
-  const size_t nloc = (size_t)m->nspec * 125, n = (size_t)E * nloc;
-  hipStream_t s = m->stream;
-  realw* d_rho = dev_upload(h_rhostore, nloc, s);
-  double* tmp = dev_alloc<double>(std::max(n, nloc * 21));
-  hipLaunchKernelGGL(k_batch_expand_rho, dim3(nblk(n)), dim3(TPB), 0, s, nloc, E, m->d_ibool, B->rho_kl, d_rho, tmp);
-  sem_to_host(h_rho_kl, tmp, n * 8, s);
-  for (int e = 0; e < E; ++e) {
-    hipLaunchKernelGGL(k_batch_cij_point_major, dim3(m->nspec), dim3(256), 0, s, B->cijkl_kl + (size_t)e * nloc * 21, tmp);
-    sem_to_host(h_cijkl_kl + (size_t)e * nloc * 21, tmp, nloc * 21 * 8, s);
-  }
-  dev_free(tmp);
-  dev_free(d_rho);
+  batch_points_to_host(B, h_rhostore, h_rho_kl, nullptr, nullptr);
+  sem_cij_to_host(m, B->cijkl_kl, (size_t)B->E * m->nspec, h_cijkl_kl);
 }
 
 // element / assembly pass time of the last timed batch run (ms) and step counts

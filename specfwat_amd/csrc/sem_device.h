@@ -108,6 +108,7 @@ struct SemMesh {
   int regular_fast_path = -1;  // element pass (fwat_set_tuning_); -1: the library's choice
   int blocks_per_cu_fwd = 0;  // element-pass workgroups per CU (0: one per element)
   int blocks_per_cu_adj = 8;
+  size_t readout_bytes = (size_t)256 << 20;  // device memory that kernels on their way out take at a time
   int graph = 0;              // whole-run loops captured into a HIP graph (fwat_set_graph_)
   // reduced-precision statics hold value/scale (FP16 needs it for range)
   float static_scale_kappa = 1.0f, static_scale_mu = 1.0f;
@@ -288,6 +289,10 @@ inline T* dev_alloc(size_t n) {
 
 // copy to ordinary host memory, complete on return; large ones through several threads (transfer.hip)
 void sem_to_host(void* host, const void* dev, size_t bytes, hipStream_t s);
+
+// device memory for n results of unit_bytes each on their way out (transfer.hip): n of them, or as
+// many as limit bytes hold (at least one), fewer when the device is full; *units = how many
+void* sem_readout_alloc(size_t n, size_t unit_bytes, size_t limit, size_t* units);
 
 template <class T>
 inline T* dev_upload(const T* h, size_t n, hipStream_t s) {
@@ -510,6 +515,8 @@ __device__ __forceinline__ void sem_seismo_block(const SemSeismo& S, int r, real
 void sem_launch_forces(SemMesh* m, int nfields, int kernel_mode, int elem_begin, int elem_count,
                        realw deltat, const int* elem_list, bool gather, const SemInterior* in = nullptr,
                        const SemSeismo* se = nullptr);
+// c_ij kernels K [n][21][125] of n elements to the caller's (21,NGLLX,NGLLY,NGLLZ,n), scaled by -1
+void sem_cij_to_host(const SemMesh* m, const double* K, size_t n, double* host);
 // true when a whole-mesh fused element pass of nfields fields finishes the element-interior points
 bool sem_interior_active(const SemMesh* m, int nfields);
 // host <-> device copies of three point fields (u, v, a) of size 3 * nglob in the

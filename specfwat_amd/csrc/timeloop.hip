@@ -571,15 +571,6 @@ __global__ void k_scale_kernel(size_t n, const double* __restrict__ K, const rea
   if (i < n) out[i] = K[i] * (factor * (double)modulus[i]);
 }
 
-// c_ij kernels of one element from rows [21][125] to the caller's [125][21], negated, through LDS
-__global__ __launch_bounds__(256) void k_cij_point_major(const double* __restrict__ K, double* __restrict__ out) {
-  __shared__ double s[2625];
-  const size_t b = (size_t)blockIdx.x * 2625;
-  for (int i = threadIdx.x; i < 2625; i += 256) s[i] = K[b + i];
-  __syncthreads();
-  for (int i = threadIdx.x; i < 2625; i += 256) out[b + i] = -s[(i % 21) * 125 + i / 21];
-}
-
 }  // namespace
 
 // ------------------------------------------------------------ internal stages
@@ -997,11 +988,7 @@ void transfer_kernels_ani_to_host_dp_(long* Mesh_pointer, double* h_cijkl_kl, in
   SemMesh* m = sem_mesh(Mesh_pointer);
   if (*NSPEC_AB != m->nspec) SEM_FAIL("NSPEC_AB mismatch");
   if (!m->d_cijkl_kl) SEM_FAIL("anisotropic kernels not prepared");
-  const size_t nloc = (size_t)m->nspec * 125;
-  double* tmp = dev_alloc<double>(nloc * 21);
-  hipLaunchKernelGGL(k_cij_point_major, dim3(m->nspec), dim3(256), 0, m->stream, m->d_cijkl_kl, tmp);
-  sem_to_host(h_cijkl_kl, tmp, nloc * 21 * 8, m->stream);
-  dev_free(tmp);
+  sem_cij_to_host(m, m->d_cijkl_kl, (size_t)m->nspec, h_cijkl_kl);
 }
 
 // approximate Hessian (sum of dt * a_adj . a_rec), (NGLLX,NGLLY,NGLLZ,NSPEC_AB)
@@ -1456,6 +1443,15 @@ void fwat_interior_info_(long* Mesh_pointer, int* n_shared, int* n_interior, int
   *n_interior = m->nglob - m->n_shared;
   *active_fwd = sem_interior_active(m, 1) ? 1 : 0;
   *active_adj = sem_interior_active(m, 2) ? 1 : 0;
+}
+
+// Device memory (bytes, default 256 MiB) that kernels on their way to the host take at a time
+// beside the accumulators, for the c_ij kernels of a run and all kernels of a batch on it; at least
+// one element's (c_ij) or one point's are taken, and fewer than asked for when the device is full.
+void fwat_set_readout_bytes_(long* Mesh_pointer, int* bytes) {
+  SemMesh* m = sem_mesh(Mesh_pointer);
+  if (*bytes < 1) SEM_FAIL("fwat_set_readout_bytes_: the read-out needs some memory");
+  m->readout_bytes = (size_t)*bytes;
 }
 
 // HIP graph capture of the whole-run loop (fused gather path): 1 = every

@@ -72,6 +72,15 @@ bool staged_to_host(char* host, const char* dev, size_t bytes, hipStream_t s) {
   return true;
 }
 
+// c_ij kernels of one element from rows [21][125] to the caller's [125][21], negated, through LDS
+__global__ __launch_bounds__(256) void k_cij_point_major(const double* __restrict__ K, double* __restrict__ out) {
+  __shared__ double s[2625];
+  const size_t b = (size_t)blockIdx.x * 2625;
+  for (int i = threadIdx.x; i < 2625; i += 256) s[i] = K[b + i];
+  __syncthreads();
+  for (int i = threadIdx.x; i < 2625; i += 256) out[b + i] = -s[(i % 21) * 125 + i / 21];
+}
+
 bool pageable(const void* host) {
   hipPointerAttribute_t at;
   if (hipPointerGetAttributes(&at, host) == hipSuccess) return at.type == hipMemoryTypeUnregistered;
@@ -87,4 +96,31 @@ void sem_to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
   if (bytes >= STAGE_MIN && pageable(host) && staged_to_host((char*)host, (const char*)dev, bytes, s)) return;
   HIP_CHECK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
   HIP_CHECK(hipStreamSynchronize(s));
+}
+
+// Kernels are scaled and reordered on the device before their copy, a bounded part at a time: a run
+// that fills the device still gets its results out.
+void* sem_readout_alloc(size_t n, size_t unit_bytes, size_t limit, size_t* units) {
+  size_t k = std::min(n, std::max<size_t>(1, limit / unit_bytes));
+  void* p = nullptr;
+  while (hipMalloc(&p, k * unit_bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    if (k == 1) SEM_FAIL("no device memory left to read results out (%zu bytes needed)", unit_bytes);
+    k = (k + 1) / 2;
+  }
+  *units = k;
+  return p;
+}
+
+void sem_cij_to_host(const SemMesh* m, const double* K, size_t n, double* host) {
+  constexpr size_t EL = 2625;
+  size_t most = 0;
+  double* tmp = (double*)sem_readout_alloc(n, EL * sizeof(double), m->readout_bytes, &most);
+  for (size_t e = 0; e < n; e += most) {
+    const size_t k = std::min(most, n - e);
+    hipLaunchKernelGGL(k_cij_point_major, dim3((unsigned)k), dim3(256), 0, m->stream, K + e * EL, tmp);
+    HIP_CHECK(hipGetLastError());
+    sem_to_host(host + e * EL, tmp, k * EL * sizeof(double), m->stream);
+  }
+  dev_free(tmp);
 }

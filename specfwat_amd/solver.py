@@ -161,6 +161,11 @@ class ElasticRun:
         it as a unit (fused gather path; captured runs are not timed)."""
         _lib.call("fwat_set_graph_", self.h, int(bool(on)))
 
+    def set_readout_bytes(self, nbytes):
+        """Device memory that c_ij kernels (and the kernels of a batch on this handle) take at a
+        time on their way to the host (default 256 MiB; fewer when the device is full)."""
+        _lib.call("fwat_set_readout_bytes_", self.h, int(nbytes))
+
     def set_kernel_block(self, nsteps):
         """Steps per fp32 partial-sum block of the mu/kappa (c_ij) kernels; 1 = fp64 every step."""
         _lib.call("fwat_set_kernel_block_", self.h, int(nsteps))

@@ -269,3 +269,34 @@ def test_windows_of_data_that_are_not_finite(bad):
         np.testing.assert_array_equal(got[c], np.array(ref).reshape(-1, 2))
         n += len(ref)
     assert n >= 4
+
+
+@pytest.mark.parametrize("nbytes", [1, 7 * 21000, 11 * 21000 + 20999, 36 * 21000])
+@pytest.mark.parametrize("aniso", [False, True])
+def test_kernels_read_out_in_parts(aniso, nbytes):
+    """Kernels leave the device through a bounded piece of memory: one element or point at a time,
+    ragged last parts, and exactly all; the same bits as in one piece, for a run and for a batch."""
+    from specfwat_amd.batch import EventBatch
+    c = make_case(seed=71, nstep=20, aniso=aniso)
+    m = c["mesh"]
+    src, rec = Sources(m, c["sxyz"], c["mt"], c["f0"]), Receivers(m, c["rxyz"])
+    adj = np.random.default_rng(4).standard_normal((2, c["nstep"], rec.nrec, 3)).astype(np.float32)
+    f, a = (ElasticRun(m, c["rho"], c["vp"], c["vs"], src, rec, c["dt"], c["nstep"], k, k == 1, cij=c["cij"]) for k in (1, 3))
+    f.iterate_time()
+    a.take_forward(f)
+    a.set_adjoint_sources(adj[0])
+    a.iterate_time()
+    b = EventBatch(m, c["rho"], c["vp"], c["vs"], [src, src], rec, c["dt"], [c["nstep"]] * 2, cij=c["cij"])
+    b.forward()
+    b.set_adjoint_sources(adj)
+    b.adjoint()
+    for run, read in ((a, a.kernels), (b.run, b.kernels)):
+        whole = read()
+        run.set_readout_bytes(nbytes if aniso else max(nbytes // 10, 1))
+        part = read()
+        for n in whole:
+            assert np.abs(whole[n]).max() > 0
+            np.testing.assert_array_equal(part[n], whole[n], err_msg=n)
+    b.close()
+    f.close()
+    a.close()
