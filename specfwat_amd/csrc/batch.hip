@@ -1029,7 +1029,7 @@ void batch_points_to_host(SemBatch* B, const realw* h_rhostore, double* rho, dou
   hipStream_t s = m->stream;
   const size_t E = (size_t)B->E, nloc = (size_t)m->nspec * 125;
   size_t most = 0;
-  double* tmp = (double*)sem_readout_alloc(nloc, E * sizeof(double) + sizeof(realw), m->readout_bytes, &most);
+  double* tmp = (double*)sem_alloc_part(nloc, E * sizeof(double) + sizeof(realw), m->readout_bytes, &most);
   realw* d_rho = (realw*)(tmp + E * most);
   for (size_t L0 = 0; L0 < nloc; L0 += most) {
     const size_t n = std::min(most, nloc - L0);

@@ -2083,12 +2083,14 @@ __global__ void k_fill_f32m(size_t n, float* __restrict__ x) {
 
 double g_meas_ms = 0.0;
 
-// Device scratch of one call, cut from a few large blocks that are given back together: giving back
-// a block of 100 MB or more takes 0.23 ms, and a call has a dozen such arrays.
+// Device scratch of one call in one block of exactly its size: giving back a block of 100 MB or more
+// takes 0.23 ms, and a call has a dozen such arrays.  arrays(f) runs f twice, first to add up what
+// it asks for, then with the block there.
 class Scratch {
   std::vector<void*> blocks_;
   char* at_ = nullptr;
-  size_t left_ = 0;
+  size_t left_ = 0, need_ = 0;
+  bool measuring_ = false;
 
  public:
   Scratch() = default;
@@ -2097,37 +2099,45 @@ class Scratch {
   ~Scratch() {
     for (void* p : blocks_) HIP_CHECK(hipFree(p));
   }
-  template <class T>
-  T* alloc(size_t n) {
-    if (n == 0) return nullptr;
-    const size_t bytes = (n * sizeof(T) + 255) & ~(size_t)255;
-    if (bytes > left_) {
-      left_ = std::max(bytes * 8, (size_t)1 << 20);  // room for arrays like this one
-      if (left_ > (size_t)1 << 30) left_ = std::max(bytes, (size_t)1 << 30);
-      void* p = nullptr;
-      if (left_ > bytes && hipMalloc(&p, left_) != hipSuccess) {
-        (void)hipGetLastError();  // little memory left: this array alone
-        p = nullptr;
-      }
-      if (!p) {
-        left_ = bytes;
-        HIP_CHECK(hipMalloc(&p, left_));
-      }
+  template <class F>
+  void arrays(F f) {
+    need_ = 0;
+    measuring_ = true;
+    f();
+    measuring_ = false;
+    void* p = nullptr;
+    if (need_ && hipMalloc(&p, need_) == hipSuccess) {
       blocks_.push_back(p);
       at_ = (char*)p;
+      left_ = need_;
+    } else {
+      (void)hipGetLastError();  // no block of that size: each array by itself
+      left_ = 0;
+    }
+    f();
+  }
+  template <class T>
+  T* alloc(size_t n) {
+    const size_t bytes = (n * sizeof(T) + 255) & ~(size_t)255;
+    if (measuring_) need_ += bytes;
+    if (measuring_ || n == 0) return nullptr;
+    if (bytes > left_) {
+      void* p = nullptr;
+      HIP_CHECK(hipMalloc(&p, bytes));
+      blocks_.push_back(p);
+      return reinterpret_cast<T*>(p);
     }
     T* p = reinterpret_cast<T*>(at_);
     at_ += bytes;
     left_ -= bytes;
     return p;
   }
-  template <class T>
-  T* upload(const T* h, size_t n, hipStream_t s) {
-    T* p = alloc<T>(n);
-    if (n) HIP_CHECK(hipMemcpyAsync(p, h, n * sizeof(T), hipMemcpyHostToDevice, s));
-    return p;
-  }
 };
+
+template <class T>
+void to_device(T* p, const T* h, size_t n, hipStream_t s) {
+  if (n) HIP_CHECK(hipMemcpyAsync(p, h, n * sizeof(T), hipMemcpyHostToDevice, s));
+}
 
 // window_taper's weights (signal.f90:419-491) for a window of npts samples
 void taper_weights_into(int npts, double pct, int type, double* w);
@@ -2176,56 +2186,63 @@ struct CcShift {
     while (nf < 2 * nl - 1) nf *= 2;
     return nf;
   }
+  // the spectra of as many traces as this many bytes hold at a time (4,096 traces of the longest
+  // windows: 16 rounds of the chip's workgroups), fewer when the device is full
+  static constexpr size_t SPECTRA = (size_t)1 << 29;
   int T;
   hipStream_t s;
+  size_t blocks = 0, spec = 0, piece = 0;
   double* bv = nullptr;
   int* bi = nullptr;
   double2* G = nullptr;
   std::vector<std::pair<int, double2*>> tw;  // one table per transform length
   CcShift(int ntrace, const std::vector<int>& nls, hipStream_t stream) : T(ntrace), s(stream) {
-    size_t blocks = 0, spec = 0;
     for (int nl : nls) {
-      if (fft(nl)) spec = std::max(spec, (size_t)points(nl) / 2 + 1);
-      else blocks = std::max(blocks, (size_t)(2 * nl - 1 + CC_LAGS - 1) / CC_LAGS);
+      if (!fft(nl)) {
+        blocks = std::max(blocks, (size_t)(2 * nl - 1 + CC_LAGS - 1) / CC_LAGS);
+        continue;
+      }
+      const int nf = points(nl);
+      spec = std::max(spec, (size_t)nf / 2 + 1);
+      if (std::none_of(tw.begin(), tw.end(), [&](auto& p) { return p.first == nf; })) tw.emplace_back(nf, nullptr);
     }
-    bv = dev_alloc<double>(T * blocks);
-    bi = dev_alloc<int>(T * blocks);
-    G = dev_alloc<double2>(T * spec);
   }
-  const double2* table(int nf) {
+  void arrays(Scratch& m) {
+    bv = m.alloc<double>(T * blocks);
+    bi = m.alloc<int>(T * blocks);
+    for (auto& p : tw) p.second = m.alloc<double2>((size_t)p.first / 2);
+  }
+  // after arrays(): the tables, and the spectra
+  void start() {
     for (auto& p : tw)
-      if (p.first == nf) return p.second;
-    double2* d = dev_alloc<double2>((size_t)nf / 2);
-    hipLaunchKernelGGL(k_twiddles, dim3((unsigned)((nf / 2 + 255) / 256)), dim3(256), 0, s, nf, d);
-    tw.emplace_back(nf, d);
-    return d;
+      hipLaunchKernelGGL(k_twiddles, dim3((unsigned)((p.first / 2 + 255) / 256)), dim3(256), 0, s, p.first, p.second);
+    if (spec) G = (double2*)sem_alloc_part((size_t)T, spec * sizeof(double2), SPECTRA, &piece);
   }
   void run(int nl, const double* D, const double* S, int* ish) {
     if (fft(nl)) {
       const int nf = points(nl), M = nf / 2;
       int logM = 0;
       while ((1 << logM) < M) ++logM;
-      const double2* w = table(nf);
+      const double2* w = std::find_if(tw.begin(), tw.end(), [&](auto& p) { return p.first == nf; })->second;
       const size_t lds = (size_t)M * sizeof(double2);
       const void* f = M >= 4096 ? reinterpret_cast<const void*>(k_cc_corr_fft<1024>)
                                 : reinterpret_cast<const void*>(k_cc_corr_fft<256>);
       if (lds > 49152) HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      if (M >= 4096)
-        hipLaunchKernelGGL(k_cc_corr_fft<1024>, dim3((unsigned)T), dim3(1024), lds, s, nl, nf, logM, w, D, S, G, ish);
-      else
-        hipLaunchKernelGGL(k_cc_corr_fft<256>, dim3((unsigned)T), dim3(256), lds, s, nl, nf, logM, w, D, S, G, ish);
+      for (size_t t = 0; t < (size_t)T; t += piece) {
+        const dim3 gr((unsigned)std::min(piece, (size_t)T - t));
+        const double *d = D + t * nl, *x = S + t * nl;
+        if (M >= 4096)
+          hipLaunchKernelGGL(k_cc_corr_fft<1024>, gr, dim3(1024), lds, s, nl, nf, logM, w, d, x, G, ish + t);
+        else
+          hipLaunchKernelGGL(k_cc_corr_fft<256>, gr, dim3(256), lds, s, nl, nf, logM, w, d, x, G, ish + t);
+      }
       return;
     }
     const int nblk = (2 * nl - 1 + CC_LAGS - 1) / CC_LAGS;
     hipLaunchKernelGGL(k_cc_corr, dim3((unsigned)nblk, (unsigned)T), dim3(256), 0, s, nl, D, S, bv, bi);
     hipLaunchKernelGGL(k_cc_pick, dim3((unsigned)((T + MTPB - 1) / MTPB)), dim3(MTPB), 0, s, T, nblk, nl, bv, bi, ish);
   }
-  void free_all() {
-    dev_free(bv);
-    dev_free(bi);
-    dev_free(G);
-    for (auto& p : tw) dev_free(p.second);
-  }
+  void free_all() { dev_free(G); }
 };
 
 // dpss_windows (utils/dpss.f90:137-262) for the multitaper measurement: the
@@ -2547,11 +2564,6 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   hipEvent_t e0, e1;
   HIP_CHECK(hipEventCreate(&e0));
   HIP_CHECK(hipEventCreate(&e1));
-  float* d_obs = scratch.upload(obs, n, s);
-  float* d_syn = scratch.upload(syn, n, s);
-  float* d_adj = scratch.alloc<float>(n);
-  int* d_ish = scratch.alloc<int>(T);
-  double* d_out = scratch.alloc<double>(8 * (size_t)nw * T);
   int maxnl = 0;
   std::vector<int> nbs(nw), nls(nw);
   std::vector<std::vector<double>> tws(nw);
@@ -2563,11 +2575,33 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     wmin = std::min(wmin, std::min(windows[2 * w], windows[2 * w + 1]));
     wmax = std::max(wmax, std::max(windows[2 * w], windows[2 * w + 1]));
   }
-  double* d_D = scratch.alloc<double>((size_t)T * maxnl);
-  double* d_S = scratch.alloc<double>((size_t)T * maxnl);
-  double* d_tw = scratch.alloc<double>(maxnl);
-  double* d_A = scratch.alloc<double>((size_t)T * maxnl);
-  CcShift shift(T, nls, s);
+  std::vector<double> fw;
+  int fnb = 0, fnl = 0;
+  if (*nsect > 0) {
+    window_range(wmin, wmax, *dt, N, fnb, fnl);
+    taper_weights(fnl, *taper_percentage, *itaper_type, fw);
+  }
+  CcShift shift(T, *imeas == 5 ? std::vector<int>() : nls, s);
+  float *d_obs, *d_syn, *d_adj, *d_sos;
+  int* d_ish;
+  double *d_out, *d_D, *d_S, *d_tw, *d_A, *d_fw;
+  scratch.arrays([&] {
+    d_obs = scratch.alloc<float>(n);
+    d_syn = scratch.alloc<float>(n);
+    d_adj = scratch.alloc<float>(n);
+    d_ish = scratch.alloc<int>(T);
+    d_out = scratch.alloc<double>(8 * (size_t)nw * T);
+    d_D = scratch.alloc<double>((size_t)T * maxnl);
+    d_S = scratch.alloc<double>((size_t)T * maxnl);
+    d_tw = scratch.alloc<double>(maxnl);
+    d_A = scratch.alloc<double>((size_t)T * maxnl);
+    d_fw = scratch.alloc<double>(fw.size());
+    d_sos = scratch.alloc<float>(6 * (size_t)*nsect);
+    shift.arrays(scratch);
+  });
+  to_device(d_obs, obs, n, s);
+  to_device(d_syn, syn, n, s);
+  shift.start();
   HIP_CHECK(hipEventRecord(e0, s));
   hipLaunchKernelGGL(k_fill_f32m, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, d_adj);
   for (int w = 0; w < nw; ++w) {
@@ -2585,15 +2619,9 @@ void fwat_cc_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
     hipLaunchKernelGGL(k_cc_put, dim3((unsigned)((T + 63) / 64), (unsigned)((nls[w] + 63) / 64)), dim3(256), 0, s, T,
                        nbs[w], nls[w], d_A, d_out + 8 * (size_t)w * T, d_adj);
   }
-  std::vector<double> fw;
-  double* d_fw = nullptr;
-  float* d_sos = nullptr;
   if (*nsect > 0) {
-    int fnb = 0, fnl = 0;
-    window_range(wmin, wmax, *dt, N, fnb, fnl);
-    taper_weights(fnl, *taper_percentage, *itaper_type, fw);
-    d_fw = scratch.upload(fw.data(), fw.size(), s);
-    d_sos = scratch.upload(sos, 6 * (size_t)*nsect, s);
+    to_device(d_fw, fw.data(), fw.size(), s);
+    to_device(d_sos, sos, 6 * (size_t)*nsect, s);
     launch_sos(s, N, T, *nsect, d_sos, d_adj);
     hipLaunchKernelGGL(k_window_final, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, N, T, fnb, fnl, d_fw,
                        d_adj);
@@ -2706,6 +2734,9 @@ void fwat_mt_adjoint_batch_(int* nstep, int* ntrace, double* dt, realw* obs, rea
   double* d_tw = dev_alloc<double>(maxnl);
   double* d_tap = dev_alloc<double>((size_t)ntaper * maxnl);
   CcShift shift(T, nls, s);
+  Scratch scratch;
+  scratch.arrays([&] { shift.arrays(scratch); });
+  shift.start();
   const int imcc = *imeas == 13 ? 11 : 12;
   float* d_obsT = dev_alloc<float>(n);
   float* d_synT = dev_alloc<float>(n);
@@ -2919,43 +2950,55 @@ void fwat_win_sel_batch_(int* nstep, int* ntrace, double* dt, realw* obs, realw*
   hipEvent_t ev0, ev1;
   HIP_CHECK(hipEventCreate(&ev0));
   HIP_CHECK(hipEventCreate(&ev1));
-  float* d_obs = scratch.upload(obs, n, s);
-  float* d_syn = scratch.upload(syn, n, s);
-  double* d_tp = scratch.upload(tp, (size_t)T, s);
-  double* d_dist = scratch.upload(dist, (size_t)T, s);
-  double* d_wt = scratch.upload(wt.data(), wt.size(), s);
-  float* d_obsT = scratch.alloc<float>(n);
-  float* d_synT = scratch.alloc<float>(n);
-  double* d_Dn = scratch.alloc<double>(n);
-  double* d_Sn = scratch.alloc<double>(n);
-  double* d_noise = scratch.alloc<double>(T);
-  double* d_ts = scratch.alloc<double>((size_t)nw * T);
-  double* d_cc = scratch.alloc<double>((size_t)nw * T);
-  int* d_ish = scratch.alloc<int>((size_t)nw * T);
-  int* d_nwin = scratch.alloc<int>(T);
-  double* d_win = scratch.alloc<double>(2 * (size_t)*maxwin * T);
-  unsigned char* d_good = scratch.alloc<unsigned char>((size_t)nw * T);
   // phase splitting: envelope transform on nf = 2 ** exponent(real(nstep)) points
   int nfe = 0, Me = 0, logMe = 0;
-  double *d_env = nullptr, *d_stl = nullptr;
-  double2 *d_g01 = nullptr, *d_twe = nullptr;
+  std::vector<double> twh;
   if (split) {
     int e2 = 0;
     std::frexp((float)N, &e2);
     nfe = 1 << e2;
     Me = nfe / 2;
     while ((1 << logMe) < Me) ++logMe;
-    std::vector<double> twh(2 * (size_t)Me);
+    twh.resize(2 * (size_t)Me);
     for (int j = 0; j < Me; ++j) {
       const long double a = -2.0L * 3.141592653589793238462643383279502884L * (long double)j / (long double)nfe;
       twh[2 * j] = (double)std::cos(a);
       twh[2 * j + 1] = (double)std::sin(a);
     }
-    d_twe = reinterpret_cast<double2*>(scratch.upload(twh.data(), twh.size(), s));
-    d_env = scratch.alloc<double>(n);
-    d_stl = scratch.alloc<double>(n);
-    d_g01 = scratch.alloc<double2>(2 * (size_t)T * (Me + 1));
   }
+  float *d_obs, *d_syn, *d_obsT, *d_synT;
+  double *d_tp, *d_dist, *d_wt, *d_Dn, *d_Sn, *d_noise, *d_ts, *d_cc, *d_win, *d_env, *d_stl;
+  double2 *d_g01, *d_twe;
+  int *d_ish, *d_nwin;
+  unsigned char* d_good;
+  scratch.arrays([&] {
+    d_obs = scratch.alloc<float>(n);
+    d_syn = scratch.alloc<float>(n);
+    d_tp = scratch.alloc<double>(T);
+    d_dist = scratch.alloc<double>(T);
+    d_wt = scratch.alloc<double>(wt.size());
+    d_obsT = scratch.alloc<float>(n);
+    d_synT = scratch.alloc<float>(n);
+    d_Dn = scratch.alloc<double>(n);
+    d_Sn = scratch.alloc<double>(n);
+    d_noise = scratch.alloc<double>(T);
+    d_ts = scratch.alloc<double>((size_t)nw * T);
+    d_cc = scratch.alloc<double>((size_t)nw * T);
+    d_ish = scratch.alloc<int>((size_t)nw * T);
+    d_nwin = scratch.alloc<int>(T);
+    d_win = scratch.alloc<double>(2 * (size_t)*maxwin * T);
+    d_good = scratch.alloc<unsigned char>((size_t)nw * T);
+    d_twe = scratch.alloc<double2>(Me);
+    d_env = scratch.alloc<double>(split ? n : 0);
+    d_stl = scratch.alloc<double>(split ? n : 0);
+    d_g01 = scratch.alloc<double2>(split ? 2 * (size_t)T * (Me + 1) : 0);
+  });
+  to_device(d_obs, obs, n, s);
+  to_device(d_syn, syn, n, s);
+  to_device(d_tp, tp, T, s);
+  to_device(d_dist, dist, T, s);
+  to_device(d_wt, wt.data(), wt.size(), s);
+  to_device(reinterpret_cast<double*>(d_twe), twh.data(), twh.size(), s);
   HIP_CHECK(hipEventRecord(ev0, s));
   const dim3 ttiles((unsigned)((T + 63) / 64), (unsigned)((N + 63) / 64));
   hipLaunchKernelGGL(k_rows_f32, ttiles, dim3(256), 0, s, N, T, d_obs, d_obsT);

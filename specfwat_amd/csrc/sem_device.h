@@ -290,9 +290,9 @@ inline T* dev_alloc(size_t n) {
 // copy to ordinary host memory, complete on return; large ones through several threads (transfer.hip)
 void sem_to_host(void* host, const void* dev, size_t bytes, hipStream_t s);
 
-// device memory for n results of unit_bytes each on their way out (transfer.hip): n of them, or as
-// many as limit bytes hold (at least one), fewer when the device is full; *units = how many
-void* sem_readout_alloc(size_t n, size_t unit_bytes, size_t limit, size_t* units);
+// device memory for work on n units of unit_bytes each that can be done in parts (transfer.hip): all
+// of them, or as many as limit bytes hold (at least one), fewer when the device is full; *units = how many
+void* sem_alloc_part(size_t n, size_t unit_bytes, size_t limit, size_t* units);
 
 template <class T>
 inline T* dev_upload(const T* h, size_t n, hipStream_t s) {

@@ -98,24 +98,24 @@ void sem_to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
   HIP_CHECK(hipStreamSynchronize(s));
 }
 
-// Kernels are scaled and reordered on the device before their copy, a bounded part at a time: a run
-// that fills the device still gets its results out.
-void* sem_readout_alloc(size_t n, size_t unit_bytes, size_t limit, size_t* units) {
+void* sem_alloc_part(size_t n, size_t unit_bytes, size_t limit, size_t* units) {
   size_t k = std::min(n, std::max<size_t>(1, limit / unit_bytes));
   void* p = nullptr;
   while (hipMalloc(&p, k * unit_bytes) != hipSuccess) {
     (void)hipGetLastError();
-    if (k == 1) SEM_FAIL("no device memory left to read results out (%zu bytes needed)", unit_bytes);
+    if (k == 1) SEM_FAIL("no device memory left (%zu bytes needed)", unit_bytes);
     k = (k + 1) / 2;
   }
   *units = k;
   return p;
 }
 
+// Kernels are reordered on the device before their copy, a bounded part at a time: a run that fills
+// the device still gets its results out.
 void sem_cij_to_host(const SemMesh* m, const double* K, size_t n, double* host) {
   constexpr size_t EL = 2625;
   size_t most = 0;
-  double* tmp = (double*)sem_readout_alloc(n, EL * sizeof(double), m->readout_bytes, &most);
+  double* tmp = (double*)sem_alloc_part(n, EL * sizeof(double), m->readout_bytes, &most);
   for (size_t e = 0; e < n; e += most) {
     const size_t k = std::min(most, n - e);
     hipLaunchKernelGGL(k_cij_point_major, dim3((unsigned)k), dim3(256), 0, m->stream, K + e * EL, tmp);

@@ -81,6 +81,23 @@ def test_correlation_shift_by_transforms(nl):
         assert meas[k, 0, 4] == pytest.approx(o["tshift"][0], abs=1e-12), k
 
 
+def test_more_traces_than_spectra_at_a_time():
+    """Spectra of the correlations take at most 512 MiB, 4,095 traces of 4,097 samples: with 4,098
+    traces the last three come in a part of their own.  Every trace as in a small call."""
+    nl, nrec, dt = 4097, 1366, 0.01
+    rng = np.random.default_rng(8)
+    obs, syn = (rng.standard_normal((nl + 7, 5, 3)).astype(np.float32) for _ in range(2))
+    q = np.arange(nrec) % 5
+    win = [[0.03, 0.03 + nl * dt + 0.001]]
+    assert misfit.get_window_info(win[0], dt)[2] == nl
+    print(f"{3 * nrec} traces", flush=True)
+    _, adj0, meas0 = misfit.event_cc_adjoint_sources(obs, syn, dt, win, imeas=12, cc_min=0.0)
+    _, adj, meas = misfit.event_cc_adjoint_sources(obs[:, q], syn[:, q], dt, win, imeas=12, cc_min=0.0)
+    assert meas0[:, 0, 6].any() and len(set(meas0[:, 0, 7])) == 15
+    np.testing.assert_array_equal(meas.reshape(nrec, 3, -1), meas0.reshape(5, 3, -1)[q])
+    np.testing.assert_array_equal(adj, adj0[:, q])
+
+
 @pytest.mark.parametrize("nrec", [1, 3, 4, 5, 9])
 def test_many_receivers_in_one_element(nrec):
     """Every receiver in one element on an absorbing side: a point's row then ends in nrec receiver
