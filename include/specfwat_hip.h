@@ -157,8 +157,9 @@ void fwat_move_stacey_store_(long *Mesh_pointer_from, long *Mesh_pointer_to);
  * element (both fields through ping-pong LDS buffers), 4 = form 3 with non-temporal hints on the
  * streamed indices, moduli and kernel partial sums, 5 = form 3 visiting the elements of a lattice
  * mesh (fwat_set_lattice_) in column blocks, layer by layer (element order elsewhere);
- * blocks_per_cu_* = persistent workgroups per CU, 0 = one per element.  Until it is called isotropic
- * all-regular meshes take form 3 with 10 (forward) and 8 (adjoint) workgroups per CU */
+ * blocks_per_cu_* = persistent workgroups per CU, 0 = one per element.  regular_path -1 = the
+ * library's choice: form 3 on isotropic all-regular meshes (blocks_per_cu_fwd 0: 10), 1 on
+ * anisotropic ones.  A handle starts with -1, 0, 8 */
 void fwat_set_tuning_(long *Mesh_pointer, int *regular_path, int *blocks_per_cu_fwd, int *blocks_per_cu_adj);
 /* The column-block element order regular_path 5 uses for a nex x ney x nez lattice and per_xcd
  * workgroups per XCD: order[nex*ney*nez], 0-based elements in traversal order.  Host only; no

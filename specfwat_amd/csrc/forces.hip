@@ -1031,7 +1031,7 @@ void fwat_column_block_order_(int* nex, int* ney, int* nez, int* per_xcd, int* o
 }
 }  // extern "C"
 
-// Element pass of a handle whose launch shape was never set (fwat_set_tuning_).  Isotropic cubes
+// Element pass of a handle that leaves it to the library (fwat_set_tuning_ not called, or with -1).  Isotropic cubes
 // take the pipelined pass, which finishes the interior points: a step (element pass and assembly)
 // of 64x64x32 elements 290 against 313 us with the folded-table pass, both fields 592 against 651;
 // 32x32x16 41.9 against 45.3 and 71.9 against 77.9; 16x16x8 16.0 against 16.7 and 18.6 against
@@ -1039,11 +1039,12 @@ void fwat_column_block_order_(int* nex, int* ney, int* nez, int* per_xcd, int* o
 // other meshes the general one, the only ones there are for them.
 static int element_path(const SemMesh* m) { return m->regular_fast_path >= 0 ? m->regular_fast_path : m->anisotropy ? 1 : 3; }
 
-// Persistent workgroups per CU of the pipelined pass chosen so: 10 with one field (five waves per
-// SIMD; 12 leave two waiting: 230 against 169 us at 64x64x32, 8: 191), 8 with two (6: 377 against 356).
+// Persistent workgroups per CU of the pipelined pass chosen so, unless the caller gives others: 10 with one
+// field (five waves per SIMD; 12 leave two waiting: 230 against 169 us at 64x64x32, 8: 191), 8, the handle's
+// initial value, with two (6: 377 against 356).
 static int element_blocks(const SemMesh* m, int nfields) {
-  if (m->regular_fast_path < 0 && element_path(m) == 3) return nfields == 2 ? 8 : 10;
-  return nfields == 2 ? m->blocks_per_cu_adj : m->blocks_per_cu_fwd;
+  if (nfields == 2) return m->blocks_per_cu_adj;
+  return m->blocks_per_cu_fwd == 0 && m->regular_fast_path < 0 && element_path(m) == 3 ? 10 : m->blocks_per_cu_fwd;
 }
 
 bool sem_interior_active(const SemMesh* m, int nfields) {

@@ -1468,13 +1468,14 @@ void fwat_set_graph_(long* Mesh_pointer, int* on) {
 // barriers per element, 4 = form 3 with non-temporal hints on the streamed
 // arrays, 5 = form 3 visiting the elements of a lattice mesh in column blocks
 // (isotropic; anisotropic passes keep 1), 0 = general
-// kernel; blocks_per_cu_* = persistent workgroups per CU
-// for the one-field and two-field passes, 0 = one workgroup per element.
+// kernel, -1 = the library's choice, which a handle starts with; blocks_per_cu_* = persistent
+// workgroups per CU for the one-field and two-field passes, 0 = one workgroup per element
+// (for the one-field pass with -1 on isotropic meshes: the library's 10).  A handle starts with 0 and 8.
 void fwat_set_tuning_(long* Mesh_pointer, int* regular_path, int* blocks_per_cu_fwd, int* blocks_per_cu_adj) {
   SemMesh* m = sem_mesh(Mesh_pointer);
   if (*blocks_per_cu_fwd < 0 || *blocks_per_cu_adj < 0 || *blocks_per_cu_fwd > 64 || *blocks_per_cu_adj > 64)
     SEM_FAIL("fwat_set_tuning_: blocks per CU must be in 0..64");
-  if (*regular_path < 0 || *regular_path > 5) SEM_FAIL("fwat_set_tuning_: regular_path must be 0 to 5");
+  if (*regular_path < -1 || *regular_path > 5) SEM_FAIL("fwat_set_tuning_: regular_path must be -1 to 5");
   m->regular_fast_path = *regular_path;
   m->blocks_per_cu_fwd = *blocks_per_cu_fwd;
   m->blocks_per_cu_adj = *blocks_per_cu_adj;

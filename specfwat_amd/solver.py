@@ -116,9 +116,11 @@ class ElasticRun:
             self.stf = sources.stf(self.nstep, self.dt)
             _lib.call("fwat_set_stf_", self.h, self.stf, self.nstep)
 
-    def set_tuning(self, regular_path=1, blocks_per_cu_fwd=0, blocks_per_cu_adj=8, brick=(0, 0, 0),
+    def set_tuning(self, regular_path=-1, blocks_per_cu_fwd=0, blocks_per_cu_adj=8, brick=(0, 0, 0),
                    brick_blocks_per_cu=0, slab_elems=0, interior=True):
-        """Element-pass launch shape; brick=(bx, by, bz) switches the brick-fused
+        """Element-pass launch shape; regular_path -1 leaves the pass to the library, as a
+        new handle does (pipelined on isotropic cubes, blocks_per_cu_fwd 0 then means its 10
+        persistent workgroups per CU); brick=(bx, by, bz) switches the brick-fused
         element + assembly pass on (lattice meshes of regular elements only);
         slab_elems > 0 runs element pass + assembly slab after slab; interior: the
         pipelined passes finish the element-interior points (set_interior)."""

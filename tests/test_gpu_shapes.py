@@ -317,3 +317,27 @@ def test_kernels_read_out_in_parts(aniso, nbytes):
     b.close()
     f.close()
     a.close()
+
+
+def test_other_knobs_leave_the_default_element_pass():
+    """A new handle takes the library's element pass, which finishes the interior points of cubes;
+    setting another knob keeps it, and after another pass -1 brings it back: the same bits throughout."""
+    c = make_case(seed=81, nstep=40)
+    m = c["mesh"]
+    src, rec = Sources(m, c["sxyz"], c["mt"], c["f0"]), Receivers(m, c["rxyz"])
+    first = None
+    for steps in ([], [{}], [dict(interior=True)], [dict(slab_elems=8), {}], [dict(regular_path=1), dict(regular_path=-1)],
+                  [dict(interior=False), dict(blocks_per_cu_adj=4)]):
+        f = ElasticRun(m, c["rho"], c["vp"], c["vs"], src, rec, c["dt"], c["nstep"], 1, True)
+        for kw in steps:
+            f.set_tuning(**kw)
+        assert f.interior_info()[2:] == (1, 1), steps
+        f.iterate_time()
+        syn = f.seismograms()
+        f.close()
+        first = syn if first is None else first
+        np.testing.assert_array_equal(syn, first)
+    f = ElasticRun(m, c["rho"], c["vp"], c["vs"], src, rec, c["dt"], c["nstep"], 1, True)
+    f.set_tuning(regular_path=1)
+    assert f.interior_info()[2:] == (0, 0)
+    f.close()
