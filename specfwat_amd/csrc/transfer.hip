@@ -8,13 +8,9 @@
 // memory copies run on several cores.  The slots and the threads live for one call.  (The other way the
 // runtime reaches 28 GB/s from memory the caller has written, and stays in use.)
 #include "sem_device.h"
+#include "staged_copy.h"
 
 #include <algorithm>
-#include <atomic>
-#include <cstring>
-#include <exception>
-#include <thread>
-#include <vector>
 
 namespace {
 
@@ -23,52 +19,38 @@ constexpr int STAGE_THREADS = 8;
 // below this the slots and threads (about 0.5 ms) cost more than they save
 constexpr size_t STAGE_MIN = (size_t)16 << 20;
 
+struct DeviceLink {
+  int device;
+  char* pinned;
+  const char* dev;
+  hipStream_t s;
+  hipEvent_t ev[STAGE_THREADS][2];
+  char* slot(int w, int b) { return pinned + (2 * (size_t)w + b) * STAGE_CHUNK; }
+  int begin(int w) {
+    int e = hipSetDevice(device);
+    if (!e) e = hipEventCreateWithFlags(&ev[w][0], hipEventDisableTiming);
+    return e ? e : (int)hipEventCreateWithFlags(&ev[w][1], hipEventDisableTiming);
+  }
+  int fetch(int w, int b, size_t offset, size_t n) {
+    const int e = hipMemcpyAsync(slot(w, b), dev + offset, n, hipMemcpyDeviceToHost, s);
+    return e ? e : (int)hipEventRecord(ev[w][b], s);
+  }
+  int wait(int w, int b) { return hipEventSynchronize(ev[w][b]); }
+  int end(int w) {
+    const int e = hipEventDestroy(ev[w][0]);
+    return e ? e : (int)hipEventDestroy(ev[w][1]);
+  }
+};
+
 bool staged_to_host(char* host, const char* dev, size_t bytes, hipStream_t s) {
-  const size_t chunks = (bytes + STAGE_CHUNK - 1) / STAGE_CHUNK;
-  int device = 0;
-  HIP_CHECK(hipGetDevice(&device));
-  char* pinned = nullptr;
-  if (hipHostMalloc((void**)&pinned, 2 * STAGE_THREADS * STAGE_CHUNK, hipHostMallocDefault) != hipSuccess) {
+  DeviceLink link{0, nullptr, dev, s, {}};
+  HIP_CHECK(hipGetDevice(&link.device));
+  if (hipHostMalloc((void**)&link.pinned, 2 * STAGE_THREADS * STAGE_CHUNK, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  std::atomic<size_t> next{0};
-  std::atomic<int> ids{0};
-  // two slots per thread: one on the link while the other is copied from
-  const auto work = [&] {
-    HIP_CHECK(hipSetDevice(device));
-    char* slot = pinned + 2 * STAGE_CHUNK * (size_t)ids.fetch_add(1);
-    hipEvent_t ev[2];
-    for (auto& e : ev) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    size_t held[2] = {chunks, chunks};  // the chunk of each slot, chunks: none
-    const auto size_of = [&](size_t c) { return std::min(STAGE_CHUNK, bytes - c * STAGE_CHUNK); };
-    const auto hand_over = [&](int b) {
-      if (held[b] == chunks) return;
-      HIP_CHECK(hipEventSynchronize(ev[b]));
-      std::memcpy(host + held[b] * STAGE_CHUNK, slot + b * STAGE_CHUNK, size_of(held[b]));
-      held[b] = chunks;
-    };
-    int b = 0;
-    for (size_t c = next.fetch_add(1); c < chunks; c = next.fetch_add(1), b ^= 1) {
-      hand_over(b);
-      HIP_CHECK(hipMemcpyAsync(slot + b * STAGE_CHUNK, dev + c * STAGE_CHUNK, size_of(c), hipMemcpyDeviceToHost, s));
-      HIP_CHECK(hipEventRecord(ev[b], s));
-      held[b] = c;
-    }
-    hand_over(b);
-    hand_over(b ^ 1);
-    for (auto& e : ev) HIP_CHECK(hipEventDestroy(e));
-  };
-  std::vector<std::thread> team;
-  const int others = (int)std::min<size_t>(STAGE_THREADS, chunks) - 1;
-  try {
-    team.reserve(others);
-    for (int t = 0; t < others; ++t) team.emplace_back(work);
-  } catch (const std::exception&) {  // fewer threads: the ones there are take all chunks
-  }
-  work();
-  for (auto& t : team) t.join();
-  HIP_CHECK(hipHostFree(pinned));
+  HIP_CHECK((hipError_t)staged_copy(host, bytes, STAGE_CHUNK, STAGE_THREADS, link));
+  HIP_CHECK(hipHostFree(link.pinned));
   return true;
 }
 
