@@ -159,9 +159,9 @@ def batch_device_bytes(mesh, nevents, nmax, store_precision=0):
     nloc, ng = mesh.nspec * 125, mesh.nglob
     nfp = mesh.num_abs_boundary_faces * 25
     e = nevents
-    store = nmax * nfp * e * (6 if store_precision else 12) + (nmax * e * 4 + nfp * e * 12 if store_precision else 0)
+    store = nmax * nfp * e * (6 if store_precision else 12) + (nmax * e * 4 + nfp * e * 24 if store_precision else 0)
     return (6 * ng * e * 12 + 2 * nloc * e * 12 + (2 * nloc + ng) * e * 12
-            + store + nfp * e * 12 + 4 * (ng + nloc + nfp) + 8 * e * nmax)
+            + store + 4 * (ng + nloc + nfp) + 8 * e * nmax)
 
 
 def tune_batch(mesh, model, sources, receivers, dt, sizes=(2, 4, 8), blocks_per_cu=(4, 6, 8, 12, 16), nstep=12,

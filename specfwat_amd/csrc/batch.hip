@@ -835,7 +835,7 @@ struct SemBatch {
   realw *u = nullptr, *v = nullptr, *a = nullptr;     // forward / adjoint field [nglob][E][3]
   realw *bu = nullptr, *bv = nullptr, *ba = nullptr;  // reconstructed field
   realw *floc0 = nullptr, *floc1 = nullptr;           // [nloc][E][3]
-  realw* face_scratch = nullptr;                      // [nfp][E][3]
+  realw* face_scratch = nullptr;                      // [nfp][E][3] tractions of a step (fp16 store)
   realw* store = nullptr;                             // [nmax][nfp][E][3] fp32 store
   int store_precision = 0;                            // 0 fp32, 1 fp16 with a scale per record and event
   uint16_t* store16 = nullptr;                        // [nmax][nfp][E][3] fp16 store
@@ -1011,12 +1011,14 @@ void ensure_store(SemBatch* B) {
     dev_free(B->store16);
     dev_free(B->store_max);
     dev_free(B->face_replay);
+    dev_free(B->face_scratch);
     if (!B->store) B->store = dev_alloc<realw>(n);
   } else {
     dev_free(B->store);
     if (!B->store16) B->store16 = dev_alloc<uint16_t>(n);
     if (!B->store_max) B->store_max = dev_alloc<unsigned int>((size_t)B->nmax * B->E);
     if (!B->face_replay) B->face_replay = dev_alloc<realw>(B->nfp * B->E * 3);
+    if (!B->face_scratch) B->face_scratch = dev_alloc<realw>(B->nfp * B->E * 3);
     const size_t ns = (size_t)B->nmax * B->E;
     hipLaunchKernelGGL(k_fill_u32, dim3(nblk(ns)), dim3(TPB), 0, s, B->store_max, ns);
   }
@@ -1165,7 +1167,6 @@ void fwat_batch_create_(long* Mesh_pointer, long* Batch_pointer, int* nevents, i
   const size_t nf3 = ng * E * 3;
   B->u = dev_alloc<realw>(nf3); B->v = dev_alloc<realw>(nf3); B->a = dev_alloc<realw>(nf3);
   B->floc0 = dev_alloc<realw>(nloc * E * 3);
-  if (nfp) B->face_scratch = dev_alloc<realw>(nfp * E * 3);  // the store: ensure_store, at the forward run
   if (m->nrec) {
     const size_t ns = (size_t)E * B->nmax * m->nrec * 3;
     B->seis = dev_alloc<realw>(ns);

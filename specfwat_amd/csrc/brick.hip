@@ -254,6 +254,7 @@ void brick_free(SemMesh* m) {
   dev_free(m->d_brick_special);
   dev_free(m->d_brick_part0);
   dev_free(m->d_brick_part1);
+  dev_free(m->d_face_scratch);
   dev_free(m->d_halo_g);
   dev_free(m->d_halo_off);
   dev_free(m->d_halo_idx);
@@ -506,6 +507,7 @@ void fwat_set_brick_(long* Mesh_pointer, int* bx, int* by, int* bz, int* blocks_
   m->d_halo_off = dev_upload(off.data(), off.size(), s);
   m->d_halo_idx = dev_upload(idx.data(), idx.size(), s);
   m->d_brick_part0 = dev_alloc<realw>((size_t)nslot * 3);
+  if (nfp) m->d_face_scratch = dev_alloc<realw>(nfp * 3);
   if (m->simulation_type == 3) m->d_brick_part1 = dev_alloc<realw>((size_t)nslot * 3);
   HIP_CHECK(hipStreamSynchronize(s));
 }

@@ -310,7 +310,6 @@ void prepare_constants_device_(long* Mesh_pointer, int* h_NGLLX, int* NSPEC_AB, 
     sem_build_assembly_csr(m->nglob, m->nspec, owner, visit, off, idx);
     upload_assembly_csr(m, off, idx);
     m->d_floc = dev_alloc<realw>(nloc * 3);
-    if (nfp) m->d_face_scratch = dev_alloc<realw>(nfp * 3);
     HIP_CHECK(hipStreamSynchronize(s));
   }
   HIP_CHECK(hipStreamSynchronize(s));

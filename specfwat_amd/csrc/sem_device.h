@@ -207,7 +207,7 @@ struct SemMesh {
   // face point, then nsources*125 source points, then nrec*125 receiver points.
   realw* d_floc = nullptr;      // [nspec][125][3]
   realw* d_floc_b = nullptr;    // second field of the adjoint pass
-  realw* d_face_scratch = nullptr;  // [nfaces*25][3] absorbing term of a non-stored field
+  realw* d_face_scratch = nullptr;  // [nfaces*25][3] absorbing term of a non-stored field (brick pass only)
   int asm_points_per_lane = 0;  // gather assembly: 1 or 2 points per lane, 0 = the default (see stage_assemble)
   int asm_block = 256;          // gather assembly: lanes per workgroup (64..1024)
   int floc_grouped = 1;         // floc rows grouped by reader (sem_floc_slot), 0: local-point order

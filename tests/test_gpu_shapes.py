@@ -341,3 +341,43 @@ def test_other_knobs_leave_the_default_element_pass():
     f.set_tuning(regular_path=1)
     assert f.interior_info()[2:] == (0, 0)
     f.close()
+
+
+@pytest.mark.parametrize("n", [24, 60])
+def test_assemblies_agree_with_many_boundary_points(n):
+    """Above 57,344 points with boundary, source or receiver terms (60x60x2: 58,081 at the bottom
+    alone) one lane walks the row of each, below eight lanes; slab by slab one lane walks every
+    row.  One and two points per lane, and slabs: the same bits, forward and adjoint."""
+    nex, ney, lz, h = n, n, 2, 625.0
+    m = BoxMesh(nex, ney, lz, nex * h, ney * h, lz * h)
+    print(f"assembly with many boundary points, {m.nspec} elements", flush=True)
+    rng = np.random.default_rng(n)
+    f = (1 + 0.03 * rng.standard_normal(m.nglob))[m.ibool0]
+    rho, vp, vs = (np.float32(v) * f.astype(np.float32) for v in (2700, 6000, 3500))
+    src = Sources(m, [[0.4 * m.lx, 0.5 * m.ly, -0.5 * m.lz]], [list(1e15 * rng.standard_normal(6))], [6.0])
+    rec = Receivers(m, np.stack([rng.uniform(0.35, 0.5, 5) * m.lx, rng.uniform(0.4, 0.6, 5) * m.ly, np.zeros(5)], axis=1))
+    steps, first = 24, None
+    adj = rng.standard_normal((steps, rec.nrec, 3)).astype(np.float32)
+    for lanes, slab in ((1, 0), (2, 0), (0, n * n), (0, 0)):
+        out = []
+        a = None
+        for k in (1, 3):
+            r = ElasticRun(m, rho, vp, vs, src, rec, 0.004, steps, k, k == 1)
+            r.set_tuning(regular_path=1, slab_elems=slab)
+            r.set_assembly_lanes(lanes)
+            if k == 1:
+                r.iterate_time()
+                out.append(r.seismograms())
+                out += list(r.fields())
+                a = r
+                continue
+            r.take_forward(a)
+            a.close()
+            r.set_adjoint_sources(adj)
+            r.iterate_time()
+            out += list(r.kernels().values())
+            r.close()
+        assert all(np.abs(x).max() > 0 for x in out)
+        first = out if first is None else first
+        for x, y in zip(out, first):
+            np.testing.assert_array_equal(x, y, err_msg=f"lanes {lanes}, slab {slab}")
