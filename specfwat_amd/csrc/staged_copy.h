@@ -9,11 +9,11 @@
 #include <thread>
 #include <vector>
 
-// Copies bytes to host by at most `threads` workers, chunk bytes at a time, each worker with two slots:
-// one on the link while the other is copied from.  Link (calls return 0 or an error):
-//   begin(w), end(w)             worker w starts, on its own thread, and ends (after a begin that succeeded)
-//   fetch(w, b, offset, n)       starts bringing n bytes from offset into slot b of w
-//   wait(w, b), slot(w, b)       waits for the last fetch into that slot; the slot's memory
+// Copies bytes to host by at most `threads` workers, chunk bytes at a time, each worker through a slot of
+// its own: the link serves the others while one copies from its slot.  Link (calls return 0 or an error):
+//   begin(w), end(w)         worker w starts, on its own thread, and ends (after a begin that succeeded)
+//   fetch(w, offset, n)      starts bringing n bytes from offset into the slot of w
+//   wait(w), slot(w)         waits for the last fetch into the slot; the slot's memory
 // Returns the first error, after which no worker starts anything more, once all workers have
 // ended: the caller alone decides what an error does to the process.
 template <class Link>
@@ -29,22 +29,11 @@ int staged_copy(char* host, size_t bytes, size_t chunk, int threads, Link& link)
   const auto work = [&] {
     const int w = ids.fetch_add(1);
     if (!ok(link.begin(w))) return;
-    size_t held[2] = {chunks, chunks};  // the chunk of each slot, chunks: none
-    const auto size_of = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
-    const auto hand_over = [&](int b) {
-      if (held[b] == chunks) return true;
-      if (error.load() || !ok(link.wait(w, b))) return false;
-      std::memcpy(host + held[b] * chunk, link.slot(w, b), size_of(held[b]));
-      held[b] = chunks;
-      return true;
-    };
-    int b = 0;
-    bool going = true;
-    for (size_t c = next.fetch_add(1); going && c < chunks; c = next.fetch_add(1), b ^= 1) {
-      going = hand_over(b) && ok(link.fetch(w, b, c * chunk, size_of(c)));
-      if (going) held[b] = c;
+    for (size_t c = next.fetch_add(1); c < chunks && !error.load(); c = next.fetch_add(1)) {
+      const size_t n = std::min(chunk, bytes - c * chunk);
+      if (!ok(link.fetch(w, c * chunk, n)) || !ok(link.wait(w))) break;
+      std::memcpy(host + c * chunk, link.slot(w), n);
     }
-    if (going && hand_over(b)) hand_over(b ^ 1);
     ok(link.end(w));
   };
   std::vector<std::thread> team;

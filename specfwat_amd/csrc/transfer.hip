@@ -1,12 +1,14 @@
 // Copies of device results to the caller's ordinary host memory.
 //
 // A copy to ordinary (pageable) memory goes through a staging buffer of the runtime on one CPU
-// thread, which also takes the page faults of fresh result arrays: 131 MB of kernels took 12 to
-// 22 ms (6 to 11 GB/s), where the link moves 57 GB/s to pinned memory.  Large copies are
-// therefore staged here: threads take chunks of the range in turn, each copying its chunk from
-// a pinned slot of its own while the other threads' slots are on the link, so that faults and
-// memory copies run on several cores.  The slots and the threads live for one call.  (The other way the
-// runtime reaches 28 GB/s from memory the caller has written, and stays in use.)
+// thread, which also takes the page faults of fresh result arrays, where the link moves 57 GB/s to
+// pinned memory.  Large copies are therefore staged here: threads take chunks of the range in
+// turn, each copying its chunk from a pinned slot of its own while the other threads' slots are on
+// the link, so that faults and memory copies run on several cores.  Not staged / staged, GB/s (MB of 2^20):
+//   fresh array      24 MB  10 / 15    48 MB 9.9 / 22    131 MB 10 / 25    375 MB 10 / 33
+//   written array    24 MB  18 / 23    48 MB  17 / 26    131 MB 17 / 27    375 MB 17 / 34
+// The slots and the threads live for one call.  (The other way the runtime reaches 28 GB/s from
+// memory the caller has written, and stays in use.)
 #include "sem_device.h"
 #include "staged_copy.h"
 
@@ -14,9 +16,15 @@
 
 namespace {
 
-constexpr size_t STAGE_CHUNK = (size_t)2 << 20;
-constexpr int STAGE_THREADS = 8;
-// below this the slots and threads (about 0.5 ms) cost more than they save
+// Slots, one per thread.  Pinned memory costs 0.09 ms a MB in most calls, hardly anything in others or up
+// to 6 MB (seen in the calls' times, not explained): with two slots of 2 MB for each of eight threads, 32 MB in
+// all, 24 MB took 0.9 to 3.8 ms, against 1.4 (written memory) and 2.5 (fresh) unstaged, 48 MB 1.6 to 4.5
+// against 2.9 and 5.1.  Six slots of 1 MB: 24 MB 1.0 to 1.7, 48 MB 1.9 to 2.2; of 512 KB 48 MB in 2.8.  Large
+// copies are worth slots of 2 MB: 90 MB 2.6 to 4.5 against 5.4 and 9.2, 375 MB 11.5 ms (1 MB: 13.1).
+constexpr int STAGE_THREADS = 6;
+constexpr size_t STAGE_CHUNK = (size_t)1 << 20;
+constexpr size_t STAGE_LARGE = (size_t)64 << 20;  // from here on 2 * STAGE_CHUNK
+// below this the slots and threads (about 0.3 ms) cost what they save
 constexpr size_t STAGE_MIN = (size_t)16 << 20;
 
 struct DeviceLink {
@@ -24,32 +32,29 @@ struct DeviceLink {
   char* pinned;
   const char* dev;
   hipStream_t s;
-  hipEvent_t ev[STAGE_THREADS][2];
-  char* slot(int w, int b) { return pinned + (2 * (size_t)w + b) * STAGE_CHUNK; }
+  size_t chunk;
+  hipEvent_t ev[STAGE_THREADS];
+  char* slot(int w) { return pinned + (size_t)w * chunk; }
   int begin(int w) {
-    int e = hipSetDevice(device);
-    if (!e) e = hipEventCreateWithFlags(&ev[w][0], hipEventDisableTiming);
-    return e ? e : (int)hipEventCreateWithFlags(&ev[w][1], hipEventDisableTiming);
+    const int e = hipSetDevice(device);
+    return e ? e : (int)hipEventCreateWithFlags(&ev[w], hipEventDisableTiming);
   }
-  int fetch(int w, int b, size_t offset, size_t n) {
-    const int e = hipMemcpyAsync(slot(w, b), dev + offset, n, hipMemcpyDeviceToHost, s);
-    return e ? e : (int)hipEventRecord(ev[w][b], s);
+  int fetch(int w, size_t offset, size_t n) {
+    const int e = hipMemcpyAsync(slot(w), dev + offset, n, hipMemcpyDeviceToHost, s);
+    return e ? e : (int)hipEventRecord(ev[w], s);
   }
-  int wait(int w, int b) { return hipEventSynchronize(ev[w][b]); }
-  int end(int w) {
-    const int e = hipEventDestroy(ev[w][0]);
-    return e ? e : (int)hipEventDestroy(ev[w][1]);
-  }
+  int wait(int w) { return hipEventSynchronize(ev[w]); }
+  int end(int w) { return hipEventDestroy(ev[w]); }
 };
 
 bool staged_to_host(char* host, const char* dev, size_t bytes, hipStream_t s) {
-  DeviceLink link{0, nullptr, dev, s, {}};
+  DeviceLink link{0, nullptr, dev, s, bytes < STAGE_LARGE ? STAGE_CHUNK : 2 * STAGE_CHUNK, {}};
   HIP_CHECK(hipGetDevice(&link.device));
-  if (hipHostMalloc((void**)&link.pinned, 2 * STAGE_THREADS * STAGE_CHUNK, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc((void**)&link.pinned, STAGE_THREADS * link.chunk, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  HIP_CHECK((hipError_t)staged_copy(host, bytes, STAGE_CHUNK, STAGE_THREADS, link));
+  HIP_CHECK((hipError_t)staged_copy(host, bytes, link.chunk, STAGE_THREADS, link));
   HIP_CHECK(hipHostFree(link.pinned));
   return true;
 }

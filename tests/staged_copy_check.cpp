@@ -12,25 +12,25 @@ struct MemoryLink {
   int fail_at = -1;  // the call (counted over all workers) that fails
   std::atomic<int> calls{0}, inside{0}, begun{0}, ended{0};
   std::vector<char> slots;
-  struct Fetch { size_t offset, n; } last[8][2];
-  MemoryLink(const std::vector<char>& s, size_t c) : src(s), chunk(c), slots(16 * c) {}
+  struct Fetch { size_t offset, n; } last[8];
+  MemoryLink(const std::vector<char>& s, size_t c) : src(s), chunk(c), slots(8 * c) {}
   int call() {
     std::this_thread::sleep_for(std::chrono::microseconds(calls.load() % 7));
     return calls.fetch_add(1) == fail_at ? 77 : 0;
   }
-  char* slot(int w, int b) { return slots.data() + (2 * (size_t)w + b) * chunk; }
+  char* slot(int w) { return slots.data() + (size_t)w * chunk; }
   int begin(int) {
     const int e = call();
     if (!e) ++inside, ++begun;
     return e;
   }
-  int fetch(int w, int b, size_t offset, size_t n) {
-    last[w][b] = {offset, n};
+  int fetch(int w, size_t offset, size_t n) {
+    last[w] = {offset, n};
     return call();
   }
-  int wait(int w, int b) {  // the data arrive here at the latest
+  int wait(int w) {  // the data arrive here at the latest
     const int e = call();
-    if (!e) std::memcpy(slot(w, b), src.data() + last[w][b].offset, last[w][b].n);
+    if (!e) std::memcpy(slot(w), src.data() + last[w].offset, last[w].n);
     return e;
   }
   int end(int) {

@@ -162,11 +162,12 @@ def test_smoothing_of_any_number_of_fields(mesh, perturb, nfield):
         assert rel(out[q], ref) < 1e-5, q  # 32-bit steps, the bar of the other smoothing tests
 
 
-@pytest.mark.parametrize("nrec", [341, 342, 347, 683])
+@pytest.mark.parametrize("nrec", [341, 342, 347, 683, 1365, 1366, 1371])
 def test_large_results_arrive_whole(nrec):
     """Adjoint sources of 4,096 samples, 48 KiB a receiver: from 16 MiB on results are copied in
-    pieces by several threads; below, at and above that size, with ragged last pieces.  The traces
-    repeat those of seven receivers, so each has to equal its part of the small call's result."""
+    pieces by several threads, of 1 MiB below 64 MiB and 2 MiB above; below, at and above these
+    sizes, with ragged last pieces.  The traces repeat those of seven receivers, so each has
+    to equal its part of the small call's result."""
     n, dt = 4096, 0.05
     rng = np.random.default_rng(nrec)
     obs, syn = (rng.standard_normal((n, 7, 3)).astype(np.float32) for _ in range(2))
