@@ -199,9 +199,8 @@ void fwat_set_slabs_(long *Mesh_pointer, int *elems_per_slab);
  * adjoint loop before they are added into the fp64 accumulators (default 16; 1 = every step in
  * fp64).  The rho kernel (summed in the assembly pass) uses the same blocks. */
 void fwat_set_kernel_block_(long *Mesh_pointer, int *nsteps);
-/* points per lane of the gather assembly: 1, 2 (twice the loads in flight per lane; the same
- * per-point sums) or 0 (default: 2 for the forward one-field pass, 1 for the adjoint two-field
- * pass); launch-shape knob, no counterpart in the reference */
+/* points per lane of the gather assembly: 1, 2 (two points' loads in flight per lane; the same
+ * per-point sums) or 0 (default: 1); launch-shape knob, no counterpart in the reference */
 void fwat_set_assembly_lanes_(long *Mesh_pointer, int *points_per_lane);
 /* lanes per workgroup of the gather assembly (64..1024, a multiple of 64; default 256): larger
  * workgroups keep longer runs of consecutive points on one XCD; launch-shape knob, no

@@ -240,10 +240,10 @@ __device__ __forceinline__ void batch_point_newmark(const BatchElemArgs& A, int 
 
 // Element pass of E events (NF = 1 forward, NF = 2 adjoint + reconstruction
 // with in-pass mu/kappa kernels), regular iso meshes, folded tables,
-// persistent XCD-chunked schedule.  The fields of all events are loaded
-// together (3E contiguous floats per lane), then the events are processed one
-// after the other out of LDS; each event's forces overwrite its own LDS slot
-// and are stored together at the end (3E contiguous floats per lane).
+// persistent XCD-chunked schedule.  The points' rows of all events (3E floats)
+// come to LDS by consecutive lanes taking consecutive pieces (EventRow), then
+// the events are processed one after the other; each event's forces overwrite
+// its own LDS slot and leave together the same way at the end.
 // INT: the element-interior points are finished here (batch_point_newmark) and
 // their rows, the last 27 of each element row, are not stored.
 // (the waves-per-SIMD floor is what the pass without the interior points reaches,

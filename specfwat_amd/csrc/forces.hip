@@ -1033,9 +1033,9 @@ void fwat_column_block_order_(int* nex, int* ney, int* nez, int* per_xcd, int* o
 
 // Element pass of a handle that leaves it to the library (fwat_set_tuning_ not called, or with -1).  Isotropic cubes
 // take the pipelined pass, which finishes the interior points: a step (element pass and assembly)
-// of 64x64x32 elements 290 against 313 us with the folded-table pass, both fields 592 against 651;
-// 32x32x16 41.9 against 45.3 and 71.9 against 77.9; 16x16x8 16.0 against 16.7 and 18.6 against
-// 19.9; the same within 2 % at 8x8x4.  Anisotropic cubes take the folded-table pass and
+// of 64x64x32 elements 298 against 340 us with the folded-table pass, both fields 592 against 669;
+// 32x32x16 37.4 against 41.1 and 65.0 against 72.7; 16x16x8 10.4 against 11.2 and 16.4 against
+// 17.4; 8x8x4 8.0 against 8.0 and 10.4 against 9.8.  Anisotropic cubes take the folded-table pass and
 // other meshes the general one, the only ones there are for them.
 static int element_path(const SemMesh* m) { return m->regular_fast_path >= 0 ? m->regular_fast_path : m->anisotropy ? 1 : 3; }
 

@@ -91,13 +91,13 @@ struct SmoothRow {
 // are moved by the lane of their point, which needs no second trip through LDS.
 // 32x32x16 cubes, 21 fields: 119 us a step with a lane per row, one field between two barriers and
 // every row stored, 118 us with a third of the gather's work done here (the gather 94 -> 46 us);
-// LDS and arithmetic are each busy half of the time.
+// of the cycles of busy compute units LDS works in 71 %, a fifth of them conflicts, VALU in 62 %.
 template <int NFP, bool REG>
 __global__ __launch_bounds__(128) void k_smooth_elem(SmoothArgs A) {
   constexpr int W = SmoothRow<NFP>::W, C = SmoothRow<NFP>::C;
   using P = SmoothPiece<W>;
   using T = typename P::T;
-  constexpr int SU = 131;  // pieces c and c + 1 of a point 12 banks apart: rows go in and out without conflicts
+  constexpr int SU = 131;  // pieces c and c + 1 of a point 12 banks apart, where rows go in and out
   __shared__ realw s_tab[128];
   __shared__ int s_g[125];
   __shared__ uint8_t s_row[125];  // local point of each row

@@ -1401,9 +1401,6 @@ void fwat_copy_probe_unrolled_(long* nbytes, int* reps, int* unroll, int* blocks
   HIP_CHECK(hipFree(b));
 }
 
-// Points per lane of the gather assembly: 1 (k_assemble), 2 (k_assemble2, twice
-// the loads in flight per lane; the same sums) or 0 (default: 2 for the one-field
-// pass, 1 for the two-field pass)
 // Lanes per workgroup of the gather assembly launches (a multiple of 64 in 64..1024;
 // default 256).  Consecutive workgroups go to the XCDs in turn, so larger workgroups keep
 // longer runs of consecutive points (and the element rows they share) on one XCD.
@@ -1413,6 +1410,8 @@ void fwat_set_assembly_block_(long* Mesh_pointer, int* lanes) {
   m->asm_block = *lanes;
 }
 
+// Points per lane of the gather assembly: 1 (k_assemble), 2 (k_assemble2: twice
+// the loads in flight per lane; the same sums) or 0 (default: 1)
 void fwat_set_assembly_lanes_(long* Mesh_pointer, int* points_per_lane) {
   SemMesh* m = sem_mesh(Mesh_pointer);
   if (*points_per_lane < 0 || *points_per_lane > 2) SEM_FAIL("fwat_set_assembly_lanes_: 0, 1 or 2 points per lane");
